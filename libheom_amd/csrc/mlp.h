@@ -14,10 +14,9 @@
 
 namespace hamd {
 
-// C[M x N] (ldc) = op(A)[M x K] * op(B)[K x N] (+ bias[N]) (tanh if act);
-// op(A)(m, k) = ta ? A[k*lda + m] : A[m*lda + k], op(B)(k, n) likewise
-void launch_sgemm(int M, int N, int K, const float* A, int lda, bool ta, const float* B, int ldb,
-                  bool tb, float* C, int ldc, const float* bias, bool act, hipStream_t st);
+// y[rows x n_out] = x[rows x n_in] W^T + b (tanh if act), W row-major n_out x n_in
+void launch_layer(int rows, int n_out, int n_in, const float* x, const float* W, const float* b,
+                  float* y, bool act, hipStream_t st);
 
 class Mlp {
  public:
@@ -45,7 +44,8 @@ class Mlp {
   long long n_par;
   DevBuf params, grads, adam_m, adam_v;
   DevBuf xm_, xs_, ym_, ys_;  // normalisation: x' = (x - xm)/xs, y = y'*ys + ym
-  DevBuf xb, tb, h1, h2, yb, dh1, dh2, dyb, partials, perm;
+  DevBuf xb, h1, h2, yb, dh1, dh2, dyb, partials, perm;
+  DevBuf gparts, loss_;  // gradient slices of the k parts (n_par each), the loss
   int cap_rows = 0;
   long long t_adam = 0;
   void ensure_rows(int rows);
@@ -55,7 +55,9 @@ class Mlp {
   float* b2() const;
   float* W3() const;
   float* b3() const;
-  void forward_normalised(int rows);  // xb -> h1, h2, yb
+  int max_grad_parts() const;
+  int grad_split(int rows) const;  // rows per k part of the weight gradients
+  void forward_hidden(int rows);  // xb -> h1, h2
   friend struct Closure;
 };
 

@@ -2,6 +2,7 @@
 // done in a fixed order (no atomics), so training is reproducible run to run.
 #include "mlp.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -13,119 +14,217 @@ namespace hamd {
 
 namespace {
 
+typedef float mf_f4 __attribute__((ext_vector_type(4)));
+
 // ---------------------------------------------------------------------------
-// SGEMM: 64 x 64 output tile per 256-thread workgroup, k in slices of 16
-// staged in LDS; thread (ty, tx) owns rows ty + 16 i and columns tx + 16 j
+// FP32 matrix products of the network on the f32 matrix cores (16x16x4, FP32
+// accumulation): a 64 x 64 output tile per workgroup of four waves (2 x 2
+// accumulators each), k in slices of 32 staged in LDS while the next slice is
+// in flight in registers.  LDS strides 36 (k contiguous) and 80 (m or n
+// contiguous): the 64 lanes of an operand read hit 64 distinct banks.
+//
+// The sizes are small (4096 rows x 256 units: 256 tiles, one per CU; 0.5 GFLOP,
+// 4 us at the f32 matrix rate), so a launch is bound by its k chain.  A weight
+// gradient has few tiles (16 at 256 x 256) and a long k (the rows): it is split
+// over k (ksplit rows per workgroup), every part into its own slice of a
+// partial buffer that grad_reduce_kernel adds up in order.
+// Loss and gradient of 4096 rows of a 49-256-256-32 network: 4850 us with
+// unsplit 64 x 64 vector-ALU products (820 us per weight gradient, 880 us per
+// serial column sum), 180 us here (19 us per layer product, 18 us the three
+// weight gradients, 10 us their sum).
 // ---------------------------------------------------------------------------
-constexpr int kT = 64, kK = 16;
+constexpr int kT = 64, kK = 32;
+constexpr int kLdK = kK + 4, kLdM = kT + 16;
+
+enum GemmEpi { EPI_PLAIN = 0, EPI_TANH = 1, EPI_TANH_BACK = 2, EPI_MSE = 3 };
+
+// C[M x N] = op(A) op(B); op(A)(m, k) = TA ? A[k*lda + m] : A[m*lda + k], op(B) likewise
+struct GemmArgs {
+  int M, N, K;
+  const float *A, *B;
+  int lda, ldb, ldc;
+  float* C;
+  const float* bias;  // added per column (null: none)
+  int epi;
+  const float* H;     // EPI_TANH_BACK: C *= 1 - H^2 (the stored activation, ld = ldc)
+  // EPI_MSE: T = normalised target rows; C = 2 (v - T) / (M N), the sum of
+  // (v - T)^2 over the tile to loss[workgroup]
+  const float *Y, *ym, *ys;
+  const int* perm;
+  double* loss;
+  // split over k (weight gradients): part z of C starts at C + z * part_stride;
+  // asum (null: none) receives the sums of op(A) over the part's k (bias gradient)
+  int ksplit;
+  long long part_stride;
+  float* asum;
+};
+
+// four consecutive elements of a row of n (zero at and past n; p: the row)
+__device__ __forceinline__ mf_f4 ld4(const float* p, int c, int n, bool vec) {
+  if (vec && c + 4 <= n) return *reinterpret_cast<const mf_f4*>(p + c);
+  mf_f4 v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (c + q < n) v[q] = p[c + q];
+  return v;
+}
+
+// TR: the operand is stored k-major (rows of k), else m-major (rows of m).
+// Thread tid takes two groups of four elements of the 64 x 32 slice at (m0, k0).
+template <bool TR>
+struct Slice {
+  mf_f4 v[2];
+  __device__ __forceinline__ void load(const float* P, int ld, int m0, int M, int k0, int k1,
+                                       bool vec) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int x = threadIdx.x + 256 * i;
+      const int r = TR ? k0 + x / 16 : m0 + x / 8;   // row in memory
+      const int c = TR ? m0 + 4 * (x % 16) : k0 + 4 * (x % 8);
+      const bool in = r < (TR ? k1 : M);
+      v[i] = in ? ld4(P + static_cast<long long>(r) * ld, c, TR ? M : k1, vec)
+                : mf_f4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  __device__ __forceinline__ void store(float* s) const {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int x = threadIdx.x + 256 * i;
+      float* d = TR ? s + (x / 16) * kLdM + 4 * (x % 16) : s + (x / 8) * kLdK + 4 * (x % 8);
+      *reinterpret_cast<mf_f4*>(d) = v[i];
+    }
+  }
+};
 
 template <bool TA, bool TB>
-__global__ void __launch_bounds__(256)
-    sgemm_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
-                 const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc,
-                 const float* __restrict__ bias, int act) {
-  __shared__ float As[kK][kT + 4];
-  __shared__ float Bs[kK][kT + 4];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int m0 = blockIdx.y * kT, n0 = blockIdx.x * kT;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += kK) {
-    for (int idx = tid; idx < kT * kK; idx += 256) {
-      int mm, kk;
-      if (TA) {
-        mm = idx % kT;
-        kk = idx / kT;
-      } else {
-        mm = idx / kK;
-        kk = idx % kK;
-      }
-      const int m = m0 + mm, k = k0 + kk;
-      float v = 0.f;
-      if (m < M && k < K) v = TA ? A[static_cast<long long>(k) * lda + m]
-                                 : A[static_cast<long long>(m) * lda + k];
-      As[kk][mm] = v;
-    }
-    for (int idx = tid; idx < kT * kK; idx += 256) {
-      int nn, kk;
-      if (TB) {
-        nn = idx / kK;
-        kk = idx % kK;
-      } else {
-        nn = idx % kT;
-        kk = idx / kT;
-      }
-      const int n = n0 + nn, k = k0 + kk;
-      float v = 0.f;
-      if (n < N && k < K) v = TB ? B[static_cast<long long>(n) * ldb + k]
-                                 : B[static_cast<long long>(k) * ldb + n];
-      Bs[kk][nn] = v;
-    }
+__device__ void gemm_tile(const GemmArgs& g, int bx, int by, int bz, int wg) {
+  __shared__ __align__(16) float As[TA ? kK * kLdM : kT * kLdK];
+  __shared__ __align__(16) float Bs[TB ? kT * kLdK : kK * kLdM];
+  __shared__ double s_loss[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lr = lane & 15, lk = lane >> 4;
+  const int m0 = by * kT, n0 = bx * kT;
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const int k0 = bz * g.ksplit, k1 = min(g.K, k0 + g.ksplit);
+  const bool va = g.lda % 4 == 0 && (reinterpret_cast<uintptr_t>(g.A) & 15) == 0;
+  const bool vb = g.ldb % 4 == 0 && (reinterpret_cast<uintptr_t>(g.B) & 15) == 0;
+  mf_f4 acc[2][2] = {};
+  float asum = 0.f;
+  Slice<TA> a;
+  Slice<!TB> b;
+  a.load(g.A, g.lda, m0, g.M, k0, k1, va);
+  b.load(g.B, g.ldb, n0, g.N, k0, k1, vb);
+  for (int k = k0; k < k1; k += kK) {
     __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < kK; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx + 16 * j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
+    a.store(As);
+    b.store(Bs);
     __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty + 16 * i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx + 16 * j;
-      if (n >= N) continue;
-      float v = acc[i][j];
-      if (bias) v += bias[n];
-      if (act) v = tanhf(v);
-      C[static_cast<long long>(m) * ldc + n] = v;
+    if (k + kK < k1) {
+      a.load(g.A, g.lda, m0, g.M, k + kK, k1, va);
+      b.load(g.B, g.ldb, n0, g.N, k + kK, k1, vb);
     }
+#pragma unroll
+    for (int s = 0; s < kK / 4; ++s) {
+      const int kk = 4 * s + lk;
+      float av[2], bv[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int m = wm + 16 * t + lr, n = wn + 16 * t + lr;
+        av[t] = TA ? As[kk * kLdM + m] : As[m * kLdK + kk];
+        bv[t] = TB ? Bs[n * kLdK + kk] : Bs[kk * kLdM + n];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+    }
+    if (TA && g.asum && bx == 0 && threadIdx.x < kT)
+      for (int kk = 0; kk < kK; ++kk) asum += As[kk * kLdM + threadIdx.x];
+  }
+  if (TA && g.asum && bx == 0 && threadIdx.x < kT && m0 + static_cast<int>(threadIdx.x) < g.M)
+    g.asum[bz * g.part_stride + m0 + threadIdx.x] = asum;
+  float* C = g.C + bz * g.part_stride;
+  double loss = 0.0;
+  const float scale = 2.f / (static_cast<float>(g.M) * static_cast<float>(g.N));
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int m = m0 + wm + 16 * i + 4 * lk + q;
+      if (m >= g.M) continue;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int n = n0 + wn + 16 * j + lr;
+        if (n >= g.N) continue;
+        const long long at = static_cast<long long>(m) * g.ldc + n;
+        float v = acc[i][j][q];
+        if (g.bias) v += g.bias[n];
+        if (g.epi == EPI_TANH) {
+          v = tanhf(v);
+        } else if (g.epi == EPI_TANH_BACK) {
+          const float h = g.H[at];
+          v *= 1.f - h * h;
+        } else if (g.epi == EPI_MSE) {
+          const long long r = g.perm ? g.perm[m] : m;
+          const float d = v - (g.Y[r * g.N + n] - g.ym[n]) / g.ys[n];
+          loss += static_cast<double>(d) * d;
+          v = scale * d;
+        }
+        C[at] = v;
+      }
+    }
+  if (g.epi == EPI_MSE) {
+    for (int o = 32; o > 0; o >>= 1) loss += __shfl_down(loss, o, 64);
+    if (lane == 0) s_loss[wave] = loss;
+    __syncthreads();
+    if (threadIdx.x == 0) g.loss[wg] = (s_loss[0] + s_loss[1]) + (s_loss[2] + s_loss[3]);
   }
 }
 
-// out[j] = sum over rows of X[r*ld + j] (bias gradients), row order fixed
-__global__ void colsum_kernel(const float* X, int rows, int cols, int ld, float* out) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= cols) return;
-  float s = 0.f;
-  for (int r = 0; r < rows; ++r) s += X[static_cast<long long>(r) * ld + j];
-  out[j] = s;
+template <bool TA, bool TB>
+__global__ void __launch_bounds__(256) gemm_kernel(const GemmArgs g) {
+  gemm_tile<TA, TB>(g, blockIdx.x, blockIdx.y, 0, blockIdx.y * gridDim.x + blockIdx.x);
 }
 
-// dH *= 1 - H^2 (derivative of tanh at the stored activation)
-__global__ void tanh_back_kernel(float* dH, const float* H, long long n) {
-  for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<long long>(gridDim.x) * blockDim.x)
-    dH[i] *= 1.f - H[i] * H[i];
+// The three weight gradients (and bias gradients) of a backward pass in one
+// launch: workgroups wg0[i] .. wg0[i+1] take the tiles and k parts of product i.
+struct GradArgs {
+  GemmArgs g[3];
+  int wg0[4], nx[3], ny[3];
+};
+
+__global__ void __launch_bounds__(256) grad_kernel(const GradArgs a) {
+  const int b = blockIdx.x;
+  const int i = b >= a.wg0[2] ? 2 : b >= a.wg0[1] ? 1 : 0;
+  const int r = b - a.wg0[i], nt = a.nx[i] * a.ny[i];
+  const int z = r / nt, t = r - z * nt;
+  gemm_tile<true, false>(a.g[i], t % a.nx[i], t / a.nx[i], z, b);
 }
 
-// dY = 2 (Yhat - T) / n and per-workgroup partial sums of (Yhat - T)^2
-__global__ void __launch_bounds__(256) mse_kernel(const float* Yhat, const float* T, float* dY,
-                                                  long long n, double* partials) {
-  __shared__ double s[256];
-  double acc = 0.0;
-  const float scale = 2.f / static_cast<float>(n);
-  for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<long long>(gridDim.x) * blockDim.x) {
-    const float d = Yhat[i] - T[i];
-    dY[i] = scale * d;
-    acc += static_cast<double>(d) * d;
+// grads[i] = sum over the parts, in order; workgroup 0 also adds up the loss
+// partials (fixed order) and divides by their element count
+__global__ void __launch_bounds__(256) grad_reduce_kernel(const float* parts, int n_parts,
+                                                          long long n, float* grads,
+                                                          const double* loss, int n_loss,
+                                                          double count, double* out) {
+  const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) {
+    float s = 0.f;
+    for (int p = 0; p < n_parts; ++p) s += parts[p * n + i];
+    grads[i] = s;
   }
-  s[threadIdx.x] = acc;
+  if (blockIdx.x != 0) return;
+  __shared__ double sd[256];
+  double l = 0.0;
+  for (int p = threadIdx.x; p < n_loss; p += 256) l += loss[p];
+  sd[threadIdx.x] = l;
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+    if (static_cast<int>(threadIdx.x) < o) sd[threadIdx.x] += sd[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) partials[blockIdx.x] = s[0];
+  if (threadIdx.x == 0) *out = sd[0] / count;
 }
 
 // Adam (Kingma & Ba, 2015) with bias-corrected moments
@@ -225,24 +324,42 @@ double uniform01(uint64_t& s) { return (splitmix(s) >> 11) * (1.0 / 900719925474
 
 }  // namespace
 
-void launch_sgemm(int M, int N, int K, const float* A, int lda, bool ta, const float* B, int ldb,
-                  bool tb, float* C, int ldc, const float* bias, bool act, hipStream_t st) {
-  if (M <= 0 || N <= 0) return;
-  const dim3 grid((N + kT - 1) / kT, (M + kT - 1) / kT);
-  const int a = act ? 1 : 0;
-  if (ta && tb)
-    hipLaunchKernelGGL((sgemm_kernel<true, true>), grid, dim3(256), 0, st, M, N, K, A, lda, B,
-                       ldb, C, ldc, bias, a);
-  else if (ta)
-    hipLaunchKernelGGL((sgemm_kernel<true, false>), grid, dim3(256), 0, st, M, N, K, A, lda, B,
-                       ldb, C, ldc, bias, a);
-  else if (tb)
-    hipLaunchKernelGGL((sgemm_kernel<false, true>), grid, dim3(256), 0, st, M, N, K, A, lda, B,
-                       ldb, C, ldc, bias, a);
-  else
-    hipLaunchKernelGGL((sgemm_kernel<false, false>), grid, dim3(256), 0, st, M, N, K, A, lda, B,
-                       ldb, C, ldc, bias, a);
+namespace {
+
+GemmArgs gemm_args(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
+                   int ldc) {
+  GemmArgs g{};
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.A = A;
+  g.B = B;
+  g.lda = lda;
+  g.ldb = ldb;
+  g.C = C;
+  g.ldc = ldc;
+  g.ksplit = K;
+  return g;
+}
+
+int gemm_tiles(int n) { return (n + kT - 1) / kT; }
+
+template <bool TA, bool TB>
+void launch_gemm(const GemmArgs& g, hipStream_t st) {
+  if (g.M <= 0 || g.N <= 0) return;
+  hipLaunchKernelGGL((gemm_kernel<TA, TB>), dim3(gemm_tiles(g.N), gemm_tiles(g.M)), dim3(256), 0,
+                     st, g);
   HAMD_HIP(hipGetLastError());
+}
+
+}  // namespace
+
+void launch_layer(int rows, int n_out, int n_in, const float* x, const float* W, const float* b,
+                  float* y, bool act, hipStream_t st) {
+  GemmArgs g = gemm_args(rows, n_out, n_in, x, n_in, W, n_in, y, n_out);
+  g.bias = b;
+  g.epi = act ? EPI_TANH : EPI_PLAIN;
+  launch_gemm<false, true>(g, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -334,27 +451,38 @@ void Mlp::fit_scaling(const float* X, const float* Y, long long n_rows) {
   HAMD_HIP(hipStreamSynchronize(stream));
 }
 
+// k parts of the weight gradients: parts of 128 rows (four k slices) give the
+// 256 x 256 gradient 16 tiles x 32 parts at 4096 rows, two workgroups per CU; at
+// most 64 parts, and at most 64 MB of partial gradients (a network with more
+// parameters than that allows fills the chip with fewer parts).
+int Mlp::max_grad_parts() const {
+  const long long fit = (64LL << 20) / static_cast<long long>(sizeof(float)) / n_par;
+  return static_cast<int>(std::max(1LL, std::min(64LL, fit)));
+}
+
+int Mlp::grad_split(int rows) const {
+  constexpr int kMin = 4;  // k slices per part
+  const int slices = (rows + kK - 1) / kK, cap = max_grad_parts();
+  return std::max(kMin, (slices + cap - 1) / cap) * kK;
+}
+
 void Mlp::ensure_rows(int rows) {
   if (rows <= cap_rows) return;
   xb.alloc(sizeof(float) * rows * static_cast<size_t>(n_in));
-  tb.alloc(sizeof(float) * rows * static_cast<size_t>(n_out));
   h1.alloc(sizeof(float) * rows * static_cast<size_t>(n_hid));
   h2.alloc(sizeof(float) * rows * static_cast<size_t>(n_hid));
   dh1.alloc(sizeof(float) * rows * static_cast<size_t>(n_hid));
   dh2.alloc(sizeof(float) * rows * static_cast<size_t>(n_hid));
   yb.alloc(sizeof(float) * rows * static_cast<size_t>(n_out));
   dyb.alloc(sizeof(float) * rows * static_cast<size_t>(n_out));
-  partials.alloc(sizeof(double) * 4096);
+  partials.alloc(sizeof(double) * gemm_tiles(n_out) * gemm_tiles(rows));
+  loss_.alloc(sizeof(double));
   cap_rows = rows;
 }
 
-void Mlp::forward_normalised(int rows) {
-  launch_sgemm(rows, n_hid, n_in, xb.as<float>(), n_in, false, W1(), n_in, true, h1.as<float>(),
-               n_hid, b1(), true, stream);
-  launch_sgemm(rows, n_hid, n_hid, h1.as<float>(), n_hid, false, W2(), n_hid, true,
-               h2.as<float>(), n_hid, b2(), true, stream);
-  launch_sgemm(rows, n_out, n_hid, h2.as<float>(), n_hid, false, W3(), n_hid, true,
-               yb.as<float>(), n_out, b3(), false, stream);
+void Mlp::forward_hidden(int rows) {
+  launch_layer(rows, n_hid, n_in, xb.as<float>(), W1(), b1(), h1.as<float>(), true, stream);
+  launch_layer(rows, n_hid, n_hid, h1.as<float>(), W2(), b2(), h2.as<float>(), true, stream);
 }
 
 void Mlp::forward(const float* X, float* Y, int n_rows) {
@@ -367,7 +495,8 @@ void Mlp::forward(const float* X, float* Y, int n_rows) {
                        dim3(256), 0, stream, X + static_cast<long long>(r0) * n_in,
                        static_cast<const int*>(nullptr), rows, n_in, xm_.as<float>(),
                        xs_.as<float>(), xb.as<float>());
-    forward_normalised(rows);
+    forward_hidden(rows);
+    launch_layer(rows, n_out, n_hid, h2.as<float>(), W3(), b3(), yb.as<float>(), false, stream);
     hipLaunchKernelGGL(denorm_kernel, dim3(grid_for(static_cast<long long>(rows) * n_out)),
                        dim3(256), 0, stream, yb.as<float>(), rows, n_out, ym_.as<float>(),
                        ys_.as<float>(), Y + static_cast<long long>(r0) * n_out);
@@ -376,57 +505,72 @@ void Mlp::forward(const float* X, float* Y, int n_rows) {
   HAMD_HIP(hipStreamSynchronize(stream));
 }
 
+// Forward, loss and gradient in eight launches (the gather, three layers with
+// the loss in the last one's epilogue, two backward products with the
+// derivative of tanh in theirs, the weight and bias gradients, their sum).
 double Mlp::loss_grad(const float* X, const float* Y, int rows, const int* perm_dev) {
   HAMD_HIP(hipSetDevice(device));
   ensure_rows(rows);
   const long long ni = static_cast<long long>(rows) * n_in, no = static_cast<long long>(rows) * n_out;
   hipLaunchKernelGGL(gather_norm_kernel, dim3(grid_for(ni)), dim3(256), 0, stream, X, perm_dev,
                      rows, n_in, xm_.as<float>(), xs_.as<float>(), xb.as<float>());
-  hipLaunchKernelGGL(gather_norm_kernel, dim3(grid_for(no)), dim3(256), 0, stream, Y, perm_dev,
-                     rows, n_out, ym_.as<float>(), ys_.as<float>(), tb.as<float>());
-  forward_normalised(rows);
-  const int gm = grid_for(no);
-  hipLaunchKernelGGL(mse_kernel, dim3(gm), dim3(256), 0, stream, yb.as<float>(), tb.as<float>(),
-                     dyb.as<float>(), no, partials.as<double>());
-  float* g = grads.as<float>();
-  float* gW1 = g;
-  float* gb1 = gW1 + static_cast<long long>(n_hid) * n_in;
-  float* gW2 = gb1 + n_hid;
-  float* gb2 = gW2 + static_cast<long long>(n_hid) * n_hid;
-  float* gW3 = gb2 + n_hid;
-  float* gb3 = gW3 + static_cast<long long>(n_out) * n_hid;
-  const long long nh = static_cast<long long>(rows) * n_hid;
-  // layer 3
-  launch_sgemm(n_out, n_hid, rows, dyb.as<float>(), n_out, true, h2.as<float>(), n_hid, false,
-               gW3, n_hid, nullptr, false, stream);
-  hipLaunchKernelGGL(colsum_kernel, dim3((n_out + 255) / 256), dim3(256), 0, stream,
-                     dyb.as<float>(), rows, n_out, n_out, gb3);
-  launch_sgemm(rows, n_hid, n_out, dyb.as<float>(), n_out, false, W3(), n_hid, false,
-               dh2.as<float>(), n_hid, nullptr, false, stream);
-  hipLaunchKernelGGL(tanh_back_kernel, dim3(grid_for(nh)), dim3(256), 0, stream, dh2.as<float>(),
-                     h2.as<float>(), nh);
-  // layer 2
-  launch_sgemm(n_hid, n_hid, rows, dh2.as<float>(), n_hid, true, h1.as<float>(), n_hid, false,
-               gW2, n_hid, nullptr, false, stream);
-  hipLaunchKernelGGL(colsum_kernel, dim3((n_hid + 255) / 256), dim3(256), 0, stream,
-                     dh2.as<float>(), rows, n_hid, n_hid, gb2);
-  launch_sgemm(rows, n_hid, n_hid, dh2.as<float>(), n_hid, false, W2(), n_hid, false,
-               dh1.as<float>(), n_hid, nullptr, false, stream);
-  hipLaunchKernelGGL(tanh_back_kernel, dim3(grid_for(nh)), dim3(256), 0, stream, dh1.as<float>(),
-                     h1.as<float>(), nh);
-  // layer 1
-  launch_sgemm(n_hid, n_in, rows, dh1.as<float>(), n_hid, true, xb.as<float>(), n_in, false, gW1,
-               n_in, nullptr, false, stream);
-  hipLaunchKernelGGL(colsum_kernel, dim3((n_hid + 255) / 256), dim3(256), 0, stream,
-                     dh1.as<float>(), rows, n_hid, n_hid, gb1);
+  forward_hidden(rows);
+  // layer 3: dY = 2 (yhat - t) / n and the loss partials, one per tile
+  GemmArgs f = gemm_args(rows, n_out, n_hid, h2.as<float>(), n_hid, W3(), n_hid, dyb.as<float>(),
+                         n_out);
+  f.bias = b3();
+  f.epi = EPI_MSE;
+  f.Y = Y;
+  f.ym = ym_.as<float>();
+  f.ys = ys_.as<float>();
+  f.perm = perm_dev;
+  f.loss = partials.as<double>();
+  const int n_loss = gemm_tiles(n_out) * gemm_tiles(rows);
+  launch_gemm<false, true>(f, stream);
+  // dH2 = dY W3 (1 - h2^2), dH1 = dH2 W2 (1 - h1^2)
+  GemmArgs b = gemm_args(rows, n_hid, n_out, dyb.as<float>(), n_out, W3(), n_hid, dh2.as<float>(),
+                         n_hid);
+  b.epi = EPI_TANH_BACK;
+  b.H = h2.as<float>();
+  launch_gemm<false, false>(b, stream);
+  b = gemm_args(rows, n_hid, n_hid, dh2.as<float>(), n_hid, W2(), n_hid, dh1.as<float>(), n_hid);
+  b.epi = EPI_TANH_BACK;
+  b.H = h1.as<float>();
+  launch_gemm<false, false>(b, stream);
+  // gradients, laid out as the parameters, one slice per k part
+  const int split = grad_split(rows), n_parts = (rows + split - 1) / split;
+  const size_t gbytes = sizeof(float) * n_par * static_cast<size_t>(n_parts);
+  if (gparts.bytes < gbytes) gparts.alloc(gbytes);
+  float* gp = gparts.as<float>();
+  float* pW1 = gp;
+  float* pb1 = pW1 + static_cast<long long>(n_hid) * n_in;
+  float* pW2 = pb1 + n_hid;
+  float* pb2 = pW2 + static_cast<long long>(n_hid) * n_hid;
+  float* pW3 = pb2 + n_hid;
+  float* pb3 = pW3 + static_cast<long long>(n_out) * n_hid;
+  GradArgs ga{};
+  ga.g[0] = gemm_args(n_hid, n_hid, rows, dh2.as<float>(), n_hid, h1.as<float>(), n_hid, pW2, n_hid);
+  ga.g[0].asum = pb2;
+  ga.g[1] = gemm_args(n_hid, n_in, rows, dh1.as<float>(), n_hid, xb.as<float>(), n_in, pW1, n_in);
+  ga.g[1].asum = pb1;
+  ga.g[2] = gemm_args(n_out, n_hid, rows, dyb.as<float>(), n_out, h2.as<float>(), n_hid, pW3, n_hid);
+  ga.g[2].asum = pb3;
+  for (int i = 0; i < 3; ++i) {
+    ga.g[i].ksplit = split;
+    ga.g[i].part_stride = n_par;
+    ga.nx[i] = gemm_tiles(ga.g[i].N);
+    ga.ny[i] = gemm_tiles(ga.g[i].M);
+    ga.wg0[i + 1] = ga.wg0[i] + ga.nx[i] * ga.ny[i] * n_parts;
+  }
+  hipLaunchKernelGGL(grad_kernel, dim3(ga.wg0[3]), dim3(256), 0, stream, ga);
+  hipLaunchKernelGGL(grad_reduce_kernel, dim3(static_cast<int>((n_par + 255) / 256)), dim3(256), 0,
+                     stream, gp, n_parts, n_par, grads.as<float>(), partials.as<double>(), n_loss,
+                     static_cast<double>(no), loss_.as<double>());
   HAMD_HIP(hipGetLastError());
-  std::vector<double> part(gm);
-  HAMD_HIP(hipMemcpyAsync(part.data(), partials.p, sizeof(double) * gm, hipMemcpyDeviceToHost,
-                          stream));
+  double loss = 0.0;
+  HAMD_HIP(hipMemcpyAsync(&loss, loss_.p, sizeof(double), hipMemcpyDeviceToHost, stream));
   HAMD_HIP(hipStreamSynchronize(stream));
-  double s = 0.0;
-  for (double v : part) s += v;
-  return s / static_cast<double>(no);
+  return loss;
 }
 
 void Mlp::adam_step(double lr, double beta1, double beta2, double eps) {
@@ -641,12 +785,12 @@ void Closure::forward(const Qme& q, const StageArgs& A, hipStream_t st) {
     return;
   }
   launch_closure_gather(q.dev, A, x.as<float>(), dm.ado_stride, st);
-  launch_sgemm(rows, n_hid, n_in, x.as<float>(), n_in, false, W1.as<float>(), n_in, true,
-               h1.as<float>(), n_hid, b1.as<float>(), true, st);
-  launch_sgemm(rows, n_hid, n_hid, h1.as<float>(), n_hid, false, W2.as<float>(), n_hid, true,
-               h2.as<float>(), n_hid, b2.as<float>(), true, st);
-  launch_sgemm(rows, n_out, n_hid, h2.as<float>(), n_hid, false, W3.as<float>(), n_hid, true,
-               y.as<float>(), n_out, b3.as<float>(), false, st);
+  launch_layer(rows, n_hid, n_in, x.as<float>(), W1.as<float>(), b1.as<float>(), h1.as<float>(),
+               true, st);
+  launch_layer(rows, n_hid, n_hid, h1.as<float>(), W2.as<float>(), b2.as<float>(), h2.as<float>(),
+               true, st);
+  launch_layer(rows, n_out, n_hid, h2.as<float>(), W3.as<float>(), b3.as<float>(), y.as<float>(),
+               false, st);
 }
 
 }  // namespace hamd

@@ -54,6 +54,29 @@ def test_gradient_matches_oracle(rows):
     assert np.abs(g - g_o).max() <= 1e-4 * np.abs(g_o).max()
 
 
+@pytest.mark.parametrize("n_in, n_hid, n_out, rows", [
+    (49, 256, 32, 4096), (1, 1, 1, 1), (5, 3, 2, 127), (64, 65, 33, 128), (20, 100, 64, 129),
+    (63, 64, 65, 31), (36, 68, 4, 8224)])
+def test_gradient_at_tile_and_part_edges(n_in, n_hid, n_out, rows):
+    """Widths and rows at the edges of the 64-wide tiles, the 32-deep k slices and
+    the 128-row parts of the weight gradients, with and without 16-byte rows; a
+    smaller call after a larger one shares its buffers.  FP32 sums of up to 256
+    products and 8224 rows: error well below 1e-4 of the largest entry."""
+    net, sc, rng = small_net(seed=rows, n_in=n_in, n_hid=n_hid, n_out=n_out)
+    X = rng.normal(size=(rows, n_in)).astype(np.float32)
+    Y = rng.normal(size=(rows, n_out)).astype(np.float32)
+    for r in (rows, max(1, rows - 32)):
+        loss, g = net.loss_grad(X[:r], Y[:r])
+        loss_o, g_o = MO.loss_grad(net.get_params().astype(np.float64), n_in, n_hid, n_out,
+                                   X[:r].astype(np.float64), Y[:r].astype(np.float64), sc)
+        assert abs(loss - loss_o) <= 1e-5 * loss_o
+        assert np.abs(g - g_o).max() <= 1e-4 * np.abs(g_o).max()
+        got = net.forward(X[:r])
+        ref = MO.forward(net.get_params().astype(np.float64), n_in, n_hid, n_out,
+                         X[:r].astype(np.float64), sc)
+        assert np.abs(got - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+
+
 def test_adam_step_matches_oracle():
     net, sc, rng = small_net(seed=11)
     X = rng.normal(size=(50, net.n_in)).astype(np.float32)
