@@ -14,6 +14,39 @@
 
 namespace hamd {
 
+namespace {
+// workgroups that cover every item group once: a multiple of eight (the kernel
+// deals consecutive eighths of the items to the eight XCDs)
+int batch_groups(int n_items, int per_group, int cap) {
+  const int per = (n_items + 8 * per_group - 1) / (8 * per_group);
+  return std::min(8 * per, cap);
+}
+
+// a table of complex128 values in the operator precision
+void upload_as(DevBuf& b, const std::vector<z128>& v, bool lo) {
+  if (!lo) {
+    b.upload(v);
+    return;
+  }
+  std::vector<z64> f(v.size());
+  for (size_t i = 0; i < v.size(); ++i) f[i] = conv<float>(v[i]);
+  b.upload(f);
+}
+
+struct CoefRow {
+  z128 iphi, psi, dir;
+  int u;
+};
+
+template <typename R>
+void upload_coef(DevBuf& b, const std::vector<CoefRow>& v) {
+  std::vector<BatchCoef<R>> f(v.size());
+  for (size_t i = 0; i < v.size(); ++i)
+    f[i] = BatchCoef<R>{conv<R>(v[i].iphi), conv<R>(v[i].psi), conv<R>(v[i].dir), v[i].u, 0};
+  b.upload(f);
+}
+}  // namespace
+
 void Qme::set_param_batch(const std::vector<Qme*>& members) {
   if (members.empty()) throw HeomError{HEOM_ERR_ARG, "batch: no members"};
   for (size_t m = 0; m < members.size(); ++m) {
@@ -30,8 +63,8 @@ void Qme::set_param_batch(const std::vector<Qme*>& members) {
   kind = kBatch;
   batch_inst.clear();
   std::vector<int> lp{0};
-  std::vector<BatchLink> bl;
-  std::vector<BatchCoef> bc;
+  std::vector<Link> bl;
+  std::vector<CoefRow> bc;
   std::vector<z128> gm, Hs, tab, dt;
   std::vector<BatchItem> items;
   long long elem = 0;
@@ -43,16 +76,19 @@ void Qme::set_param_batch(const std::vector<Qme*>& members) {
     BatchInst I{};
     I.N = q.N;
     I.N2 = q.N2;
-    I.n_hrchy = q.hs.n_hrchy;
-    I.apw = 64 / q.N2;
-    I.ado_base = total_ado;
-    I.h_off = static_cast<int>(Hs.size());
-    I.tab_off = static_cast<int>(tab.size());
-    I.dterm_off = static_cast<int>(dt.size());
-    I.real_v = q.real_v ? 1 : 0;
     I.elem_base = elem;
     I.rs_off = rs;
-    I.coef_off = static_cast<int>(bc.size());
+    BatchItem W{};
+    W.base = elem;
+    W.N = q.N;
+    W.h_off = static_cast<int>(Hs.size());
+    W.tab_off = static_cast<int>(tab.size());
+    W.dterm_off = static_cast<int>(dt.size());
+    W.coef_off = static_cast<int>(bc.size());
+    W.flags = q.real_v ? kItemRealV : 0;
+    bool direct = false;
+    for (const LinkFlat& f : q.flat_host) direct = direct || f.u >= q.dev.n_noise;
+    if (q.dev.n_noise == 1 && !direct) W.flags |= kItemOneNoise;
     rs += q.N2;
     batch_inst.push_back(I);
     const int base_link = lp.back();
@@ -69,16 +105,24 @@ void Qme::set_param_batch(const std::vector<Qme*>& members) {
         auto it = ids.find(key);
         if (it == ids.end()) {
           it = ids.emplace(key, static_cast<int>(ids.size())).first;
-          bc.push_back(BatchCoef{f.iphi, f.psi, f.dir});
+          bc.push_back(CoefRow{f.iphi, f.psi, f.dir, f.u});
         }
-        bl.push_back(BatchLink{f.nbr, f.u, it->second, 0});
+        bl.push_back(Link{f.nbr, it->second});
       }
     }
     gm.insert(gm.end(), q.ngamma.begin(), q.ngamma.end());
     Hs.insert(Hs.end(), q.H_host.begin(), q.H_host.end());
     tab.insert(tab.end(), q.cmac_host.begin(), q.cmac_host.end());
     dt.insert(dt.end(), q.dterm_host.begin(), q.dterm_host.end());
-    for (int a = 0; a < q.hs.n_hrchy; a += I.apw) items.push_back(BatchItem{static_cast<int>(m), a});
+    const int apw = 64 / q.N2;  // ADOs per wavefront
+    for (int a = 0; a < q.hs.n_hrchy; a += apw) {
+      W.elem = elem + static_cast<long long>(a) * q.N2;
+      W.n_ado = std::min(apw, q.hs.n_hrchy - a);
+      W.g = total_ado + a;
+      W.l0 = base_link + q.link_ptr[a];
+      W.l1 = base_link + q.link_ptr[a + 1];
+      items.push_back(W);
+    }
     elem += q.main_size();
     total_ado += q.hs.n_hrchy;
     N = std::max(N, q.N);
@@ -99,11 +143,14 @@ void Qme::set_param_batch(const std::vector<Qme*>& members) {
   HAMD_HIP(hipSetDevice(opt.device));
   d_link_ptr.upload(lp);
   d_blink.upload(bl);
-  d_bcoef.upload(bc);
-  d_gam.upload(gm);
-  d_H.upload(Hs);
-  d_cmac.upload(tab);
-  d_dterm.upload(dt);
+  if (lo())
+    upload_coef<float>(d_bcoef, bc);
+  else
+    upload_coef<double>(d_bcoef, bc);
+  upload_as(d_gam, gm, lo());
+  upload_as(d_H, Hs, lo());
+  upload_as(d_cmac, tab, lo());
+  upload_as(d_dterm, dt, lo());
   d_inst.upload(batch_inst);
   d_items.upload(items);
   dev = FormDev{};
@@ -113,18 +160,18 @@ void Qme::set_param_batch(const std::vector<Qme*>& members) {
   dev.n_hrchy = total_ado;
   dev.main_size = elem;
   dev.link_ptr = d_link_ptr.as<int>();
-  dev.blink = d_blink.as<BatchLink>();
-  dev.bcoef = d_bcoef.as<BatchCoef>();
-  dev.gam = d_gam.as<z128>();
-  dev.H = d_H.as<z128>();
-  dev.cmac_tab = d_cmac.as<z128>();
-  dev.dterm = d_dterm.as<z128>();
+  dev.blink = d_blink.as<Link>();
+  dev.b_coef = d_bcoef.p;
+  dev.b_gam = d_gam.p;
+  dev.b_H = d_H.p;
+  dev.b_tab = d_cmac.p;
+  dev.b_dterm = d_dterm.p;
   dev.diag_v = 1;
   dev.n_inst = static_cast<int>(batch_inst.size());
   dev.n_items = static_cast<int>(items.size());
   dev.inst = d_inst.as<BatchInst>();
   dev.items = d_items.as<BatchItem>();
-  dev.batch_grid = std::min(dev.n_items, kMaxGrid);
+  dev.batch_grid = batch_groups(dev.n_items, 1, kMaxGrid);
   dev.batch_ipw = 1;
   dev.batch_wpb = 1;
   ready = true;
@@ -185,12 +232,12 @@ void Qme::autotune_batch() {
   HAMD_HIP(hipEventCreate(&e0));
   HAMD_HIP(hipEventCreate(&e1));
   float best = std::numeric_limits<float>::max();
-  int best_g = std::min(dev.n_items, kMaxGrid), best_ipw = 1, best_wpb = 1;
+  int best_g = batch_groups(dev.n_items, 1, kMaxGrid), best_ipw = 1, best_wpb = 1;
   tune_log.clear();
   for (int ipw : {1, 2}) {
     for (int wpb : {1, 2, 4}) {
       // one workgroup per group of ipw * wpb items, or fewer persistent ones
-      const int groups = std::min((dev.n_items + ipw * wpb - 1) / (ipw * wpb), kMaxGrid / wpb);
+      const int groups = batch_groups(dev.n_items, ipw * wpb, kMaxGrid / wpb);
       std::vector<int> cands;
       for (int g : {4096, 16384})
         if (g < groups) cands.push_back(g);
@@ -226,7 +273,7 @@ void Qme::autotune_batch() {
   // a shape other than one item per one-wavefront workgroup must be clearly
   // faster (3%): closer timings are within what separates these passes from
   // the solver's own stages
-  const int plain_g = std::min(dev.n_items, kMaxGrid);
+  const int plain_g = batch_groups(dev.n_items, 1, kMaxGrid);
   for (const TuneEntry& t : tune_log) {
     if (t.ipw == 1 && t.wpb == 1 && t.grid == plain_g && 1e3f * best / 6.0f > 0.97f * t.us) {
       best_g = plain_g;

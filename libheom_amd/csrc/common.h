@@ -153,31 +153,32 @@ struct alignas(16) BlockMap {
 // One member of a batch of independent Hilbert-form hierarchies packed into
 // one set of device tables (Qme::set_param_batch).
 struct BatchInst {
-  int N, N2, n_hrchy;
-  int apw;        // ADOs per 64-lane wavefront (64 / N^2)
-  int ado_base;   // first index in the packed link_ptr / gam arrays
-  int h_off;      // H in the packed H array (z128 units)
-  int tab_off;    // (v_i - v_j, v_i + v_j) table (z128 units)
-  int dterm_off;  // delta table (z128 units)
-  int real_v;
-  int rs_off;     // offset of the member's rho_S in a gathered all-members block
-  int coef_off;   // first entry of the member's link coefficients (BatchCoef)
+  int N, N2;
+  int rs_off;           // offset of the member's rho_S in a gathered all-members block
   long long elem_base;  // first element of the member's state
 };
 
-// Link of the batch kernel: the neighbour, the noise index and the index of
-// its coefficients in the member's table (a member has few distinct ones: one
-// per mode, occupation and direction), 16 bytes instead of the 64 of LinkFlat.
-struct alignas(16) BatchLink {
-  int nbr, u, cid, pad;
-};
-struct alignas(16) BatchCoef {
-  z128 iphi, psi, dir;
+// A member's link coefficients (one entry per mode, occupation and direction;
+// a few KB), in the operator precision; the links themselves are Link records
+// (neighbour within the member, entry of the member's table).
+template <typename R>
+struct alignas(8 * sizeof(R)) BatchCoef {
+  cx<R> iphi, psi, dir;
+  int u;  // noise row of the (v_i - v_j, v_i + v_j) table
+  int pad;
 };
 
-// one wavefront of work: `apw` ADOs of member `inst` starting at local ADO `ado`
-struct BatchItem {
-  int inst, ado;
+// One wavefront of work: n_ado consecutive ADOs (at most 64 / N^2) of one
+// member, with everything the kernel needs to start their loads.
+constexpr int kItemRealV = 1, kItemOneNoise = 2, kItemFast = kItemRealV | kItemOneNoise;
+struct alignas(64) BatchItem {
+  long long elem;  // first element of the item
+  long long base;  // first element of the member's state
+  int N, n_ado;
+  int g;           // first ADO in the packed link_ptr / gam arrays
+  int l0, l1;      // links of that ADO
+  int h_off, tab_off, dterm_off, coef_off;  // the member's tables
+  int flags;       // kItemRealV: V real; kItemOneNoise: one noise, no direct links
 };
 
 constexpr int kBatch = 16;  // Qme / FormDev kind of a packed batch (not a public kind)
@@ -251,8 +252,10 @@ struct FormDev {
   int batch_wpb;  // wavefronts per workgroup (1, 2 or 4), picked by the autotuner
   const BatchInst* inst;
   const BatchItem* items;
-  const BatchLink* blink;  // links of all members (member order, as link_ptr)
-  const BatchCoef* bcoef;  // the members' coefficient tables
+  const Link* blink;  // links of all members (member order, as link_ptr)
+  // the members' tables in the operator precision (cx<R>, BatchCoef<R>): H,
+  // (v_i - v_j, v_i + v_j), delta term, Gamma_n, link coefficients
+  const void *b_H, *b_tab, *b_dterm, *b_gam, *b_coef;
 };
 
 // Dormand-Prince 5(4) tableau (rkdp.h:21-57): A (stage inputs), B (5th-order

@@ -53,29 +53,39 @@ __device__ __forceinline__ LinkFlat ld_link_coef(cptr<Link> lk, cptr<Coef> cf, i
   return f;
 }
 
-__device__ __forceinline__ z128 ldz(const void* p, bool lo, long long i) {
-  if (!lo) return static_cast<const z128*>(p)[i];
-  const z64 v = static_cast<const z64*>(p)[i];
+// Element base + off of a state-sized buffer.  A kernel whose lanes share the
+// base (a block or an item) passes it apart: the address is then a scalar base
+// and a 32-bit lane offset, the same offset for every operand.
+struct At {
+  long long base;
+  int off;
+  __device__ __forceinline__ At(long long b, int o = 0) : base(b), off(o) {}
+};
+
+__device__ __forceinline__ z128 ldz(const void* p, bool lo, At i) {
+  if (!lo) return (static_cast<const z128*>(p) + i.base)[i.off];
+  const z64 v = (static_cast<const z64*>(p) + i.base)[i.off];
   return z128{static_cast<double>(v.re), static_cast<double>(v.im)};
 }
 
 // ldz with a non-temporal load (streamed operands that later loads must not evict)
-__device__ __forceinline__ z128 ldz_nt(const void* p, bool lo, long long i) {
+__device__ __forceinline__ z128 ldz_nt(const void* p, bool lo, At i) {
   typedef double d2v __attribute__((ext_vector_type(2)));
   typedef float f2v __attribute__((ext_vector_type(2)));
   if (!lo) {
-    const d2v w = __builtin_nontemporal_load(static_cast<const d2v*>(p) + i);
+    const d2v w = __builtin_nontemporal_load(static_cast<const d2v*>(p) + i.base + i.off);
     return z128{w.x, w.y};
   }
-  const f2v w = __builtin_nontemporal_load(static_cast<const f2v*>(p) + i);
+  const f2v w = __builtin_nontemporal_load(static_cast<const f2v*>(p) + i.base + i.off);
   return z128{static_cast<double>(w.x), static_cast<double>(w.y)};
 }
 
-__device__ __forceinline__ void stz(void* p, bool lo, long long i, z128 v) {
+__device__ __forceinline__ void stz(void* p, bool lo, At i, z128 v) {
   if (!lo)
-    static_cast<z128*>(p)[i] = v;
+    (static_cast<z128*>(p) + i.base)[i.off] = v;
   else
-    static_cast<z64*>(p)[i] = z64{static_cast<float>(v.re), static_cast<float>(v.im)};
+    (static_cast<z64*>(p) + i.base)[i.off] =
+        z64{static_cast<float>(v.re), static_cast<float>(v.im)};
 }
 
 __device__ __forceinline__ double zabs(z128 a) { return sqrt(a.re * a.re + a.im * a.im); }
@@ -96,7 +106,7 @@ struct PreT {
 using Pre = PreT<kMaxPre>;
 
 template <bool F64, int KP, bool NT = false>
-__device__ __forceinline__ void prefetch(PreT<KP>& p, const StageArgs& A, int cur, long long gi,
+__device__ __forceinline__ void prefetch(PreT<KP>& p, const StageArgs& A, int cur, At gi,
                                          bool ok) {
 #pragma unroll
   for (int s = 0; s < KP; ++s) {
@@ -131,8 +141,8 @@ __device__ __forceinline__ z128 combine(const PreT<KP>& p, const double* c, int 
 // Epilogue shared by all operator kernels.  D is the operator applied to the
 // stage input at flat element gi; returns w^2 of the error norm (or 0).
 template <bool F64, typename R, int KP>
-__device__ __forceinline__ double epilogue(const PreT<KP>& p, const StageArgs& A, int cur,
-                                           long long gi, cx<R> Dr, z128 alpha) {
+__device__ __forceinline__ double epilogue(const PreT<KP>& p, const StageArgs& A, int cur, At gi,
+                                           cx<R> Dr, z128 alpha) {
   const z128 D = conv<double>(Dr);
   const z128 k{-(alpha.re * D.re - alpha.im * D.im), -(alpha.re * D.im + alpha.im * D.re)};
   if (A.mode == MODE_DIFF) {

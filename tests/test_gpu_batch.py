@@ -74,6 +74,33 @@ def test_batch_calc_diff_mixed_n(complex_diag):
         assert err <= TOL * max(1.0, np.abs(ref).max()), (k, m["name"], err)
 
 
+@pytest.mark.parametrize("dtype, tol", [("complex128", TOL), ("complex64", 1e-5)])
+def test_batch_direct_links_and_single_ados(dtype, tol):
+    """Members that leave the compiled-in paths (off-diagonal gamma links, two
+    noises, complex V, sizes other than 2, 4 and 8) beside ones that take them,
+    and hierarchies of depth 0 (no link at all), in both precisions.  FP32: a few
+    tens of products of order 1 per element, so errors of some 1e-6 of the
+    largest."""
+    ms = []
+    for k, (N, nn, L, off) in enumerate([(8, 1, 3, True), (4, 1, 3, True), (2, 2, 3, True),
+                                         (8, 2, 2, False), (7, 1, 3, False), (4, 1, 0, False),
+                                         (8, 1, 0, False), (5, 2, 2, True), (2, 1, 6, False),
+                                         (8, 1, 4, False), (4, 1, 5, False)]):
+        ms.append(configs.random_model(N, nn, 2, L, seed=500 + k, dense_v=False,
+                                       offdiag_gamma=off))
+        if k in (3, 9):
+            for z in ms[-1]["noises"]:
+                z["V"] = z["V"] * (1 + 0.5j)
+    qs = [H.heom_hilb(m["max_depth"], dtype=dtype, parity_q1=False).load(m, eng()) for m in ms]
+    b = H.heom_batch(qs)
+    rho = b.pack([m["rho0"] for m in ms])
+    got = b.calc_diff_impl(None, np.zeros_like(rho), rho, 1.0, 0.0)
+    for m, g in zip(ms, b.unpack(got)):
+        o = O.Oracle(O.HILB, m["N"], m["max_depth"], n_threads=8, parity_q1=False).load(m)
+        ref = o.calc_diff(m["rho0"], 1.0, 0.0)
+        assert np.abs(g - ref).max() <= tol * max(1.0, np.abs(ref).max()), m["name"]
+
+
 def test_batch_calc_diff_full_sweep():
     """All 512 instances of the sweep (N in {2,4,8}, K 2..4, L 4..12) in one launch."""
     ms = configs.batched_sweep()
