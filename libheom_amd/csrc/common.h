@@ -235,9 +235,10 @@ struct FormDev {
   int real_vd;
   // learned truncation closure: rows clos_lo .. clos_lo + clos_n - 1 of the
   // ADOs (the last tier) get clos[(a - clos_lo) * 2 N^2 + e] (real part) and
-  // [... + N^2 + e] (imaginary part) added to D; null when no closure is bound
+  // [... + N^2 + e] (imaginary part) added to D, summed over clos_parts blocks of
+  // clos_n rows; null when no closure is bound
   const float* clos;
-  int clos_lo, clos_n;
+  int clos_lo, clos_n, clos_parts;
   // Redfield: Lambda_u and Lambda_u^+ (n_noise x N x N); rf_T: n_noise x N x N
   // scratch of the two-pass Hilbert kernel (N > 16), in the operator precision
   const z128* rf_L;

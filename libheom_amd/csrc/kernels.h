@@ -39,12 +39,21 @@ void launch_closure_gather(const FormDev& d, const StageArgs& A, float* x, int a
                            hipStream_t stream);
 void launch_gather_rho_s(const FormDev& d, void* dst, const void* src, hipStream_t stream);
 // the whole per-ADO closure network in one launch (gather + three layers on
-// the matrix cores): widths n_in <= 64, n_hid a multiple of 16 up to 256,
-// n_out a multiple of 16 up to 64 (closure_mlp_fits)
+// the matrix cores): widths n_in, n_out <= 128, n_hid <= 256 (closure_mlp_fits),
+// each padded with zeros to a multiple of 16.  Weights in operand order: value
+// (n, k) of a layer with KG = K / 16 groups at
+// ((n/16 * KG + k/16) * 64 + (k%16)/4 * 16 + n%16) * 4 + k%4.  `parts` workgroups
+// (closure_mlp_parts) share 16 rows; part p writes its partial outputs to rows
+// p * rows .. of y.
+struct ClosureNet {
+  int n_in, n_out, in_pad, hid, out_pad, parts;
+  const float *x;  // rows x n_in, the constant columns filled in
+  const float *W1, *b1, *W2, *b2, *W3, *b3;
+  float* y;
+};
 bool closure_mlp_fits(int n_in, int n_hid, int n_out);
-void launch_closure_mlp(const FormDev& d, const StageArgs& A, const float* xc, int n_in,
-                        int n_hid, int n_out, const float* W1, const float* b1, const float* W2,
-                        const float* b2, const float* W3, const float* b3, float* y,
+int closure_mlp_parts(int rows, int hid_pad);
+void launch_closure_mlp(const FormDev& d, const StageArgs& A, const ClosureNet& n,
                         hipStream_t stream);
 
 // Resident fixed-step integrator (heom_hilb with diagonal V and at most 8

@@ -715,6 +715,19 @@ void closure_rows(Qme& deep, Qme& shallow, const void* rho_deep, const float* fe
   HAMD_HIP(hipStreamSynchronize(st));
 }
 
+namespace {
+// a row-major n x k weight matrix, padded with zeros to np x kp, in the operand
+// order of closure_mlp_kernel (see ClosureNet)
+std::vector<float> operand_order(const std::vector<float>& w, int n, int k, int np, int kp) {
+  std::vector<float> o(static_cast<size_t>(np) * kp, 0.f);
+  for (int a = 0; a < n; ++a)
+    for (int b = 0; b < k; ++b)
+      o[((static_cast<size_t>(a / 16) * (kp / 16) + b / 16) * 64 + (b % 16) / 4 * 16 + a % 16) * 4 +
+        b % 4] = w[static_cast<size_t>(a) * k + b];
+  return o;
+}
+}  // namespace
+
 void Closure::bind(Qme& q, const Mlp& m, const float* features, int n_features, int layout) {
   if (q.kind != HEOM_HILB)
     throw HeomError{HEOM_ERR_UNSUPPORTED, "closure: heom_hilb only"};
@@ -752,13 +765,38 @@ void Closure::bind(Qme& q, const Mlp& m, const float* features, int n_features, 
           p[oW3 + static_cast<long long>(o) * n_hid + j] * ys[o];
     bb3[o] = p[ob3 + o] * ys[o] + ym[o];
   }
+  const std::vector<float> w2(p.begin() + oW2, p.begin() + ob2),
+      bb2(p.begin() + ob2, p.begin() + oW3);
   HAMD_HIP(hipSetDevice(q.opt.device));
-  W1.upload(w1);
-  b1.upload(bb1);
-  W2.upload(std::vector<float>(p.begin() + oW2, p.begin() + ob2));
-  b2.upload(std::vector<float>(p.begin() + ob2, p.begin() + oW3));
-  W3.upload(w3);
-  b3.upload(bb3);
+  // per-ADO rows of a network that fits: one fused launch per operator pass
+  fused = layout == HEOM_CLOSURE_PER_ADO && closure_mlp_fits(n_in, n_hid, n_out);
+  net = ClosureNet{};
+  if (fused) {
+    auto pad16 = [](int n) { return (n + 15) / 16 * 16; };
+    net.n_in = n_in;
+    net.n_out = n_out;
+    net.in_pad = pad16(n_in);
+    net.hid = pad16(n_hid);
+    net.out_pad = pad16(n_out);
+    net.parts = closure_mlp_parts(dm.rows, net.hid);
+    auto bias = [](std::vector<float> b, int n) {
+      b.resize(n, 0.f);
+      return b;
+    };
+    W1.upload(operand_order(w1, n_hid, n_in, net.hid, net.in_pad));
+    W2.upload(operand_order(w2, n_hid, n_hid, net.hid, net.hid));
+    W3.upload(operand_order(w3, n_out, n_hid, net.out_pad, net.hid));
+    b1.upload(bias(bb1, net.hid));
+    b2.upload(bias(bb2, net.hid));
+    b3.upload(bias(bb3, net.out_pad));
+  } else {
+    W1.upload(w1);
+    b1.upload(bb1);
+    W2.upload(w2);
+    b2.upload(bb2);
+    W3.upload(w3);
+    b3.upload(bb3);
+  }
   // the constant input columns are written once
   std::vector<float> xh(static_cast<size_t>(dm.rows) * n_in, 0.f);
   const std::vector<float> cst = closure_constants(q, dm, layout, features, n_features);
@@ -766,22 +804,30 @@ void Closure::bind(Qme& q, const Mlp& m, const float* features, int n_features, 
     for (int c = 0; c < dm.n_cst; ++c)
       xh[static_cast<size_t>(r) * n_in + dm.cst_off + c] = cst[static_cast<size_t>(r) * dm.n_cst + c];
   x.upload(xh);
-  h1.alloc(sizeof(float) * dm.rows * static_cast<size_t>(n_hid));
-  h2.alloc(sizeof(float) * dm.rows * static_cast<size_t>(n_hid));
-  y.upload(std::vector<float>(static_cast<size_t>(dm.rows) * n_out, 0.f));
+  if (!fused) {
+    h1.alloc(sizeof(float) * dm.rows * static_cast<size_t>(n_hid));
+    h2.alloc(sizeof(float) * dm.rows * static_cast<size_t>(n_hid));
+  }
+  const int parts = fused ? net.parts : 1;
+  y.upload(std::vector<float>(static_cast<size_t>(parts) * dm.rows * n_out, 0.f));
   q.dev.clos = y.as<float>();
   q.dev.clos_lo = dm.lo;
   q.dev.clos_n = dm.n_ado;
-  // per-ADO rows of a network that fits: one fused launch per operator pass
-  fused = layout == HEOM_CLOSURE_PER_ADO && closure_mlp_fits(n_in, n_hid, n_out);
+  q.dev.clos_parts = parts;
+  net.x = x.as<float>();
+  net.W1 = W1.as<float>();
+  net.b1 = b1.as<float>();
+  net.W2 = W2.as<float>();
+  net.b2 = b2.as<float>();
+  net.W3 = W3.as<float>();
+  net.b3 = b3.as<float>();
+  net.y = y.as<float>();
 }
 
 void Closure::forward(const Qme& q, const StageArgs& A, hipStream_t st) {
   const int n_in = dm.n_in, n_out = dm.n_out, rows = dm.rows;
   if (fused) {
-    launch_closure_mlp(q.dev, A, x.as<float>(), n_in, n_hid, n_out, W1.as<float>(),
-                       b1.as<float>(), W2.as<float>(), b2.as<float>(), W3.as<float>(),
-                       b3.as<float>(), y.as<float>(), st);
+    launch_closure_mlp(q.dev, A, net, st);
     return;
   }
   launch_closure_gather(q.dev, A, x.as<float>(), dm.ado_stride, st);

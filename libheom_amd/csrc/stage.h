@@ -271,8 +271,11 @@ __device__ __forceinline__ void add_closure(const FormDev& d, long long gi, cx<R
   if (r < 0 || r >= d.clos_n) return;
   const int e = static_cast<int>(gi - a * d.N2);
   const float* y = d.clos + static_cast<long long>(r) * 2 * d.N2;
-  D.re += static_cast<R>(y[e]);
-  D.im += static_cast<R>(y[d.N2 + e]);
+  for (int p = 0; p < d.clos_parts; ++p) {
+    D.re += static_cast<R>(y[e]);
+    D.im += static_cast<R>(y[d.N2 + e]);
+    y += static_cast<long long>(d.clos_n) * 2 * d.N2;
+  }
 }
 // Partial sum of the error norm of one wavefront (no workgroup barrier),
 // written to slot `slot`.

@@ -225,6 +225,40 @@ def test_bound_closure_matches_network_on_the_same_rows():
         q.set_closure(None)
 
 
+@pytest.mark.parametrize("N, depth, n_hid, n_feat, dtype", [
+    (4, 3, 256, 9, "complex128"),   # 120 rows: four workgroups per row block
+    (4, 6, 64, 9, "complex128"),    # 1716 rows: two
+    (4, 7, 32, 0, "complex64"),     # 3432 rows: one
+    (2, 1, 1, 0, "complex128"), (3, 2, 16, 3, "complex64"), (5, 2, 100, 11, "complex128"),
+    (6, 2, 48, 40, "complex128"),   # 124 inputs, 72 outputs
+    (8, 1, 80, 0, "complex64"),     # 144 inputs: the unfused layers
+    (4, 2, 300, 0, "complex128")])  # 300 units: the unfused layers
+def test_bound_network_at_tile_and_part_edges(N, depth, n_hid, n_feat, dtype):
+    """The network inside an operator pass, for widths at the edges of its 16-wide
+    tiles and row counts on every side of the workgroup-sharing rule, against the
+    float64 restatement on the same rows (FP32 sums of up to 256 products of order
+    1: errors of some 1e-6; the operator in FP32: 1e-6 of its largest entry)."""
+    m = configs.chain4(5, max_depth=depth, N=N)
+    q0 = H.heom_hilb(depth, dtype=dtype).load(m, eng())
+    q = H.heom_hilb(depth, dtype=dtype).load(m, eng())
+    feat = np.linspace(-1.0, 1.0, n_feat).astype(np.float32)
+    rows, n_in, n_out = C.dims(q, 0, n_feat)
+    net, sc, rng = small_net(seed=7, n_in=n_in, n_hid=n_hid, n_out=n_out)
+    q.set_closure(net, feat)
+    rho = (rng.normal(size=q.main_size()) + 1j * rng.normal(size=q.main_size())) * 0.3
+    plain = q0.calc_diff_impl(None, np.zeros_like(rho), rho, 1.0, 0.0)
+    got = q.calc_diff_impl(None, np.zeros_like(rho), rho, 1.0, 0.0)
+    idx = q.hrchy_tables()[0]
+    blocks = rho.reshape(-1, N * N)[-rows:]
+    X = np.concatenate([blocks.real, blocks.imag, idx[-rows:],
+                        np.tile(feat.astype(np.float64), (rows, 1))], 1)
+    y = MO.forward(net.get_params().astype(np.float64), n_in, n_hid, n_out, X, sc)
+    ref = plain.copy().reshape(-1, N * N)
+    ref[-rows:] -= y[:, :N * N] + 1j * y[:, N * N:]
+    err = np.abs(got.reshape(-1, N * N) - ref).max()
+    assert err <= 2e-5 * max(1.0, np.abs(ref).max())
+
+
 def test_trained_closure_recovers_the_dropped_term():
     """What training gains: on held-out models' deep states the trained network
     recovers part of the tier-(L+1) term that plain truncation drops (plain
