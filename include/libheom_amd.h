@@ -281,8 +281,9 @@ int heom_solver_reset(heom_solver_handle s); /* forget dt_save (adaptive_step_si
  * (diagonal V, FP64, at most 1024 elements -- 960 for Dormand-Prince -- and at
  * most 8 links per ADO) or a small redfield_hilb problem (diagonal V, FP64,
  * its tables within LDS) in resident launches with the state in LDS: one per
- * RK4 / lsrk4 output interval, or one per heom_solve_dev call (RK4, lsrk4 and
- * Dormand-Prince with the step control on the device); 0: launch every stage
+ * output interval (RK4, lsrk4; Dormand-Prince for a heom_hilb problem of 1, 2 or
+ * 4 levels), or one per heom_solve_dev call (RK4, lsrk4 and Dormand-Prince with
+ * the step control on the device); 0: launch every stage
  * kernel directly.  Fixed-step results are identical either way; Dormand-Prince
  * sums its error norm in another order, so a borderline attempt may be decided
  * differently (the states agree within the tolerance).  No counterpart in the

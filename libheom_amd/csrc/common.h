@@ -291,7 +291,7 @@ struct ResidentStage {
 };
 // The stage programs of rk4 and lsrk4 as the solver builds them (slots
 // renumbered by first use: rk4 y, sa, acc, sb; lsrk4 y, y_new, buff), compiled
-// into the resident kernel; the solver checks its own program against them.
+// into the resident kernel.
 struct ResidentProg {
   int n_stages, n_buf;
   ResidentStage st[4];
@@ -310,9 +310,6 @@ constexpr ResidentProg kResidentLsrk4{
      {1, 2, {1, 2, 0, 0}, 2, {{1.0, 1.0 / 4.0 * -1.0, 0, 0}, {0.0, -1.0, 0, 0}}, {1.0 / 4.0, 1.0}, {0, 2}}}};
 
 struct ResidentArgs {
-  int n_stages, n_buf;
-  ResidentStage st[4];
-  const ResidentStage* prog;  // the same program in device memory (read by the kernel)
   z128* y;          // the FP64 state in HBM (read at the start, written at the end)
   long long n_full; // steps of dt, then one step of dt_last
   double dt, dt_last;
@@ -323,7 +320,7 @@ struct ResidentArgs {
   const long long* n_full_i;
   const double* dt_last_i;
   z128* rho_s;
-  int scheme;  // 0: the program at prog; 1: kResidentRk4; 2: kResidentLsrk4
+  int scheme;  // 0: none (the problem does not qualify); 1: kResidentRk4; 2: kResidentLsrk4
 };
 
 // Resident Dormand-Prince: the whole solve of a small problem in one launch
@@ -334,10 +331,12 @@ constexpr int kResidentDopriMax = 960;
 struct ResidentDopriArgs {
   z128* y;               // FP64 state in HBM (read at the start, written at the end)
   int n_int;             // output intervals
-  const double* t_list;  // n_int + 1 output times, device memory
+  const double* t_list;  // n_int + 1 output times, device memory (null: t0, t1)
+  double t0, t1;
+  int tree;              // order of the error norm's wave sums (see the kernel)
   double dt_first;       // dt of the first attempt (dt_save, else the caller's dt)
   double atol, rtol, inv_n;
-  z128* rho_s;           // rho_S at the n_int + 1 output times
+  z128* rho_s;           // rho_S at the n_int + 1 output times (may be null)
   Ctrl* ctrl;            // the final control block (counters, dt_save, any give-up)
 };
 

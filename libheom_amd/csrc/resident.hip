@@ -17,12 +17,15 @@ namespace {
 // ---------------------------------------------------------------------------
 // One lane's element of a resident problem: the link coefficients and
 // neighbour elements (computed once) and the operator D at that element.
-template <int MAXL>
+// NS: the number of levels (0: any); KH (two levels): the lane keeps its row and
+// column of H.
+template <int MAXL, int NS, bool KH = false>
 struct ResidentElem {
   int g, i, j, nl;
   z128 diag;
   int nbr[MAXL];
   z128 cf[MAXL];
+  z128 hr[KH ? 2 : 1], hc[KH ? 2 : 1];
 
   __device__ __forceinline__ void init(const FormDev& d, int e, bool ok) {
     const int N = d.N, N2 = d.N2;
@@ -33,6 +36,13 @@ struct ResidentElem {
     const int l0 = d.link_ptr[g], l1 = d.link_ptr[g + 1];
     nl = ok ? l1 - l0 : 0;
     diag = d.gam[g] + d.dterm[ee];
+    if constexpr (KH) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        hr[k] = d.H[i * 2 + k];
+        hc[k] = d.H[k * 2 + j];
+      }
+    }
 #pragma unroll
     for (int l = 0; l < MAXL; ++l) {
       nbr[l] = 0;
@@ -58,20 +68,39 @@ struct ResidentElem {
     for (int x = threadIdx.x; x < d.N2; x += blockDim.x) tab[x] = d.H[x];
   }
 
-  // D at element e of the state X (same expression order as hilb_fast_kernel)
-  __device__ __forceinline__ z128 op(const z128* X, const z128* s_H, int e, int N, int N2) const {
+  // D at element e of the state X, x its own element (same expression order as
+  // the stage kernels).  AHEAD: every neighbour's load before the first product
+  template <bool AHEAD>
+  __device__ __forceinline__ z128 op(const z128* X, const z128* s_H, z128 x, int n, int n2) const {
+    const int N = NS ? NS : n, N2 = NS ? NS * NS : n2;
     const z128* Xg = X + static_cast<size_t>(g) * N2;
+    z128 xn[MAXL];
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int l = 0; l < MAXL; ++l)
+        if (l < nl) xn[l] = X[nbr[l]];
+    }
     z128 acc{0.0, 0.0};
+    constexpr int U = NS ? NS : 1;
+#pragma unroll U
     for (int k = 0; k < N; ++k) {
-      cmac(acc, s_H[i * N + k], Xg[k * N + j]);
+      z128 h0, h1;
+      if constexpr (KH) {
+        h0 = hr[k];
+        h1 = hc[k];
+      } else {
+        h0 = s_H[i * N + k];
+        h1 = s_H[k * N + j];
+      }
+      cmac(acc, h0, Xg[k * N + j]);
       const z128 t = Xg[i * N + k];
-      cmac(acc, z128{-t.re, -t.im}, s_H[k * N + j]);
+      cmac(acc, z128{-t.re, -t.im}, h1);
     }
     z128 D = times_i(acc);
-    cmac(D, diag, X[e]);
+    cmac(D, diag, x);
 #pragma unroll
     for (int l = 0; l < MAXL; ++l)
-      if (l < nl) cmac(D, cf[l], X[nbr[l]]);
+      if (l < nl) cmac(D, cf[l], AHEAD ? xn[l] : X[nbr[l]]);
     return D;
   }
 };
@@ -106,7 +135,8 @@ struct RedfieldElem {
     j = ee - i * d.N;
     nn = d.n_noise;
   }
-  __device__ __forceinline__ z128 op(const z128* X, const z128* tab, int e, int N, int N2) const {
+  template <bool>
+  __device__ __forceinline__ z128 op(const z128* X, const z128* tab, z128, int N, int N2) const {
     const z128* HL = tab;
     const z128* HR = tab + N2;
     z128 D{0.0, 0.0};
@@ -131,19 +161,40 @@ struct RedfieldElem {
   }
 };
 
-template <class E, int SCHEME>
-__global__ void __launch_bounds__(1024) resident_kernel(const FormDev d, const ResidentArgs a) {
+// LDS buffers of a stage program: one for each slot that some stage reads as
+// its operator input; every other operand stays in the lane's registers.
+constexpr int res_buf(const ResidentProg& P, int slot) {
+  int n = 0;
+  for (int q = 0; q < P.n_buf; ++q) {
+    bool in = false;
+    for (int s = 0; s < P.n_stages; ++s) in = in || P.st[s].in == q;
+    if (q == slot) return in ? n : -1;
+    n += in ? 1 : 0;
+  }
+  return -1;
+}
+
+// What bounds it: one workgroup, a barrier per stage, and between two barriers
+// the LDS reads (own row and column, up to MAXL neighbours), the chain of FP64
+// sums and one LDS write.  With the level count compiled in and every operand
+// but the stage input in registers a stage of the 264-element spin-boson
+// hierarchy takes 0.47 us (0.58 us with rolled loops and all operands in LDS);
+// what is left is FP64 issue: some 80 instructions of 4 cycles per wavefront, two
+// wavefronts on one SIMD.
+template <class E, int SCHEME, int BS>
+__global__ void __launch_bounds__(BS) resident_kernel(const FormDev d, const ResidentArgs a) {
   extern __shared__ __align__(16) unsigned char res_lds[];
+  constexpr const ResidentProg& P = SCHEME == 1 ? kResidentRk4 : kResidentLsrk4;
   z128* buf = reinterpret_cast<z128*>(res_lds);
-  // the stage program: uniform reads through a read-only pointer (scalar loads)
-  const ResidentStage* __restrict__ prog = a.prog;
   const int ms = static_cast<int>(d.main_size);
   const int N = d.N, N2 = d.N2;
-  z128* s_H = buf + static_cast<size_t>(a.n_buf) * ms;  // the element type's tables
+  z128* s_H = buf + static_cast<size_t>(P.n_buf) * ms;  // the element type's tables
   const int e = threadIdx.x;
   const bool ok = e < ms;
-  for (int x = e; x < a.n_buf * ms; x += blockDim.x)
-    buf[x] = x < ms ? a.y[x] : z128{0.0, 0.0};
+  z128 r[4];  // the lane's element of every slot; slot 0: the state
+  r[0] = ok ? a.y[e] : z128{0.0, 0.0};
+  r[1] = r[2] = r[3] = z128{0.0, 0.0};
+  if (ok) buf[e] = r[0];
   E::stage(d, s_H);
   E el;
   el.init(d, e, ok);
@@ -152,148 +203,153 @@ __global__ void __launch_bounds__(1024) resident_kernel(const FormDev d, const R
   for (int iv = 0; iv < n_int; ++iv) {
     const long long n_full = a.n_int > 0 ? a.n_full_i[iv] : a.n_full;
     const double dt_last = a.n_int > 0 ? a.dt_last_i[iv] : a.dt_last;
-    if (a.n_int > 0 && e < N2) a.rho_s[static_cast<size_t>(iv) * N2 + e] = buf[e];
+    if (a.n_int > 0 && e < N2) a.rho_s[static_cast<size_t>(iv) * N2 + e] = r[0];
     const long long n_steps = n_full + 1;
     for (long long step = 0; step < n_steps; ++step) {
       const double dt = step < n_full ? a.dt : dt_last;
-      auto stage = [&](const ResidentStage& st) {
+#pragma unroll
+      for (int s = 0; s < P.n_stages; ++s) {
         if (ok) {
-          const z128 D = el.op(buf + static_cast<size_t>(st.in) * ms, s_H, e, N, N2);
+          const z128 D = el.template op<BS <= 512>(
+              buf + static_cast<size_t>(res_buf(P, P.st[s].in)) * ms, s_H,
+              r[P.st[s].in], N, N2);
           const z128 k{-(dt * D.re - 0.0 * D.im), -(dt * D.im + 0.0 * D.re)};
-          z128 pv[kResidentPre];
+          z128 v[2];
 #pragma unroll
-          for (int p = 0; p < kResidentPre; ++p)
-            pv[p] = p < st.npre ? buf[static_cast<size_t>(st.pre[p]) * ms + e] : z128{0.0, 0.0};
-          for (int c = 0; c < st.ncombo; ++c) {
-            z128 v{0.0, 0.0};
+          for (int c = 0; c < P.st[s].ncombo; ++c) {
+            v[c] = z128{0.0, 0.0};
 #pragma unroll
-            for (int p = 0; p < kResidentPre; ++p) {
-              if (p < st.npre) {
-                v.re = fma(st.cc[c][p], pv[p].re, v.re);
-                v.im = fma(st.cc[c][p], pv[p].im, v.im);
-              }
+            for (int p = 0; p < P.st[s].npre; ++p) {
+              v[c].re = fma(P.st[s].cc[c][p], r[P.st[s].pre[p]].re, v[c].re);
+              v[c].im = fma(P.st[s].cc[c][p], r[P.st[s].pre[p]].im, v[c].im);
             }
-            v.re = fma(st.ck[c], k.re, v.re);
-            v.im = fma(st.ck[c], k.im, v.im);
-            buf[static_cast<size_t>(st.dst[c]) * ms + e] = v;
+            v[c].re = fma(P.st[s].ck[c], k.re, v[c].re);
+            v[c].im = fma(P.st[s].ck[c], k.im, v[c].im);
+          }
+#pragma unroll
+          for (int c = 0; c < P.st[s].ncombo; ++c) {
+            const int dst = P.st[s].dst[c];
+            r[dst] = v[c];
+            if (res_buf(P, dst) >= 0) buf[static_cast<size_t>(res_buf(P, dst)) * ms + e] = v[c];
           }
         }
         __syncthreads();
-      };
-      if constexpr (SCHEME == 0) {
-        for (int s = 0; s < a.n_stages; ++s) stage(prog[s]);
-      } else {
-        constexpr const ResidentProg& P = SCHEME == 1 ? kResidentRk4 : kResidentLsrk4;
-#pragma unroll
-        for (int s = 0; s < P.n_stages; ++s) stage(P.st[s]);
       }
     }
   }
-  if (a.n_int > 0 && e < N2) a.rho_s[static_cast<size_t>(a.n_int) * N2 + e] = buf[e];
-  if (ok) a.y[e] = buf[e];
+  if (a.n_int > 0 && e < N2) a.rho_s[static_cast<size_t>(a.n_int) * N2 + e] = r[0];
+  if (ok) a.y[e] = r[0];
 }
 
-// Resident Dormand-Prince: the whole adaptive solve of a small heom_hilb
-// problem (diagonal V, FP64) in one workgroup.  Stage arithmetic follows the
-// stage kernels (k = -dt*D; y + sum a_ij k_j as one fma chain in operand order;
-// the error combination and weights of rkdp.h:136-153), the step control is
-// dopri_control on a control block in LDS, and each output interval starts as
-// ctrl_init_kernel does.  The error norm is summed in a fixed order (wavefront
-// shuffles, then the waves in order).  LDS buffers: 0/1 the y / y_new pair
-// (swapped by Ctrl::cur on acceptance), 2..7 k1..k6, 8/9 the stage inputs.
-template <class E>
-__global__ void __launch_bounds__(1024)
+// Resident Dormand-Prince: the adaptive solve of a small heom_hilb problem
+// (diagonal V, FP64) in one workgroup.  Stage arithmetic follows the stage
+// kernels (k = -dt*D; y + sum a_ij k_j as one fma chain in operand order; the
+// error combination and weights of rkdp.h:136-153) and each output interval
+// starts as ctrl_init_kernel does.  Up to 512 elements, where a lane has 256
+// registers, y, y_new and k1..k6 stay in registers; LDS holds the operator
+// inputs: 0/1 the y / y_new pair (swapped on acceptance), 2/3 the stage inputs,
+// and 4..9 the lanes' own k's of the larger problems.  The error norm is summed in a fixed order (wavefront
+// shuffles, then the waves: one after another, or with a.tree as
+// err_finalize_kernel adds the partials of one-wave workgroups).  Up to eight
+// wavefronts every lane runs the step control on it (no round trip through LDS);
+// with more, lane 0 does (all sixteen wavefronts computing the power of the error
+// took 20% of a solve).
+template <class E, int BS>
+__global__ void __launch_bounds__(BS)
     resident_dopri_kernel(const FormDev d, const ResidentDopriArgs a) {
   extern __shared__ __align__(16) unsigned char res_lds[];
-  __shared__ Ctrl s_c;
   __shared__ double s_red[16];
-  __shared__ int s_gave_up;
+  __shared__ Ctrl s_c;
   z128* buf = reinterpret_cast<z128*>(res_lds);
   const int ms = static_cast<int>(d.main_size);
   const int N = d.N, N2 = d.N2;
   z128* s_H = buf + static_cast<size_t>(kResidentDopriBuf) * ms;
   const int e = threadIdx.x;
   const bool ok = e < ms;
-  for (int x = e; x < kResidentDopriBuf * ms; x += blockDim.x)
-    buf[x] = x < ms ? a.y[x] : z128{0.0, 0.0};
+  z128 y = ok ? a.y[e] : z128{0.0, 0.0};
+  if (ok) buf[e] = y;
+  if (e < 16) s_red[e] = 0.0;
   E::stage(d, s_H);
   E el;
   el.init(d, e, ok);
-  if (e == 0) {
-    s_c = Ctrl{};
-    s_c.dt = a.dt_first;
-    s_gave_up = 0;
+  // the control block: in the lane's registers, or (beyond 512 elements) in LDS
+  // and written by lane 0
+  constexpr bool REG = BS <= 512;
+  Ctrl c_reg;
+  Ctrl& c = REG ? c_reg : s_c;
+  const bool owner = REG || e == 0;
+  if (owner) {
+    c = Ctrl{};
+    c.dt = a.dt_first;
   }
+  int gave_up = 0;
   __syncthreads();
-  if (e < N2) a.rho_s[e] = buf[e];
-  z128* K = buf + 2 * static_cast<size_t>(ms);
-  z128* SA = buf + 8 * static_cast<size_t>(ms);
-  z128* SB = buf + 9 * static_cast<size_t>(ms);
+  if (a.rho_s && e < N2) a.rho_s[e] = y;
+  z128* SA = buf + 2 * static_cast<size_t>(ms);
+  z128* SB = buf + 3 * static_cast<size_t>(ms);
+  z128* KL = buf + 4 * static_cast<size_t>(ms);  // k1..k6 beyond 512 elements
   for (int iv = 0; iv < a.n_int; ++iv) {
-    if (e == 0) {  // ctrl_init_kernel: dt carries over from the last attempt
-      const double t0 = a.t_list[iv], t1 = a.t_list[iv + 1];
-      double dt = s_c.dt;
-      s_c.t = t0;
-      s_c.t_bound = t1;
-      s_c.count = 1;
-      s_c.gave_up = 0;
+    // ctrl_init_kernel: dt carries over from the last attempt
+    const double t0 = a.t_list ? a.t_list[iv] : a.t0, t1 = a.t_list ? a.t_list[iv + 1] : a.t1;
+    if (owner) {
+      c.t = t0;
+      c.t_bound = t1;
+      c.count = 1;
+      c.gave_up = 0;
       // a zero-length interval takes no attempt and keeps the step size
-      s_c.done = (t1 > t0) ? 0 : 1;
-      if (!s_c.done) {
-        if (t0 + dt > t1) dt = t1 - t0;
-        s_c.dt = dt;
-      }
+      c.done = (t1 > t0) ? 0 : 1;
+      if (!c.done && t0 + c.dt > t1) c.dt = t1 - t0;
     }
-    __syncthreads();
-    while (!s_c.done) {
-      const double dt = s_c.dt;
-      const int cur = s_c.cur;
+    if (!REG) __syncthreads();
+    while (!c.done) {
+      const double dt = c.dt;
+      const int cur = c.cur;
       const z128* Y = buf + (cur ? ms : 0);
       z128* YN = buf + (cur ? 0 : ms);
+      z128 Kr[REG ? 6 : 1], x = y;  // x (REG): the stage input of the lane's element
+      auto K = [&](int j) -> z128& {
+        if constexpr (REG)
+          return Kr[j];
+        else
+          return KL[static_cast<size_t>(j) * ms + e];
+      };
 #pragma unroll
       for (int st = 0; st < 6; ++st) {
         const z128* in = st == 0 ? Y : ((st & 1) ? SA : SB);
         z128* out = st == 5 ? YN : ((st & 1) ? SB : SA);
         if (ok) {
-          const z128 D = el.op(in, s_H, e, N, N2);
+          const z128 D = el.template op<REG>(in, s_H, REG ? x : in[e], N, N2);
           const z128 k{-(dt * D.re - 0.0 * D.im), -(dt * D.im + 0.0 * D.re)};
-          K[static_cast<size_t>(st) * ms + e] = k;
-          const z128 y = Y[e];
-          z128 v{fma(1.0, y.re, 0.0), fma(1.0, y.im, 0.0)};
-          if (st < 5) {
+          K(st) = k;
+          const z128 y0 = REG ? y : Y[e];
+          z128 v{fma(1.0, y0.re, 0.0), fma(1.0, y0.im, 0.0)};
 #pragma unroll
-            for (int j = 0; j < st; ++j) {
-              const z128 kj = K[static_cast<size_t>(j) * ms + e];
-              v.re = fma(kDpA[st + 1][j], kj.re, v.re);
-              v.im = fma(kDpA[st + 1][j], kj.im, v.im);
+          for (int j = 0; j < st; ++j) {
+            const double w = st < 5 ? kDpA[st + 1][j] : kDpB[j];
+            if (st < 5 || w != 0.0) {
+              const z128 kj = K(j);
+              v.re = fma(w, kj.re, v.re);
+              v.im = fma(w, kj.im, v.im);
             }
-            v.re = fma(kDpA[st + 1][st], k.re, v.re);
-            v.im = fma(kDpA[st + 1][st], k.im, v.im);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 5; ++j) {
-              if (kDpB[j] != 0.0) {
-                const z128 kj = K[static_cast<size_t>(j) * ms + e];
-                v.re = fma(kDpB[j], kj.re, v.re);
-                v.im = fma(kDpB[j], kj.im, v.im);
-              }
-            }
-            v.re = fma(kDpB[5], k.re, v.re);
-            v.im = fma(kDpB[5], k.im, v.im);
           }
+          const double w = st < 5 ? kDpA[st + 1][st] : kDpB[5];
+          v.re = fma(w, k.re, v.re);
+          v.im = fma(w, k.im, v.im);
           out[e] = v;
+          if (REG) x = v;
         }
         __syncthreads();
       }
       double w2 = 0.0;
       if (ok) {
-        const z128 D = el.op(YN, s_H, e, N, N2);
+        const z128 yn = REG ? x : YN[e], yo = REG ? y : Y[e];
+        const z128 D = el.template op<REG>(YN, s_H, yn, N, N2);
         const z128 k{-(dt * D.re - 0.0 * D.im), -(dt * D.im + 0.0 * D.re)};
         z128 er{0.0, 0.0};
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
           if (kDpE[j] != 0.0) {
-            const z128 kj = K[static_cast<size_t>(j) * ms + e];
+            const z128 kj = K(j);
             er.re = fma(kDpE[j], kj.re, er.re);
             er.im = fma(kDpE[j], kj.im, er.im);
           }
@@ -303,31 +359,52 @@ __global__ void __launch_bounds__(1024)
         er.im = fma(0.0, 0.0, er.im);
         er.re = fma(kDpE[6], k.re, er.re);
         er.im = fma(kDpE[6], k.im, er.im);
-        const double a1 = zabs(YN[e]), a0 = zabs(Y[e]);
-        const double w = zabs(er) / (a.atol + a.rtol * (a1 > a0 ? a1 : a0));
+        // |z| with the fma on the part that the stage kernels put it on (a.tree),
+        // so that the norm is theirs to the last bit
+        const double a1 = sqrt(fma(yn.re, yn.re, yn.im * yn.im));
+        const double a0 = sqrt(fma(yo.re, yo.re, yo.im * yo.im));
+        const double e2 = a.tree ? fma(er.im, er.im, er.re * er.re)
+                                 : fma(er.re, er.re, er.im * er.im);
+        const double w = sqrt(e2) / (a.atol + a.rtol * (a1 > a0 ? a1 : a0));
         w2 = w * w;
       }
       for (int off = 32; off > 0; off >>= 1) w2 += __shfl_down(w2, off, 64);
       if ((e & 63) == 0) s_red[e >> 6] = w2;
       __syncthreads();
-      if (e == 0) {
+      // (the next write to s_red comes six barriers later)
+      if (owner) {
         double t = 0.0;
-        for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) t += s_red[w];
-        dopri_control(&s_c, sqrt(t * a.inv_n));
-        if (s_c.gave_up) s_gave_up = 1;
+        if (a.tree) {
+          // the 16-lane shuffle tree; rolled, its operands would take 32 registers
+          double c0 = 0.0, c1 = 0.0;
+#pragma unroll 1
+          for (int w = 0; w < 4; ++w) {
+            const double b = (s_red[w] + s_red[w + 8]) + (s_red[w + 4] + s_red[w + 12]);
+            if (w & 1)
+              c1 += b;
+            else
+              c0 += b;
+          }
+          t = c0 + c1;
+        } else {
+          for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) t += s_red[w];
+        }
+        dopri_control(&c, sqrt(t * a.inv_n));
       }
-      __syncthreads();
+      if (!REG) __syncthreads();
+      if (c.gave_up) gave_up = 1;
+      if (REG && c.cur != cur) y = x;
     }
-    // every wave has read done = 1 before thread 0 rewrites the control block
-    // for the next interval
-    __syncthreads();
-    if (e < N2) a.rho_s[static_cast<size_t>(iv + 1) * N2 + e] = buf[(s_c.cur ? ms : 0) + e];
+    if (!REG && ok) y = buf[(c.cur ? ms : 0) + e];
+    if (a.rho_s && e < N2) a.rho_s[static_cast<size_t>(iv + 1) * N2 + e] = y;
+    // every wave has read the control block before lane 0 starts the next interval
+    if (!REG) __syncthreads();
   }
-  if (ok) a.y[e] = buf[(s_c.cur ? ms : 0) + e];
+  if (ok) a.y[e] = y;
   if (e == 0) {
-    Ctrl c = s_c;
-    c.gave_up = s_gave_up;
-    *a.ctrl = c;
+    Ctrl out = c;
+    out.gave_up = gave_up;
+    *a.ctrl = out;
   }
 }
 
@@ -342,7 +419,7 @@ bool resident_ok(const FormDev& d, int max_links) {
 namespace {
 size_t resident_tab_elems(const FormDev& d) {
   return d.kind == HEOM_REDFIELD_HILB ? RedfieldElem::tab_elems(d.N, d.n_noise)
-                                      : ResidentElem<4>::tab_elems(d.N, d.n_noise);
+                                      : ResidentElem<4, 0>::tab_elems(d.N, d.n_noise);
 }
 }  // namespace
 
@@ -350,36 +427,69 @@ size_t resident_lds_bytes(const FormDev& d, int n_buf) {
   return sizeof(z128) * (static_cast<size_t>(n_buf) * d.main_size + resident_tab_elems(d));
 }
 
+namespace {
+// f(element type tag) for the problem's element type
+template <class E>
+struct Tag {
+  using type = E;
+};
+template <int MAXL, bool KH, class F>
+void with_levels(int N, F f) {
+  if (N == 2) return f(Tag<ResidentElem<MAXL, 2, KH>>{});
+  if (N == 4) return f(Tag<ResidentElem<MAXL, 4>>{});
+  return f(Tag<ResidentElem<MAXL, 0>>{});
+}
+template <bool KH, class F>
+void with_elem(const FormDev& d, int max_links, F f) {
+  if (d.kind == HEOM_REDFIELD_HILB) return f(Tag<RedfieldElem>{});
+  if (max_links <= 4) return with_levels<4, KH>(d.N, f);
+  if (max_links <= 6) return with_levels<6, KH>(d.N, f);
+  return with_levels<8, KH>(d.N, f);
+}
+
+template <class E, int SCHEME, int BS>
+void launch_resident_as(const FormDev& d, const ResidentArgs& a, int bs, size_t lds,
+                        hipStream_t st) {
+  static bool once = (allow_lds(resident_kernel<E, SCHEME, BS>, kResidentLds), true);
+  (void)once;
+  hipLaunchKernelGGL((resident_kernel<E, SCHEME, BS>), dim3(1), dim3(bs), lds, st, d, a);
+}
+
+template <class E, int BS>
+void launch_resident_dopri_as(const FormDev& d, const ResidentDopriArgs& a, int bs, size_t lds,
+                              hipStream_t st) {
+  static bool once = (allow_lds(resident_dopri_kernel<E, BS>, kResidentLds), true);
+  (void)once;
+  hipLaunchKernelGGL((resident_dopri_kernel<E, BS>), dim3(1), dim3(bs), lds, st, d, a);
+}
+}  // namespace
+
+// Up to 512 elements a lane may use 256 registers, beyond 128.
 void launch_resident(const FormDev& d, int max_links, const ResidentArgs& a, hipStream_t stream) {
   const int ms = static_cast<int>(d.main_size);
-  if (!resident_ok(d, max_links) || a.n_stages < 1 || a.n_stages > 4 || a.n_buf < 1 || !a.prog)
+  if (!resident_ok(d, max_links) || (a.scheme != 1 && a.scheme != 2))
     throw HeomError{HEOM_ERR_STATE, "resident integrator: unsupported problem"};
-  const size_t lds = resident_lds_bytes(d, a.n_buf);
+  const int n_buf = a.scheme == 1 ? kResidentRk4.n_buf : kResidentLsrk4.n_buf;
+  const size_t lds = resident_lds_bytes(d, n_buf);
   if (lds > kResidentLds) throw HeomError{HEOM_ERR_STATE, "resident integrator: LDS exceeded"};
   const int bs = ((ms + 63) / 64) * 64;
-#define HAMD_RES(E, S)                                                                \
-  do {                                                                                \
-    static bool once = (allow_lds(resident_kernel<E, S>, kResidentLds), true);        \
-    (void)once;                                                                       \
-    hipLaunchKernelGGL((resident_kernel<E, S>), dim3(1), dim3(bs), lds, stream, d, a); \
-  } while (0)
-#define HAMD_RES_S(E)       \
-  do {                      \
-    if (a.scheme == 1)      \
-      HAMD_RES(E, 1);       \
-    else if (a.scheme == 2) \
-      HAMD_RES(E, 2);       \
-    else                    \
-      HAMD_RES(E, 0);       \
-  } while (0)
-  if (d.kind == HEOM_REDFIELD_HILB)
-    HAMD_RES_S(RedfieldElem);
-  else if (max_links <= 4)
-    HAMD_RES_S(ResidentElem<4>);
-  else
-    HAMD_RES_S(ResidentElem<8>);
-#undef HAMD_RES_S
-#undef HAMD_RES
+  if (bs <= 512) {
+    with_elem<true>(d, max_links, [&](auto tag) {
+      using E = typename decltype(tag)::type;
+      if (a.scheme == 1)
+        launch_resident_as<E, 1, 512>(d, a, bs, lds, stream);
+      else
+        launch_resident_as<E, 2, 512>(d, a, bs, lds, stream);
+    });
+  } else {
+    with_elem<false>(d, max_links, [&](auto tag) {
+      using E = typename decltype(tag)::type;
+      if (a.scheme == 1)
+        launch_resident_as<E, 1, 1024>(d, a, bs, lds, stream);
+      else
+        launch_resident_as<E, 2, 1024>(d, a, bs, lds, stream);
+    });
+  }
   HAMD_HIP(hipGetLastError());
 }
 
@@ -396,19 +506,14 @@ void launch_resident_dopri(const FormDev& d, int max_links, const ResidentDopriA
   const size_t lds = resident_lds_bytes(d, kResidentDopriBuf);
   if (lds > kResidentLds) throw HeomError{HEOM_ERR_STATE, "resident Dormand-Prince: LDS exceeded"};
   const int bs = ((ms + 63) / 64) * 64;
-#define HAMD_RDP(E)                                                                      \
-  do {                                                                                   \
-    static bool once = (allow_lds(resident_dopri_kernel<E>, kResidentLds), true);        \
-    (void)once;                                                                          \
-    hipLaunchKernelGGL((resident_dopri_kernel<E>), dim3(1), dim3(bs), lds, stream, d, a); \
-  } while (0)
-  if (d.kind == HEOM_REDFIELD_HILB)
-    HAMD_RDP(RedfieldElem);
-  else if (max_links <= 4)
-    HAMD_RDP(ResidentElem<4>);
+  if (bs <= 512)
+    with_elem<true>(d, max_links, [&](auto tag) {
+      launch_resident_dopri_as<typename decltype(tag)::type, 512>(d, a, bs, lds, stream);
+    });
   else
-    HAMD_RDP(ResidentElem<8>);
-#undef HAMD_RDP
+    with_elem<false>(d, max_links, [&](auto tag) {
+      launch_resident_dopri_as<typename decltype(tag)::type, 1024>(d, a, bs, lds, stream);
+    });
   HAMD_HIP(hipGetLastError());
 }
 

@@ -261,64 +261,43 @@ void Solver::build_stages(double atol, double rtol) {
   }
 }
 
-// The fixed-step stage program in LDS-buffer form for the resident integrator
-// (slot SL_Y -> buffer 0, the other slots in order of first use).
+// Whether (and with which compiled-in stage program) the resident integrator
+// runs this fixed-step problem.
 void Solver::build_resident() {
   res = ResidentArgs{};
   if (!use_graphs || kind == HEOM_RKDP || in_bytes != 8 || q->opt.renorm_rho0 ||
       !resident_ok(q->dev, q->dev.max_links))
     return;
-  std::map<int, int> bmap{{SL_Y, 0}};
-  auto b = [&](int slot) {
-    auto it = bmap.find(slot);
-    if (it != bmap.end()) return it->second;
-    const int id = static_cast<int>(bmap.size());
-    bmap[slot] = id;
-    return id;
-  };
-  ResidentArgs r{};
-  r.n_stages = static_cast<int>(specs.size());
-  if (r.n_stages > 4) return;
-  for (int s = 0; s < r.n_stages; ++s) {
-    const StageSpec& sp = specs[s];
-    if (static_cast<int>(sp.pre.size()) > kResidentPre || sp.ncombo > 2 || sp.k_slot >= 0 ||
-        sp.do_err)
-      return;
-    ResidentStage& t = r.st[s];
-    t.in = b(sp.in_slot);
-    t.npre = static_cast<int>(sp.pre.size());
-    for (int p = 0; p < t.npre; ++p) t.pre[p] = b(sp.pre[p]);
-    t.ncombo = sp.ncombo;
-    for (int c = 0; c < sp.ncombo; ++c) {
-      for (int p = 0; p < t.npre; ++p) t.cc[c][p] = sp.cc[c][p];
-      t.ck[c] = sp.ck[c];
-      t.dst[c] = b(sp.dst[c]);
-      if (sp.dst2[c] >= 0) return;
-    }
-  }
-  r.n_buf = static_cast<int>(bmap.size());
-  if (resident_lds_bytes(q->dev, r.n_buf) > kResidentLds) return;
-  std::vector<ResidentStage> prog(r.st, r.st + r.n_stages);
-  d_res_prog.upload(prog);
-  r.prog = d_res_prog.as<ResidentStage>();
-  // the compiled-in program when the solver's equals it field by field
-  auto same = [&](const ResidentProg& P) {
-    if (P.n_stages != r.n_stages || P.n_buf != r.n_buf) return false;
-    for (int s = 0; s < r.n_stages; ++s) {
-      const ResidentStage &x = P.st[s], &y = r.st[s];
-      if (x.in != y.in || x.npre != y.npre || x.ncombo != y.ncombo) return false;
-      for (int p = 0; p < x.npre; ++p)
-        if (x.pre[p] != y.pre[p]) return false;
-      for (int c = 0; c < x.ncombo; ++c) {
-        if (x.ck[c] != y.ck[c] || x.dst[c] != y.dst[c]) return false;
-        for (int p = 0; p < x.npre; ++p)
-          if (x.cc[c][p] != y.cc[c][p]) return false;
-      }
-    }
-    return true;
-  };
-  r.scheme = same(kResidentRk4) ? 1 : same(kResidentLsrk4) ? 2 : 0;
-  res = r;
+  const ResidentProg& P = kind == HEOM_RK4 ? kResidentRk4 : kResidentLsrk4;
+  if (resident_lds_bytes(q->dev, P.n_buf) > kResidentLds) return;
+  res.scheme = kind == HEOM_RK4 ? 1 : 2;
+}
+
+// One Dormand-Prince interval of a small problem in one resident launch, as
+// rkdp_interval: the state stays in slot SL_Y, the control block's counters add
+// up over the intervals.
+int Solver::rkdp_interval_resident(double t0, double t1, double dt_first, double atol,
+                                   double rtol) {
+  ResidentDopriArgs a{};
+  a.y = static_cast<z128*>(P[SL_Y].p);
+  a.n_int = 1;
+  a.t0 = t0;
+  a.t1 = t1;
+  a.tree = 1;
+  a.dt_first = dt_first;
+  a.atol = atol;
+  a.rtol = rtol;
+  a.inv_n = 1.0 / static_cast<double>(ms);
+  a.ctrl = d_ctrl.as<Ctrl>();
+  launch_resident_dopri(q->dev, q->dev.max_links, a, q->stream);
+  const Ctrl before = *h_ctrl;
+  HAMD_HIP(hipMemcpyAsync(h_ctrl, d_ctrl.p, sizeof(Ctrl), hipMemcpyDeviceToHost, q->stream));
+  HAMD_HIP(hipStreamSynchronize(q->stream));
+  h_ctrl->cur = 0;
+  h_ctrl->attempts += before.attempts;
+  h_ctrl->accepted += before.accepted;
+  h_ctrl->rejected += before.rejected;
+  return h_ctrl->gave_up;
 }
 
 // rho_0 projection after a step / attempt (heom_options.renorm_rho0)
@@ -410,7 +389,7 @@ void Solver::rk4_interval(double t0, double t1, double dt) {
   long long n_full = 0;
   double dt_1 = dt;
   fixed_steps(t0, t1, dt, n_full, dt_1);
-  if (res.n_stages > 0) {  // the whole interval in one launch
+  if (res.scheme != 0) {  // the whole interval in one launch
     ResidentArgs a = res;
     a.y = static_cast<z128*>(P[SL_Y].p);
     a.n_full = n_full;
@@ -514,9 +493,18 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
     on_output(n_t - 1, P[SL_Y].p);
     HAMD_HIP(hipMemcpyAsync(rho_dev, P[SL_Y].p, bytes, hipMemcpyDeviceToDevice, st));
   } else {
+    // Small problems: an interval per resident launch.  The levels for which a
+    // wavefront holds the same ADOs as a workgroup of the stage kernels: the
+    // error norm is then the same sum, so the steps are decided alike (spin-boson
+    // depth 6, ten intervals: 4.7 ms with the stage kernels, 0.8 ms here).
+    const bool resident = use_graphs && in_bytes == 8 && !q->opt.renorm_rho0 &&
+                          q->kind == HEOM_HILB && (q->N == 1 || q->N == 2 || q->N == 4) &&
+                          resident_dopri_ok(q->dev, q->dev.max_links);
     std::memset(h_ctrl, 0, sizeof(Ctrl));
-    HAMD_HIP(hipMemcpyAsync(ctrl_dev(), h_ctrl, sizeof(Ctrl), hipMemcpyHostToDevice, st));
-    HAMD_HIP(hipStreamSynchronize(st));
+    if (!resident) {
+      HAMD_HIP(hipMemcpyAsync(ctrl_dev(), h_ctrl, sizeof(Ctrl), hipMemcpyHostToDevice, st));
+      HAMD_HIP(hipStreamSynchronize(st));
+    }
     double first = dt_save > 0.0 ? dt_save : dt;
     int batch = 4;
     int cur = 0;
@@ -526,7 +514,11 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
       // a zero-length interval takes no attempt and keeps the step size (the
       // reference would clamp the step to 0 and never finish the next interval)
       if (!(t_list[i + 1] > t_list[i])) continue;
-      gave_up |= rkdp_interval(t_list[i], t_list[i + 1], started ? -1.0 : first, batch);
+      if (resident)
+        gave_up |= rkdp_interval_resident(t_list[i], t_list[i + 1], started ? h_ctrl->dt : first,
+                                          atol, rtol);
+      else
+        gave_up |= rkdp_interval(t_list[i], t_list[i + 1], started ? -1.0 : first, batch);
       started = true;
       cur = h_ctrl->cur;
     }
@@ -567,7 +559,7 @@ int Solver::solve_gather(void* rho_dev, const double* t_list, int n_t, double dt
   HAMD_HIP(hipSetDevice(q->opt.device));
   build_stages(atol, rtol);
   build_resident();
-  if (res.n_stages == 0) {
+  if (res.scheme == 0) {
     reset_graphs();
     return solve(rho_dev, t_list, n_t, dt, atol, rtol, [&](int i, const void* cur) {
       HAMD_HIP(hipMemcpyAsync(static_cast<char*>(rho_s_dev) + rs_bytes * i, cur, rs_bytes,

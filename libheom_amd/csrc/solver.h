@@ -126,10 +126,10 @@ class Solver {
   void capture(GraphExec& g, F&& body);
   void reset_graphs();
   void rk4_interval(double t0, double t1, double dt);
-  // resident integrator (small heom_hilb problems): stage program built by
-  // build_stages when the problem qualifies, else n_stages == 0
+  // resident integrator (small problems): scheme != 0 when the problem qualifies
   ResidentArgs res{};
-  DevBuf d_res_prog, d_res_nf, d_res_dl, d_res_t;
+  DevBuf d_res_nf, d_res_dl, d_res_t;
+  int rkdp_interval_resident(double t0, double t1, double dt_first, double atol, double rtol);
   int solve_resident_dopri(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
                            double rtol, void* rho_s_dev);
   // fixed_step_size_solver::solve_1's step sequence over [t0, t1]: n_full steps

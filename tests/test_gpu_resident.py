@@ -113,6 +113,40 @@ def test_dopri_resident_matches_oracle(case):
     assert np.abs(rho - rho_d).max() <= 1e-12 * scale
 
 
+@pytest.mark.parametrize("n_pade, depth", [
+    (1, 0), (1, 1), (1, 6),   # one ADO, one wavefront, two
+    (1, 14), (1, 15),         # 480 and 544 elements: both sides of 512
+    (1, 20),                  # 924 elements, fifteen wavefronts
+    (2, 8), (3, 6)])          # up to 6 and 8 links per ADO
+@pytest.mark.parametrize("solver", ["rk4", "rkdp"])
+def test_host_solve_runs_interval_by_interval(n_pade, depth, solver):
+    """solve() with a callback: a small problem's output interval is one resident
+    launch.  Same counts as the stage kernels (set_graphs(False)), states within
+    their rounding, the oracle's states within the FP64 bar, rho_S in the
+    caller's array at every output, a zero-length interval among them."""
+    m = configs.spin_boson(max_depth=depth, n_pade=n_pade, T=0.6)
+    t = np.array([0.0, 0.1, 0.1, 0.35, 0.5])
+    kw = {"dt": 0.02, "atol": 1e-10, "rtol": 1e-8}
+    out = []
+    for graphs in (True, False):
+        g = H.heom_hilb(depth).load(m, eng())
+        s = H.qme_solver(eng(), g, getattr(H, solver)())
+        s.set_graphs(graphs)
+        rho, seen = m["rho0"].copy(), []
+        s.solve(rho, t, lambda tt: seen.append((tt, rho[:4].copy())), kw)
+        assert [x[0] for x in seen] == list(t)
+        out.append((rho, np.array([x[1] for x in seen]), s.stats()))
+    (r1, s1, st1), (r0, s0, st0) = out
+    for k in ("n_rhs", "n_attempts", "n_accepted", "n_rejected"):
+        assert st1[k] == st0[k], k
+    assert np.abs(r1 - r0).max() <= 1e-12 and np.abs(s1 - s0).max() <= 1e-12
+    o = O.Oracle(O.HILB, 2, depth).load(m)
+    rho_o, rs_o, st_o, _, _ = o.solve(m["rho0"], t, getattr(O, solver.upper()), kw["dt"],
+                                      kw["atol"], kw["rtol"])
+    assert np.abs(r1 - rho_o).max() <= TOL
+    assert np.abs(s1 - rs_o.reshape(s1.shape)).max() <= TOL
+
+
 def test_dopri_resident_dt_save_carries_over():
     """dt_save of one solve seeds the next (adaptive_step_size_solver.h:39-41, 55)."""
     m = configs.spin_boson(max_depth=4)
