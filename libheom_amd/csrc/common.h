@@ -185,7 +185,9 @@ constexpr int kBatch = 16;  // Qme / FormDev kind of a packed batch (not a publi
 
 // Operator tables of one QME in device memory.
 struct FormDev {
-  int kind;  // public kind (HEOM_HILB .. HEOM_REDFIELD_LIOU) or kBatch
+  // kernel family: HEOM_HILB (also heom_liou and heom_ado, see Qme::upload),
+  // HEOM_REDFIELD_HILB, HEOM_REDFIELD_LIOU or kBatch
+  int kind;
   int N, N2, n_hrchy, n_noise;
   long long main_size;
   const int* link_ptr;   // n_hrchy+1
@@ -206,11 +208,7 @@ struct FormDev {
   // (v_i - v_j, v_i + v_j); real V stores the pair as (re, im) of one z128,
   // complex V as two z128
   const z128* cmac_tab;
-  // liou: CSR superoperators (N2 x N2): R0, then Phi_u, Psi_u
-  const int* sop_ptr;    // (1 + 2*n_noise) * (N2 + 1)
-  const int* sop_col;
-  const z128* sop_val;
-  // ado: global CSR
+  // redfield_liou: the superoperator as CSR
   const long long* R_ptr;
   const int* R_col;
   const z128* R_val;

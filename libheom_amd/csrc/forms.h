@@ -19,10 +19,6 @@ int launch_hilb_mfma_dense(const FormDev& d, const StageArgs& A, hipStream_t st)
 template <typename R, bool F64>
 int launch_batch(const FormDev& d, const StageArgs& A, hipStream_t st);
 template <typename R, bool F64>
-int launch_liou(const FormDev& d, const StageArgs& A, hipStream_t st);
-template <typename R, bool F64>
-int launch_ado(const FormDev& d, const StageArgs& A, hipStream_t st);
-template <typename R, bool F64>
 int launch_redfield(const FormDev& d, const StageArgs& A, hipStream_t st);
 
 #define HAMD_FORM_INSTANCES(f)                                              \

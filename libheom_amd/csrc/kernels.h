@@ -7,6 +7,8 @@ namespace hamd {
 
 constexpr int kMaxGrid = 1 << 18;  // grid cap = partial-sum slots of the error norm
 
+constexpr size_t kMfmaLdsCap = 150 * 1024;  // dynamic LDS the matrix-core kernels may use
+
 // Redfield Hilbert form: LDS elements (complex, operator precision) the
 // one-workgroup kernel stages -- rho, H or HL, HR (a block kept for both), per
 // noise Lambda_u and Lambda_u^+ (and V_u for dense V), then the diagonals of V

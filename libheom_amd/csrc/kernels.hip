@@ -132,10 +132,6 @@ int launch_form(const FormDev& d, const StageArgs& A, hipStream_t st) {
   switch (d.kind) {
     case HEOM_HILB:
       return launch_hilb<R, F64>(d, A, st);
-    case HEOM_LIOU:
-      return launch_liou<R, F64>(d, A, st);
-    case HEOM_ADO:
-      return launch_ado<R, F64>(d, A, st);
     case kBatch:
       return launch_batch<R, F64>(d, A, st);
     default:

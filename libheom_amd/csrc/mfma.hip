@@ -76,7 +76,6 @@ __device__ __forceinline__ mf_f4 mac3(const Split8& a, const Split8& b, mf_f4 c)
 }
 
 constexpr int kMfmaBS = 256;
-constexpr size_t kMfmaLdsCap = 150 * 1024;  // dynamic LDS the matrix-core kernel may use
 
 // Coefficient of a neighbour element at (i, j) with the diagonals of every V_u
 // in LDS (sv: n_noise + 1 rows of n, the last row zero; real V as R, complex V

@@ -244,18 +244,8 @@ void Qme::set_param() {
   H_work_ = Hw;
   build_links();
 
-  // superoperators for heom_liou / heom_ado (heom_liou.h:66-107)
-  std::vector<std::vector<std::map<int, z128>>> ops;
-  std::vector<int> sop_ptr, sop_col;
-  std::vector<z128> sop_val;
-  if (kind == HEOM_LIOU || kind == HEOM_ADO) {
-    if (N > 32) throw HeomError{HEOM_ERR_UNSUPPORTED, "heom_liou/heom_ado: n_level > 32"};
-    build_superops(sop_ptr, sop_col, sop_val, ops);
-  }
-  if (kind == HEOM_ADO) build_ado(ops);
-  sop_ptr_ = std::move(sop_ptr);
-  sop_col_ = std::move(sop_col);
-  sop_val_ = std::move(sop_val);
+  if ((kind == HEOM_LIOU || kind == HEOM_ADO) && N > 32)
+    throw HeomError{HEOM_ERR_UNSUPPORTED, "heom_liou/heom_ado: n_level > 32"};
   upload();
   ready = true;
 }
@@ -382,138 +372,6 @@ std::vector<BlockMap> Qme::build_block_map() const {
   return map;
 }
 
-void Qme::build_superops(std::vector<int>& ptr, std::vector<int>& col, std::vector<z128>& val,
-                         std::vector<std::vector<std::map<int, z128>>>& ops) {
-  const int nn = static_cast<int>(noise_work_.size());
-  SupOp L(N2);
-  kron_x_1(L, kI, H_work_, N);
-  kron_1_x_T(L, zscale(-1.0, kI), H_work_, N);
-  std::vector<SupOp> Phi(nn, SupOp(N2)), Psi(nn, SupOp(N2)), Xi(nn);
-  for (int u = 0; u < nn; ++u) {
-    kron_x_1(Phi[u], kI, noise_work_[u].V, N);
-    kron_1_x_T(Phi[u], zscale(-1.0, kI), noise_work_[u].V, N);
-    optimize(Phi[u]);
-    kron_x_1(Psi[u], kOne, noise_work_[u].V, N);
-    kron_1_x_T(Psi[u], kOne, noise_work_[u].V, N);
-    optimize(Psi[u]);
-    Xi[u] = supop_gemm(zscale(-1.0, noise_work_[u].s_delta), Phi[u], Phi[u]);
-  }
-  SupOp R0(N2);
-  supop_axpy(R0, kOne, L);
-  for (int u = 0; u < nn; ++u) supop_axpy(R0, kOne, Xi[u]);
-  ops.clear();
-  ops.push_back(R0);
-  for (int u = 0; u < nn; ++u) {
-    ops.push_back(Phi[u]);
-    ops.push_back(Psi[u]);
-  }
-  ptr.clear();
-  col.clear();
-  val.clear();
-  for (auto& op : ops) {
-    for (int r = 0; r < N2; ++r) {
-      ptr.push_back(static_cast<int>(col.size()));
-      for (auto& kv : op[r]) {
-        col.push_back(kv.first);
-        val.push_back(kv.second);
-      }
-    }
-    ptr.push_back(static_cast<int>(col.size()));
-  }
-}
-
-void Qme::build_ado(const std::vector<std::vector<std::map<int, z128>>>& ops) {
-  // heom_ado::set_param (heom_ado.h:62-189)
-  const int nn = static_cast<int>(noise_work_.size());
-  const int K = hs.n_dim, nh = hs.n_hrchy, pv = nh;
-  const bool sq = opt.sqrt_norm != 0;
-  const SupOp& R0 = ops[0];
-  std::vector<std::vector<SupOp>> Theta(nn);
-  for (int u = 0; u < nn; ++u) {
-    const SupOp& Phi = ops[1 + 2 * u];
-    const SupOp& Psi = ops[2 + 2 * u];
-    for (int k = 0; k < noise_work_[u].len; ++k) {
-      SupOp T(N2);
-      supop_axpy(T, s[u][k], Phi);
-      supop_axpy(T, zscale(-1.0, a[u][k]), Psi);
-      optimize(T);
-      Theta[u].push_back(std::move(T));
-    }
-  }
-  std::vector<long long> rptr;
-  std::vector<int> rcol;
-  std::vector<z128> rval;
-  rptr.reserve(static_cast<size_t>(nh) * N2 + 1);
-  rptr.push_back(0);
-  std::vector<std::pair<int, z128>> row;
-  for (int l = 0; l < nh; ++l) {
-    const int* nl = &hs.n[static_cast<size_t>(l) * K];
-    for (int a_ = 0; a_ < N2; ++a_) {
-      row.clear();
-      for (int u = 0; u < nn; ++u)
-        for (int k = 0; k < noise_work_[u].len; ++k) {
-          int m = hs.ptr_m1[static_cast<size_t>(l) * K + lk[u][k]];
-          if (m == pv) continue;
-          double nk = nl[lk[u][k]];
-          for (auto& kv : Theta[u][k][a_]) {
-            z128 v = zscale(sq ? std::sqrt(nk) : nk, kv.second);
-            if (!zzero(v)) row.emplace_back(m * N2 + kv.first, v);
-          }
-        }
-      row.emplace_back(l * N2 + a_, ngamma[l]);
-      if (!opt.parity_q1) {
-        for (int u = 0; u < nn; ++u) {
-          const NoiseParams& z = noise_work_[u];
-          for (int j = 0; j < z.len; ++j)
-            for (int k = 0; k < z.len; ++k) {
-              z128 v = z.gamma[j * z.len + k];
-              if (j == k || zzero(v)) continue;
-              int q1 = hs.ptr_m1[static_cast<size_t>(l) * K + lk[u][j]];
-              if (q1 == pv) continue;
-              int q = hs.ptr_p1[static_cast<size_t>(q1) * K + lk[u][k]];
-              if (q == pv) continue;
-              double nj = nl[lk[u][j]], nk = nl[lk[u][k]];
-              row.emplace_back(q * N2 + a_, zscale(sq ? std::sqrt(nj * (nk + 1)) : nj, v));
-            }
-        }
-      }
-      for (auto& kv : R0[a_]) row.emplace_back(l * N2 + kv.first, kv.second);
-      for (int u = 0; u < nn; ++u)
-        for (int k = 0; k < noise_work_[u].len; ++k) {
-          int p = hs.ptr_p1[static_cast<size_t>(l) * K + lk[u][k]];
-          if (p == pv) continue;
-          double nk = nl[lk[u][k]];
-          for (auto& kv : ops[1 + 2 * u][a_]) {
-            z128 v = kv.second;
-            if (sq) v = zscale(std::sqrt(nk + 1), v);
-            v = zmul(v, noise_work_[u].sigma[k]);
-            if (!zzero(v)) row.emplace_back(p * N2 + kv.first, v);
-          }
-        }
-      std::stable_sort(row.begin(), row.end(),
-                       [](const std::pair<int, z128>& x, const std::pair<int, z128>& y) {
-                         return x.first < y.first;
-                       });
-      for (size_t i = 0; i < row.size();) {
-        size_t j = i;
-        z128 acc{0.0, 0.0};
-        while (j < row.size() && row[j].first == row[i].first) {
-          acc = acc + row[j].second;
-          ++j;
-        }
-        rcol.push_back(row[i].first);
-        rval.push_back(acc);
-        i = j;
-      }
-      rptr.push_back(static_cast<long long>(rcol.size()));
-    }
-  }
-  ado_nnz = static_cast<long long>(rcol.size());
-  R_ptr_ = std::move(rptr);
-  R_col_ = std::move(rcol);
-  R_val_ = std::move(rval);
-}
-
 void Qme::upload() {
   const int nn = static_cast<int>(noise_work_.size());
   HAMD_HIP(hipSetDevice(opt.device));
@@ -583,20 +441,20 @@ void Qme::upload() {
   dterm_host = dterm;
   H_host = H_work_;
   d_sdelta.upload(sd);
-  if (!sop_ptr_.empty()) {
-    d_sop_ptr.upload(sop_ptr_);
-    d_sop_col.upload(sop_col_);
-    d_sop_val.upload(sop_val_);
-  }
-  if (!R_ptr_.empty()) {
-    d_R_ptr.upload(R_ptr_);
-    d_R_col.upload(R_col_);
-    d_R_val.upload(R_val_);
-    R_ptr_.clear();
-    R_col_.clear();
-    R_val_.clear();
-  }
-  dev.kind = kind;
+  // heom_liou and heom_ado (heom_liou.h:151-255, heom_ado.h:191-202) apply the
+  // same operator as superoperators of up to N^4 entries (per ADO, or merged over
+  // the hierarchy): a commutator or an anticommutator from the left and the right
+  // is 2 N products per element where the sparse row is 2 N - 1 gathered ones, so
+  // the Hilbert-form kernels compute all three forms.  (160 stages on the 7-site
+  // chain at depth 2: 4.3 ms with per-ADO sparse rows, 1.7 ms here.)
+  const bool hilb = kind == HEOM_HILB || kind == HEOM_LIOU || kind == HEOM_ADO;
+  bool diag = diag_v;
+  // those two forms take any number of noises: past the LDS tables of the diagonal
+  // kernels (see launch_hilb_n) they use the dense one
+  if (hilb && kind != HEOM_HILB && N <= 16 &&
+      sizeof(z128) * (nn + 1) * static_cast<size_t>(N) > 48 * 1024)
+    diag = false;
+  dev.kind = hilb ? HEOM_HILB : kind;
   dev.N = N;
   dev.N2 = N2;
   dev.n_hrchy = hs.n_hrchy;
@@ -611,7 +469,7 @@ void Qme::upload() {
   dev.Vd = d_Vd.as<z128>();
   dev.dterm = d_dterm.as<z128>();
   dev.sdelta = d_sdelta.as<z128>();
-  dev.diag_v = diag_v ? 1 : 0;
+  dev.diag_v = diag ? 1 : 0;
   dev.real_v = real_v ? 1 : 0;
   dev.flat = d_flat.as<LinkFlat>();
   dev.bmap = d_bmap.as<BlockMap>();
@@ -619,21 +477,23 @@ void Qme::upload() {
   dev.max_links = 0;
   for (int l = 0; l < hs.n_hrchy; ++l)
     dev.max_links = std::max(dev.max_links, link_ptr[l + 1] - link_ptr[l]);
-  dev.sop_ptr = d_sop_ptr.as<int>();
-  dev.sop_col = d_sop_col.as<int>();
-  dev.sop_val = d_sop_val.as<z128>();
-  dev.R_ptr = d_R_ptr.as<long long>();
-  dev.R_col = d_R_col.as<int>();
-  dev.R_val = d_R_val.as<z128>();
   // matrix-core commutator: heom_hilb, 16 < N <= 64, diagonal V (tiles of 32 or
   // 64 rows; H is zero-padded to the tile in its planes)
-  const bool big = kind == HEOM_HILB && N > 16 && N <= 64;
+  const bool big = hilb && N > 16 && N <= 64;
   const bool mfma_ok = big && diag_v;
   const bool mfma_dense = big && !diag_v;
   dev.mfma = 0;
   if (opt.matrix_cores && mfma_ok) dev.mfma = dtype == HEOM_C64_BF16X3 ? 2 : 1;
   if (opt.matrix_cores && mfma_dense && dtype != HEOM_C64_BF16X3) dev.mfma = 3;
-  if (dtype == HEOM_C64_BF16X3 && dev.mfma != 2)
+  if (kind != HEOM_HILB) {
+    // heom_liou / heom_ado: matrix_cores = 0 has no vector kernel for dense V, and
+    // many noises leave the LDS tables of the matrix-core kernel
+    if (mfma_dense) dev.mfma = 3;
+    if (mfma_ok && 2 * sizeof(double) * 32 * 33 + sizeof(z128) * (nn + 1) * static_cast<size_t>(N) >
+                       kMfmaLdsCap)
+      dev.mfma = 0;
+  }
+  if (dtype == HEOM_C64_BF16X3 && (dev.mfma != 2 || kind != HEOM_HILB))
     throw HeomError{HEOM_ERR_UNSUPPORTED,
                     "HEOM_C64_BF16X3 is provided for heom_hilb with 16 < n_level <= 64, diagonal "
                     "coupling operators and matrix_cores = 1"};

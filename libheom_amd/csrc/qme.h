@@ -90,9 +90,8 @@ class Qme {
   hipStream_t stream = nullptr;
   DevBuf d_link_ptr, d_links, d_flat, d_cmac, d_coef, d_gam, d_H, d_V, d_Vd, d_dterm, d_sdelta;
   DevBuf d_bmap;
-  DevBuf d_sop_ptr, d_sop_col, d_sop_val;
   DevBuf d_R_ptr, d_R_col, d_R_val;
-  long long ado_nnz = 0;
+  long long csr_nnz = 0;  // redfield_liou
 
   void set_param();
   bool redfield() const { return kind == HEOM_REDFIELD_HILB || kind == HEOM_REDFIELD_LIOU; }
@@ -140,19 +139,11 @@ class Qme {
   // parameters after the col_major transform (identical for row_major)
   std::vector<NoiseParams> noise_work_;
   std::vector<z128> H_work_;
-  std::vector<int> sop_ptr_, sop_col_;
-  std::vector<z128> sop_val_;
-  std::vector<long long> R_ptr_;
-  std::vector<int> R_col_;
-  std::vector<z128> R_val_;
 
   void build_links();
   // Work-unit order of the one-ADO-per-workgroup kernels (see BlockMap)
   std::vector<BlockMap> build_block_map() const;
   void set_param_redfield();
-  void build_superops(std::vector<int>& ptr, std::vector<int>& col, std::vector<z128>& val,
-                      std::vector<std::vector<std::map<int, z128>>>& ops);
-  void build_ado(const std::vector<std::vector<std::map<int, z128>>>& ops);
   void upload();
 };
 

@@ -225,9 +225,6 @@ void Qme::set_param_redfield() {
   real_v = false;
   noise_work_ = nz;
   H_work_ = Hw;
-  sop_ptr_.clear();
-  sop_col_.clear();
-  sop_val_.clear();
 
   std::vector<z128> L(static_cast<size_t>(nn) * N2), Ld(static_cast<size_t>(nn) * N2);
   for (int u = 0; u < nn; ++u) {
@@ -256,20 +253,27 @@ void Qme::set_param_redfield() {
     }
     supop_axpy(R, kOne, Lop);
     optimize(R);
-    R_ptr_.assign(1, 0);
-    R_col_.clear();
-    R_val_.clear();
+    std::vector<long long> ptr(1, 0);
+    std::vector<int> col;
+    std::vector<z128> val;
     for (int r = 0; r < N2; ++r) {
       for (auto& kv : R[r]) {
-        R_col_.push_back(kv.first);
-        R_val_.push_back(kv.second);
+        col.push_back(kv.first);
+        val.push_back(kv.second);
       }
-      R_ptr_.push_back(static_cast<long long>(R_col_.size()));
+      ptr.push_back(static_cast<long long>(col.size()));
     }
-    ado_nnz = static_cast<long long>(R_col_.size());
+    csr_nnz = static_cast<long long>(col.size());
+    HAMD_HIP(hipSetDevice(opt.device));
+    d_R_ptr.upload(ptr);
+    d_R_col.upload(col);
+    d_R_val.upload(val);
   }
 
   upload();
+  dev.R_ptr = d_R_ptr.as<long long>();
+  dev.R_col = d_R_col.as<int>();
+  dev.R_val = d_R_val.as<z128>();
   d_rf_L.upload(L);
   d_rf_Ld.upload(Ld);
   dev.rf_L = d_rf_L.as<z128>();

@@ -498,7 +498,7 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
     // error norm is then the same sum, so the steps are decided alike (spin-boson
     // depth 6, ten intervals: 4.7 ms with the stage kernels, 0.8 ms here).
     const bool resident = use_graphs && in_bytes == 8 && !q->opt.renorm_rho0 &&
-                          q->kind == HEOM_HILB && (q->N == 1 || q->N == 2 || q->N == 4) &&
+                          q->dev.kind == HEOM_HILB && (q->N == 1 || q->N == 2 || q->N == 4) &&
                           resident_dopri_ok(q->dev, q->dev.max_links);
     std::memset(h_ctrl, 0, sizeof(Ctrl));
     if (!resident) {
@@ -724,17 +724,17 @@ void Solver::stage_bytes(std::vector<double>& out) {
   out.assign(ns, 0.0);
   auto size_of = [&](int slot) { return slo[slot] ? 8.0 : 16.0; };
   double tables = 0.0;
-  if (q->kind == HEOM_ADO || q->kind == HEOM_REDFIELD_LIOU) {
-    tables = 20.0 * q->ado_nnz + 8.0 * (ms + 1);
+  if (q->kind == HEOM_REDFIELD_LIOU) {
+    tables = 20.0 * q->csr_nnz + 8.0 * (ms + 1);
   } else if (q->kind == HEOM_REDFIELD_HILB) {
     // H, and V_u, Lambda_u, Lambda_u^+ per noise
     tables = 16.0 * q->N2 * (1.0 + 3.0 * static_cast<double>(q->noise.size()));
   } else {
     // the fast Hilbert kernel (diagonal V, 6 <= N <= 16) reads 8-byte links and
     // the coefficient table, the other diagonal-V Hilbert kernels LinkFlat
-    const bool fast = q->kind == HEOM_HILB && q->diag_v && q->N >= 6 && q->N <= 16;
+    const bool fast = q->dev.kind == HEOM_HILB && q->dev.diag_v && q->N >= 6 && q->N <= 16;
     const double lrec = q->kind == kBatch || fast           ? sizeof(Link)
-                        : (q->kind == HEOM_HILB && q->diag_v) ? sizeof(LinkFlat)
+                        : (q->dev.kind == HEOM_HILB && q->dev.diag_v) ? sizeof(LinkFlat)
                                                                : sizeof(Link);
     tables = lrec * q->n_links + 4.0 * (q->hs.n_hrchy + 1) + 16.0 * q->hs.n_hrchy;
     if (q->kind == kBatch)

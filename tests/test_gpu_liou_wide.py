@@ -56,6 +56,24 @@ def test_wide_calc_diff_parity(form, N, dense_v):
 
 
 @pytest.mark.parametrize("form", ["liou", "ado"])
+@pytest.mark.parametrize("N, n_noise, dense_v, matrix_cores", [
+    (16, 191, False, True), (16, 192, False, True), (5, 620, False, True),  # the LDS table limit
+    (17, 2, True, False), (20, 2, False, False), (20, 425, False, True),
+    (1, 2, False, True), (6, 1, True, True)])
+def test_forms_take_every_size(form, N, n_noise, dense_v, matrix_cores):
+    """Both forms take any number of noises and matrix_cores = 0 for every V: the
+    sizes on both sides of what the diagonal kernels hold in LDS."""
+    cls, okind = FORMS[form]
+    m = configs.random_model(N, n_noise, 1, 1, seed=40 + N, dense_v=dense_v)
+    g = cls(1, matrix_cores=matrix_cores).load(m, eng())
+    o = O.Oracle(O.HILB, N, 1, n_threads=8).load(m)
+    rho = m["rho0"]
+    ref = o.calc_diff(rho)
+    got = g.calc_diff_impl(None, np.zeros_like(rho), rho, 1.0, 0.0)
+    assert np.abs(got - ref).max() <= TOL * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("form", ["liou", "ado"])
 def test_wide_rkdp_solve(form):
     """Dormand-Prince at n_level 20 with dense V (every stage kernel variant):
     the oracle's accepted / rejected counts and its state at 1e-10."""
