@@ -31,7 +31,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-GRAPHS = True  # replay stage sequences from HIP graphs (--no-graphs: direct launches)
+GRAPHS = True  # small problems in resident launches (--no-graphs: every stage launched)
 
 
 def alg_bytes_per_ado_stage(n_level, n_dim, method, sc=16):

@@ -262,9 +262,8 @@ int heom_solve_dev(heom_solver_handle s, void* rho_dev, const double* t_list, in
 /* No counterpart in the reference: heom_solve_dev for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, results and errors as
- * heom_solve_dev with its stage kernels launched directly (no graph replay, no
- * resident integrator), and no hipMalloc / hipFree / graph instantiation on the
- * call: the Dormand-Prince control block, the error-norm partials and rho_S of
+ * heom_solve_dev without the resident integrators, and no hipMalloc / hipFree on
+ * the call: the Dormand-Prince control blocks, the error-norm partials and rho_S of
  * every output time live in one fixed 8 MiB device array per GPU, held until
  * the process ends.  Limit: n_t * n_level^2 * 16 bytes of rho_S <= 6 MiB (for a
  * batch, n_level^2 is the sum over its members); larger requests return
@@ -276,15 +275,13 @@ int heom_solve_dev_noalloc(heom_solver_handle s, void* rho_dev, const double* t_
                            double dt, double atol, double rtol, double* rho_s_out);
 int heom_solver_stats(heom_solver_handle s, heom_stats* out);
 int heom_solver_reset(heom_solver_handle s); /* forget dt_save (adaptive_step_size_solver.h:28) */
-/* 1 (default): replay the fixed stage sequences (RK4 steps of the full dt,
- * Dormand-Prince attempts) from HIP graphs, and run a small heom_hilb problem
- * (diagonal V, FP64, at most 1024 elements -- 960 for Dormand-Prince -- and at
- * most 8 links per ADO) or a small redfield_hilb problem (diagonal V, FP64,
+/* 1 (default): run a small heom_hilb problem (diagonal V, FP64, at most 1024
+ * elements -- 960 for Dormand-Prince -- and at most 8 links per ADO) or a small redfield_hilb problem (diagonal V, FP64,
  * its tables within LDS) in resident launches with the state in LDS: one per
  * output interval (RK4, lsrk4; Dormand-Prince for a heom_hilb problem of 1, 2 or
  * 4 levels), or one per heom_solve_dev call (RK4, lsrk4 and Dormand-Prince with
  * the step control on the device); 0: launch every stage
- * kernel directly.  Fixed-step results are identical either way; Dormand-Prince
+ * kernel.  Fixed-step results are identical either way; Dormand-Prince
  * sums its error norm in another order, so a borderline attempt may be decided
  * differently (the states agree within the tolerance).  No counterpart in the
  * reference. */

@@ -522,6 +522,6 @@ class qme_solver:
         _capi.check(_capi.load().heom_solver_reset(self._s))
 
     def set_graphs(self, enable):
-        """Replay fixed stage sequences from HIP graphs (default) or launch directly."""
+        """Small problems in resident launches (default) or every stage kernel launched."""
         self._graphs = bool(enable)
         _capi.check(_capi.load().heom_solver_set_graphs(self._s, int(bool(enable))))

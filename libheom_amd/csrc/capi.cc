@@ -539,11 +539,13 @@ int heom_solve_dev(heom_solver_handle s, void* rho_dev, const double* t_list, in
     sv.check_qme();
     const bool batch = sv.q->kind == hamd::kBatch;
     const int N2 = batch ? sv.q->batch_rs_size : sv.q->N2;
-    hamd::DevBuf rs;
-    if (rho_s_out) rs.alloc(sizeof(hamd::z128) * N2 * static_cast<size_t>(n_t));
+    if (n_t < 1) throw hamd::HeomError{HEOM_ERR_ARG, "solve: n_t < 1"};
+    hamd::DevBuf own;
+    const size_t rs_bytes = sizeof(hamd::z128) * N2 * static_cast<size_t>(n_t);
+    void* rs = rho_s_out ? sv.workspace(sv.d_rho_s, own, rs_bytes) : nullptr;
     auto out = [&](int i, const void* cur) {
       if (!rho_s_out) return;
-      char* dst = static_cast<char*>(rs.p) + sizeof(hamd::z128) * N2 * i;
+      char* dst = static_cast<char*>(rs) + sizeof(hamd::z128) * N2 * i;
       if (batch)
         hamd::launch_gather_rho_s(sv.q->dev, dst, cur, sv.q->stream);
       else
@@ -551,11 +553,10 @@ int heom_solve_dev(heom_solver_handle s, void* rho_dev, const double* t_list, in
                                 sv.q->stream));
     };
     int rc = (rho_s_out && !batch)
-                 ? sv.solve_gather(rho_dev, t_list, n_t, dt, atol, rtol, rs.p)
+                 ? sv.solve_gather(rho_dev, t_list, n_t, dt, atol, rtol, rs)
                  : sv.solve(rho_dev, t_list, n_t, dt, atol, rtol, out);
     if (rho_s_out)
-      HAMD_HIP(hipMemcpy(rho_s_out, rs.p, sizeof(hamd::z128) * N2 * static_cast<size_t>(n_t),
-                         hipMemcpyDeviceToHost));
+      HAMD_HIP(hipMemcpy(rho_s_out, rs, rs_bytes, hipMemcpyDeviceToHost));
     if (rc != HEOM_OK)
       hamd::set_error(rc, "rkdp: step rejected 1000 times; interval skipped as in the reference");
     return rc;
@@ -601,9 +602,9 @@ int heom_solve(heom_solver_handle s, double* rho_host, const double* t_list, int
     const long long ms = sv.q->main_size();
     const int N2 = sv.q->N2;
     const size_t bytes = sizeof(hamd::z128) * ms;
-    hamd::DevBuf d;
-    d.alloc(bytes);
-    HAMD_HIP(hipMemcpy(d.p, rho_host, bytes, hipMemcpyHostToDevice));
+    hamd::DevBuf own;
+    void* d = sv.workspace(sv.d_state, own, bytes);
+    HAMD_HIP(hipMemcpy(d, rho_host, bytes, hipMemcpyHostToDevice));
     std::vector<double> rs(2 * N2);
     auto out = [&](int i, const void* cur) {
       if (full_copy) {
@@ -617,8 +618,8 @@ int heom_solve(heom_solver_handle s, double* rho_host, const double* t_list, int
         if (cb) cb(t_list[i], rs.data(), nullptr, user);
       }
     };
-    int rc = sv.solve(d.p, t_list, n_t, dt, atol, rtol, out);
-    HAMD_HIP(hipMemcpy(rho_host, d.p, bytes, hipMemcpyDeviceToHost));
+    int rc = sv.solve(d, t_list, n_t, dt, atol, rtol, out);
+    HAMD_HIP(hipMemcpy(rho_host, d, bytes, hipMemcpyDeviceToHost));
     if (rc != HEOM_OK)
       hamd::set_error(rc, "rkdp: step rejected 1000 times; interval skipped as in the reference");
     return rc;
@@ -645,7 +646,7 @@ int heom_solver_reset(heom_solver_handle s) {
 int heom_solver_set_graphs(heom_solver_handle s, int enable) {
   return guard([&] {
     if (!s || !s->s) throw hamd::HeomError{HEOM_ERR_ARG, "null solver handle"};
-    s->s->use_graphs = enable != 0;
+    s->s->use_resident = enable != 0;
     return HEOM_OK;
   });
 }

@@ -75,9 +75,9 @@ struct Link {
   int cid;  // index into the Coef table
 };
 
-// Dormand-Prince control block, resident in device memory.  The last block of
-// the final stage kernel of an attempt updates it (rkdp.h:97-177) so that the
-// host never reads back inside a step.
+// Dormand-Prince control block, resident in device memory.  The pass between two
+// attempts (dopri_step_kernel) updates it (rkdp.h:97-177), so the host never
+// reads back inside a solve.
 struct Ctrl {
   double t, t_bound, dt, err;
   int cur;      // which buffer of each ping-pong pair holds the current state
@@ -86,6 +86,39 @@ struct Ctrl {
   int gave_up;
   long long attempts, accepted, rejected;
   long long projected;  // accepted attempts whose rho_0 the projection has handled
+  int seq;   // step passes since the solve (or the host-driven interval) began
+  int i_int; // output interval, when the device walks through the list of times
+};
+
+// The pass between two Dormand-Prince attempts (dopri_step_kernel): error norm of
+// the attempt that ended, step control, output of finished intervals, and the
+// stage input of the next attempt's second evaluation,
+//   sa = y + a21 * (-dt * D(y)),
+// from D of the current state, which the last stage of the attempt that produced
+// the state has stored: an attempt evaluates the operator six times, not seven.
+enum StepMode { STEP_CONTROL = 1, STEP_FIRST = 2, STEP_INPUT = 4 };
+struct StepArgs {
+  int mode;
+  // the control block is read from prev and written to next (every workgroup
+  // takes the decision for itself); without STEP_CONTROL both are the same
+  const Ctrl* prev;
+  Ctrl* next;
+  const double* partials;
+  int nparts;
+  double inv_n;
+  // output times (device memory) and where rho_S goes at each of them; null: the
+  // host drives one interval at a time
+  const double* t_list;
+  int n_int;
+  z128* rho_s;
+  int n_rs;
+  const z128* y[2];   // by Ctrl::cur
+  const void* D[2];
+  int lo;             // D and sa are complex64
+  void* sa;
+  double a21;
+  long long n;
+  unsigned long long* mail;  // host memory: seq << 2 | last << 1 | done
 };
 
 enum SlotType { ST_C128 = 0, ST_C64 = 1 };
@@ -101,7 +134,8 @@ constexpr int kMaxPre = 8;  // state-sized operands an epilogue may read per ele
 //   pv[s] = pre[cur][s] at this element (loaded before the operator work)
 // MODE_DIFF : dst[0] = beta*pv[0] - alpha*D      (pv[0] = old drho when beta != 0)
 // MODE_STAGE: k = -dt*D (dt from the control block when attached, else a_re)
-//             k[cur] <- k (optional)
+//             k[cur] <- k, or D itself with k_raw (optional)
+//             d_pre: operand 1 holds a stored D; it stands for k_1 = -dt*D
 //             dst[c] (and dst2[c]) <- sum_s cc[c][s]*pv[s] + ck[c]*k, summed in s order
 //             with zero coefficients skipped (so the order follows the reference)
 //   error norm (rkdp.h:142-153): e = sum_s ec[s]*pv[s] + ek*k,
@@ -116,6 +150,8 @@ struct StageArgs {
   unsigned pre_lo;
   void* k[2];  // null: k not stored
   int k_lo;
+  int k_raw;
+  int d_pre;
   int ncombo;
   double cc[2][kMaxPre];
   double ck[2];
@@ -127,11 +163,8 @@ struct StageArgs {
   double ek;
   int ynew_pre, yold_pre;
   double atol, rtol;
-  int control;  // 1: the finalize pass runs the step control
-  double inv_n;
   Ctrl* ctrl;
   double* partials;
-  int max_partials;
 };
 
 // One neighbour link with its coefficients inlined (fast Hilbert kernel):

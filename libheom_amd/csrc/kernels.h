@@ -26,12 +26,14 @@ __host__ __device__ inline size_t redfield_lds_elems(int N2, int N, int n_noise,
 // Returns the grid size used (the number of error-norm partials written).
 int launch_operator(const FormDev& d, int real_bytes, const StageArgs& A, hipStream_t stream);
 
-// Combine the error-norm partials of the last stage pass (nparts = its grid)
-// and run the Dormand-Prince step control.
-void launch_err_finalize(const StageArgs& A, int nparts, hipStream_t stream);
+// The pass between two Dormand-Prince attempts: error norm from the partials of
+// the last stage pass, step control, outputs, next stage input (see StepArgs).
+void launch_dopri_step(const StepArgs& A, hipStream_t stream);
 
-// Set up the Dormand-Prince control block for one output interval.
-void launch_ctrl_init(Ctrl* c, double t0, double t_bound, double dt, hipStream_t stream);
+// Set up the Dormand-Prince control block for output interval i_int: at the
+// start of a solve (dt >= 0) or, with dt < 0, keeping its step size and counters.
+void launch_ctrl_init(Ctrl* c, double t0, double t_bound, double dt, int i_int,
+                      hipStream_t stream);
 
 // rho_S of every member of a batch (d.kind == kBatch), gathered in member
 // order from an FP64 state

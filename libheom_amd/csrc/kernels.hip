@@ -7,7 +7,7 @@
 //   k     = -dt*D  (calc_diff_impl with alpha = dt, beta = 0; rk4.h:48)
 //   y_i+1 = y + sum_j a_ij k_j  (the next stage input, written in the same pass)
 //   e     = sum_j E_j k_j and per-workgroup partial sums of the error norm
-//           (rkdp.h:142-153); err_finalize_kernel reduces them in a fixed
+//           (rkdp.h:142-153); dopri_step_kernel reduces them in a fixed
 //           order and runs the step control on the device (rkdp.h:97-177).
 //
 // Threads map to matrix elements: thread e of an ADO's lane group handles
@@ -20,34 +20,114 @@ namespace hamd {
 
 namespace {
 
-// Sums the partials of the last stage pass in a fixed order (deterministic)
-// and runs the step control (one workgroup of 1024 threads; every thread sums
-// a strided slice with four independent accumulators).
-__global__ void __launch_bounds__(1024) err_finalize_kernel(const StageArgs A, int nparts) {
-  __shared__ double s_red[16];
-  if (A.ctrl && A.ctrl->done) return;
-  double x0 = 0.0, x1 = 0.0, x2 = 0.0, x3 = 0.0;
-  int b = threadIdx.x;
-  for (; b + 3 * 1024 < nparts; b += 4 * 1024) {
-    x0 += A.partials[b];
-    x1 += A.partials[b + 1024];
-    x2 += A.partials[b + 2048];
-    x3 += A.partials[b + 3072];
+// Move the control block on to the next output interval of positive length
+// (an interval of no length takes no attempt and keeps the step size); done
+// stays set after the last one.
+__device__ void next_interval(Ctrl& c, const StepArgs& A) {
+  while (c.i_int < A.n_int) {
+    const int i = ++c.i_int;
+    if (i >= A.n_int) return;
+    const double t0 = A.t_list[i], t1 = A.t_list[i + 1];
+    if (!(t1 > t0)) continue;
+    c.t = t0;
+    c.t_bound = t1;
+    c.done = 0;
+    c.count = 1;
+    if (t0 + c.dt > t1) c.dt = t1 - t0;
+    return;
   }
-  for (; b < nparts; b += 1024) x0 += A.partials[b];
-  double x = (x0 + x1) + (x2 + x3);
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = x;
-  __syncthreads();
+}
+
+// The pass between two Dormand-Prince attempts (see StepArgs).  Every workgroup
+// sums the partials in the same fixed order and takes the step decision for
+// itself (no launch of its own for the decision, no exchange between the
+// workgroups); workgroup 0 writes the control block, rho_S at output times
+// and the host's progress word.  Then a stream over the state: y and D read, the
+// stage input written.  Bound: latency of the reduction (12 650 partials: 101 KB
+// per workgroup from L2), then memory.
+// The next stage input of an element: y + a21 k, k = -dt D.
+template <typename T>
+__device__ __forceinline__ void step_input(const StepArgs& A, const z128* y, const T* D, T* sa,
+                                           double dt) {
+  const z128 alpha{dt, 0.0};
+  const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
+  for (long long x = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; x < A.n;
+       x += stride) {
+    const z128 k = scaled_k(alpha, conv<double>(D[x])), y0 = y[x];
+    z128 v{fma(1.0, y0.re, 0.0), fma(1.0, y0.im, 0.0)};
+    v.re = fma(A.a21, k.re, v.re);
+    v.im = fma(A.a21, k.im, v.im);
+    sa[x] = T{static_cast<decltype(T::re)>(v.re), static_cast<decltype(T::re)>(v.im)};
+  }
+}
+
+constexpr int kStepBS = 1024;
+constexpr int kStepFusedParts = 16384;
+
+__global__ void __launch_bounds__(kStepBS) dopri_step_kernel(const StepArgs A) {
+  __shared__ double s_red[kStepBS / 64];
+  __shared__ Ctrl s_c;
+  __shared__ int s_out[2];  // output times to write: [0] .. [1] - 1
+  const bool decide = (A.mode & STEP_CONTROL) && !(A.mode & STEP_FIRST) && !A.prev->done;
+  if (decide) {
+    double x0 = 0.0, x1 = 0.0, x2 = 0.0, x3 = 0.0;
+    int b = threadIdx.x;
+    for (; b + 3 * kStepBS < A.nparts; b += 4 * kStepBS) {
+      x0 += A.partials[b];
+      x1 += A.partials[b + kStepBS];
+      x2 += A.partials[b + 2 * kStepBS];
+      x3 += A.partials[b + 3 * kStepBS];
+    }
+    for (; b < A.nparts; b += kStepBS) x0 += A.partials[b];
+    double x = (x0 + x1) + (x2 + x3);
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
+    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = x;
+    __syncthreads();
+  }
   if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < 16; ++w) t += s_red[w];
-    double err = sqrt(t * A.inv_n);
-    if (A.control)
-      dopri_control(A.ctrl, err);
-    else if (A.ctrl)
-      A.ctrl->err = err;
+    Ctrl c = *A.prev;
+    s_out[0] = s_out[1] = 0;
+    if (decide) {
+      double t = 0.0;
+      for (int w = 0; w < kStepBS / 64; ++w) t += s_red[w];
+      dopri_control(&c, sqrt(t * A.inv_n));
+      if (c.done && A.t_list) {
+        s_out[0] = c.i_int + 1;
+        next_interval(c, A);
+        s_out[1] = (c.i_int < A.n_int ? c.i_int : A.n_int) + 1;
+      }
+    } else if ((A.mode & STEP_FIRST) && A.t_list) {
+      s_out[1] = c.i_int + 1;
+    }
+    if (A.mode & STEP_CONTROL) {
+      c.seq += 1;
+      if (blockIdx.x == 0) {
+        *A.next = c;
+        if (A.mail) {
+          const bool last =
+              !c.done && !(c.t + c.dt < c.t_bound) && (!A.t_list || c.i_int + 1 >= A.n_int);
+          __hip_atomic_store(A.mail,
+                             static_cast<unsigned long long>(c.seq) << 2 | (last ? 2u : 0u) |
+                                 (c.done ? 1u : 0u),
+                             __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+      }
+    }
+    s_c = c;
   }
+  __syncthreads();
+  const int cur = s_c.cur;
+  const z128* y = pick(A.y, cur);
+  if (blockIdx.x == 0 && A.rho_s)
+    for (int o = s_out[0]; o < s_out[1]; ++o)
+      for (int x = threadIdx.x; x < A.n_rs; x += kStepBS)
+        A.rho_s[static_cast<long long>(o) * A.n_rs + x] = y[x];
+  if (s_c.done || !(A.mode & STEP_INPUT)) return;
+  const void* D = pick(A.D, cur);
+  if (A.lo)
+    step_input(A, y, static_cast<const z64*>(D), static_cast<z64*>(A.sa), s_c.dt);
+  else
+    step_input(A, y, static_cast<const z128*>(D), static_cast<z128*>(A.sa), s_c.dt);
 }
 // rho_0 renormalisation (optional): Tr rho_0 of the initial state, then after
 // every step rho_0 <- (rho_0 + rho_0^+)/2 * tr0 / Tr, in FP64.  One workgroup of
@@ -102,14 +182,19 @@ __global__ void __launch_bounds__(1024) rho0_renorm_kernel(z128* y0, z128* y1, z
   }
   if (ctrl && threadIdx.x == 0) ctrl->projected = ctrl->accepted;
 }
-__global__ void ctrl_init_kernel(Ctrl* c, double t0, double t_bound, double dt) {
+__global__ void ctrl_init_kernel(Ctrl* c, double t0, double t_bound, double dt, int i_int) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (dt < 0.0) dt = c->dt;  // keep dt_save (adaptive_step_size_solver.h:39-41,55)
+  if (dt < 0.0)
+    dt = c->dt;  // keep dt_save (adaptive_step_size_solver.h:39-41,55)
+  else
+    *c = Ctrl{};  // the start of a solve
   c->t = t0;
   c->t_bound = t_bound;
   c->done = 0;
   c->count = 1;
   c->gave_up = 0;
+  c->seq = 0;
+  c->i_int = i_int;
   if (t0 + dt > t_bound) dt = t_bound - t0;
   c->dt = dt;
 }
@@ -156,13 +241,28 @@ int launch_operator(const FormDev& d, int real_bytes, const StageArgs& A, hipStr
   return g;
 }
 
-void launch_err_finalize(const StageArgs& A, int nparts, hipStream_t stream) {
-  hipLaunchKernelGGL(err_finalize_kernel, dim3(1), dim3(1024), 0, stream, A, nparts);
+// One launch, or, where every workgroup reading every partial would cost more
+// than a launch (4.6 us), the decision by one workgroup and then the stage input.
+void launch_dopri_step(const StepArgs& A, hipStream_t stream) {
+  const long long per = 2 * kStepBS;  // elements per workgroup until the grid is full
+  const int grid = static_cast<int>(std::max(1LL, std::min(512LL, (A.n + per - 1) / per)));
+  StepArgs a = A;
+  if ((a.mode & STEP_CONTROL) && ((a.mode & STEP_INPUT) == 0 || a.nparts > kStepFusedParts)) {
+    a.mode &= ~STEP_INPUT;
+    hipLaunchKernelGGL(dopri_step_kernel, dim3(1), dim3(kStepBS), 0, stream, a);
+    HAMD_HIP(hipGetLastError());
+    if (!(A.mode & STEP_INPUT)) return;
+    a.mode = STEP_INPUT;
+    a.prev = a.next;
+    a.rho_s = nullptr;
+  }
+  hipLaunchKernelGGL(dopri_step_kernel, dim3(grid), dim3(kStepBS), 0, stream, a);
   HAMD_HIP(hipGetLastError());
 }
 
-void launch_ctrl_init(Ctrl* c, double t0, double t_bound, double dt, hipStream_t stream) {
-  hipLaunchKernelGGL(ctrl_init_kernel, dim3(1), dim3(64), 0, stream, c, t0, t_bound, dt);
+void launch_ctrl_init(Ctrl* c, double t0, double t_bound, double dt, int i_int,
+                      hipStream_t stream) {
+  hipLaunchKernelGGL(ctrl_init_kernel, dim3(1), dim3(64), 0, stream, c, t0, t_bound, dt, i_int);
   HAMD_HIP(hipGetLastError());
 }
 void launch_rho0_trace(const void* y, int N, double* tr0, hipStream_t stream) {

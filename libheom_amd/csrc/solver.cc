@@ -1,15 +1,16 @@
 // RK4 (rk4.h:40-65) and Dormand-Prince 5(4) (rkdp.h:21-179) drivers.  Every
-// stage is one fused operator pass (kernels.hip); the Dormand-Prince step
-// control runs on the device, so the host only reads the control block back
-// once per batch of attempts instead of once per attempt.
+// stage is one fused operator pass (kernels.hip).  The Dormand-Prince step
+// control and the walk through the output times run on the device; the host
+// keeps one attempt queued behind the running one and reads a progress word in
+// host memory instead of synchronising.
 #include "solver.h"
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <limits>
-#include <map>
 #include <set>
+#include <thread>
 
 #include "kernels.h"
 
@@ -19,8 +20,11 @@ namespace {
 // slot numbers
 enum {
   SL_Y = 0, SL_YNEW = 1, SL_Y32 = 2, SL_YNEW32 = 3,
-  SL_SA = 4, SL_SB = 5, SL_ACC = 6, SL_K1 = 7,  // K1..K5 = 7..11
-  SL_E = 13  // Dormand-Prince: sum_{j<6} E_j k_j, always FP64
+  SL_SA = 4, SL_SB = 5, SL_ACC = 6, SL_K1 = 7,  // K2..K5 = 8..11
+  SL_E = 13,  // Dormand-Prince: sum_{j<6} E_j k_j, always FP64
+  // Dormand-Prince: D of y and of y_new (k_1 = -dt*D(y) for any dt: an attempt's last
+  // evaluation is the next attempt's first, and a rejected attempt keeps its own)
+  SL_D = 14, SL_DNEW = 15
 };
 }  // namespace
 
@@ -81,7 +85,9 @@ Solver::Solver(std::shared_ptr<Qme> q_, int kind_)
   if (kind == HEOM_RK4 || kind == HEOM_LSRK4) {
     mk(SL_ACC, z128b, 0);  // rk4: the accumulator; lsrk4: buff
   } else {
-    for (int k = 0; k < 5; ++k) mk(SL_K1 + k, sinb, lo);
+    for (int k = 1; k < 5; ++k) mk(SL_K1 + k, sinb, lo);
+    mk(SL_D, sinb, lo);
+    mk(SL_DNEW, sinb, lo);
     mk(SL_E, z128b, 0);
   }
   if (q->opt.renorm_rho0) {
@@ -90,16 +96,51 @@ Solver::Solver(std::shared_ptr<Qme> q_, int kind_)
     if (q->N > 64) throw HeomError{HEOM_ERR_UNSUPPORTED, "renorm_rho0: n_level > 64"};
     d_tr0.alloc(sizeof(double));
   }
-  d_ctrl.alloc(sizeof(Ctrl));
-  HAMD_HIP(hipMemset(d_ctrl.p, 0, sizeof(Ctrl)));
+  d_ctrl.alloc(2 * sizeof(Ctrl));
+  HAMD_HIP(hipMemset(d_ctrl.p, 0, 2 * sizeof(Ctrl)));
   d_partials.alloc(sizeof(double) * kMaxGrid);
-  HAMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_ctrl), sizeof(Ctrl), hipHostMallocDefault));
+  HAMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_ctrl), sizeof(Ctrl) + 128,
+                         hipHostMallocCoherent));
   std::memset(h_ctrl, 0, sizeof(Ctrl));
+  // the progress word on a cache line of its own
+  const uintptr_t after = reinterpret_cast<uintptr_t>(h_ctrl) + sizeof(Ctrl);
+  mail = reinterpret_cast<unsigned long long*>((after + 63) & ~uintptr_t(63));
   build_stages(0.0, 0.0);
 }
 
 Solver::~Solver() {
   if (h_ctrl) (void)hipHostFree(h_ctrl);
+  if (h_times) (void)hipHostFree(h_times);
+}
+
+// Output times to device memory by way of pinned memory: no allocation, and no
+// wait, while the list is no longer than an earlier one.  Both buffers are idle:
+// every solve waits for its stream before it returns.
+void Solver::upload_times(const double* t, int n) {
+  if (n > n_times) {
+    if (h_times) (void)hipHostFree(h_times);
+    h_times = nullptr;
+    n_times = 0;
+    HAMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_times), sizeof(double) * n,
+                           hipHostMallocDefault));
+    d_res_t.alloc(sizeof(double) * n);
+    n_times = n;
+  }
+  std::memcpy(h_times, t, sizeof(double) * n);
+  HAMD_HIP(hipMemcpyAsync(d_res_t.p, h_times, sizeof(double) * n, hipMemcpyHostToDevice,
+                          q->stream));
+}
+
+// Workspace of a solve call (its state or rho_S in device memory): kept up to
+// kKeepWork bytes, so that repeated solves allocate nothing; a larger one is the
+// call's own.
+void* Solver::workspace(DevBuf& kept, DevBuf& own, size_t bytes) {
+  if (bytes > kKeepWork) {
+    own.alloc(bytes);
+    return own.p;
+  }
+  if (kept.bytes < bytes) kept.alloc(bytes);
+  return kept.p;
 }
 
 void Solver::check_qme() const {
@@ -111,11 +152,11 @@ void Solver::check_qme() const {
                                     "created; create a new solver"};
 }
 
-// Physical buffer of a slot for ping-pong parity `cur` (slots 0..3 swap
-// within their pair when cur == 1).
+// Physical buffer of a slot for ping-pong parity `cur` (slots 0..3 and the D
+// pair swap within their pair when cur == 1).
 void* Solver::slot_ptr(int s, int cur) const {
   if (s < 0) return nullptr;
-  if (s < 4) return sp[(s & 2) + ((s & 1) ^ cur)];
+  if (s < 4 || s >= SL_D) return sp[s ^ cur];
   return sp[s];
 }
 
@@ -139,6 +180,8 @@ StageArgs Solver::resolve(const StageSpec& s) const {
   for (size_t j = 0; j < s.pre.size(); ++j)
     if (s.pre[j] >= 0 && slo[s.pre[j]]) a.pre_lo |= 1u << j;
   a.k_lo = s.k_slot >= 0 ? slo[s.k_slot] : 0;
+  a.k_raw = s.k_slot >= SL_D ? 1 : 0;
+  a.d_pre = s.pre.size() > 1 && s.pre[1] == SL_D ? 1 : 0;
   a.ncombo = s.ncombo;
   std::memcpy(a.cc, s.cc, sizeof(a.cc));
   std::memcpy(a.ck, s.ck, sizeof(a.ck));
@@ -151,11 +194,8 @@ StageArgs Solver::resolve(const StageSpec& s) const {
   a.ek = s.ek;
   a.ynew_pre = s.ynew_pre;
   a.yold_pre = s.yold_pre;
-  a.control = s.control;
-  a.inv_n = 1.0 / static_cast<double>(ms);
   if (kind == HEOM_RKDP) a.ctrl = ctrl_dev();
   a.partials = partials_dev();
-  a.max_partials = kMaxGrid;
   return a;
 }
 
@@ -212,36 +252,43 @@ void Solver::build_stages(double atol, double rtol) {
       specs.push_back(a);
     }
   } else {
-    // Dormand-Prince: stage i (0-based) evaluates k_i at its input and writes
-    // the input of stage i+1 (rkdp.h:111-127); stage 5 also forms the new
+    // Dormand-Prince: stage 0 evaluates D(y) and runs only where no attempt has left
+    // it (the start of a solve, after a projection of rho_0); the step pass forms
+    // the input of stage 1 from it.  Stage i (0-based, 1..5) evaluates k_{i+1} at its
+    // input and writes the input of stage i+1 (rkdp.h:111-127); stage 5 forms the new
     // state (rkdp.h:130-132) and, from the same operands, the error sum
     // e6 = sum_{j<6} E_j k_j in the order of rkdp.h:142-145 (k_6 itself is
-    // not stored); stage 6 evaluates k_7 at the new state, completes
-    // e = e6 + E_7 k_7 and the error norm (rkdp.h:144-153).  The error vector
-    // is the same fma chain as summing all seven terms in the last stage.
+    // not stored); stage 6 evaluates D at the new state, stores it as the next
+    // attempt's stage 0, completes e = e6 + E_7 k_7 and the error norm
+    // (rkdp.h:144-153).  The error vector is the same fma chain as summing all
+    // seven terms in the last stage.
     const int sin_[6] = {y_in, SL_SA, SL_SB, SL_SA, SL_SB, SL_SA};
     const int sout[5] = {SL_SA, SL_SB, SL_SA, SL_SB, SL_SA};
+    const auto k_of = [](int j) { return j == 0 ? int(SL_D) : SL_K1 + j; };
     for (int i = 0; i < 6; ++i) {
       StageSpec a;
       a.in_slot = sin_[i];
       std::vector<std::pair<int, double>> terms{{SL_Y, 1.0}};
-      if (i < 5) {
+      if (i == 0) {
+        a.k_slot = SL_D;
+      } else if (i < 5) {
         a.k_slot = SL_K1 + i;
-        for (int j = 0; j < i; ++j) terms.push_back({SL_K1 + j, kDpA[i + 1][j]});
+        for (int j = 0; j < i; ++j) terms.push_back({k_of(j), kDpA[i + 1][j]});
         a.combo(terms, kDpA[i + 1][i], sout[i]);
       } else {
         for (int j = 0; j < 5; ++j)
-          if (kDpB[j] != 0.0) terms.push_back({SL_K1 + j, kDpB[j]});
+          if (kDpB[j] != 0.0) terms.push_back({k_of(j), kDpB[j]});
         a.combo(terms, kDpB[5], SL_YNEW, lo ? SL_YNEW32 : -1);
         std::vector<std::pair<int, double>> eterms;
         for (int j = 0; j < 5; ++j)
-          if (kDpE[j] != 0.0) eterms.push_back({SL_K1 + j, kDpE[j]});
+          if (kDpE[j] != 0.0) eterms.push_back({k_of(j), kDpE[j]});
         a.combo(eterms, kDpE[5], SL_E);
       }
       specs.push_back(a);
     }
     StageSpec a;
     a.in_slot = lo ? SL_YNEW32 : SL_YNEW;
+    a.k_slot = SL_DNEW;
     a.do_err = 1;
     a.ec[a.pre_index(SL_E)] = 1.0;
     a.ek = kDpE[6];
@@ -250,7 +297,6 @@ void Solver::build_stages(double atol, double rtol) {
     a.pre.push_back(SL_Y);
     a.ynew_pre = 1;
     a.yold_pre = 2;
-    a.control = 1;
     specs.push_back(a);
   }
   for (auto& s : specs) {
@@ -265,7 +311,7 @@ void Solver::build_stages(double atol, double rtol) {
 // runs this fixed-step problem.
 void Solver::build_resident() {
   res = ResidentArgs{};
-  if (!use_graphs || kind == HEOM_RKDP || in_bytes != 8 || q->opt.renorm_rho0 ||
+  if (!use_resident || kind == HEOM_RKDP || in_bytes != 8 || q->opt.renorm_rho0 ||
       !resident_ok(q->dev, q->dev.max_links))
     return;
   const ResidentProg& P = kind == HEOM_RK4 ? kResidentRk4 : kResidentLsrk4;
@@ -306,71 +352,20 @@ void Solver::renorm(bool with_ctrl) {
   launch_rho0_renorm(slot_ptr(SL_Y, 0), slot_ptr(SL_Y, with_ctrl ? 1 : 0),
                      lo ? slot_ptr(SL_Y32, 0) : nullptr,
                      lo ? slot_ptr(SL_Y32, with_ctrl ? 1 : 0) : nullptr,
-                     with_ctrl ? ctrl_dev() : nullptr, q->N, d_tr0.as<double>(), q->stream);
+                     with_ctrl ? ctrl_dev() + par : nullptr, q->N, d_tr0.as<double>(), q->stream);
 }
 
 void Solver::launch_stage(int s, double dt) {
   StageArgs a = stages[s];
   a.a_re = dt;
-  int grid = q->operate(in_bytes, a, q->stream);
-  if (a.do_err) launch_err_finalize(a, grid, q->stream);
-}
-
-// Record the kernels `body` launches on the library stream into g (stream
-// capture; the stage launches enqueue kernels only, no memory operations).
-template <typename F>
-void Solver::capture(GraphExec& g, F&& body) {
-  g.reset();
-  hipStream_t st = q->stream;
-  HAMD_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  hipGraph_t graph = nullptr;
-  try {
-    body();
-  } catch (...) {
-    (void)hipStreamEndCapture(st, &graph);
-    if (graph) (void)hipGraphDestroy(graph);
-    throw;
-  }
-  HAMD_HIP(hipStreamEndCapture(st, &graph));
-  const hipError_t e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
-  (void)hipGraphDestroy(graph);
-  HAMD_HIP(e);
-}
-
-void Solver::reset_graphs() {
-  g_rk4.clear();
-  g_dopri.clear();
-  g_rk4_dt = 0.0;
-}
-
-// Graph of n repetitions of `one` (cached by n; the cache holds a few sizes).
-GraphExec& Solver::graph_for(std::map<long long, std::unique_ptr<GraphExec>>& cache, long long n,
-                             const std::function<void()>& one) {
-  auto it = cache.find(n);
-  if (it != cache.end()) return *it->second;
-  if (cache.size() >= kMaxGraphs) cache.erase(cache.begin());
-  auto g = std::make_unique<GraphExec>();
-  capture(*g, [&] {
-    for (long long k = 0; k < n; ++k) one();
-  });
-  return *cache.emplace(n, std::move(g)).first->second;
-}
-
-// `count` repetitions of `one` as graph launches of power-of-two sizes
-void Solver::replay(std::map<long long, std::unique_ptr<GraphExec>>& cache, long long count,
-                    const std::function<void()>& one) {
-  while (count > 0) {
-    long long n = kMaxGraphSteps;
-    while (n > count) n >>= 1;
-    HAMD_HIP(hipGraphLaunch(graph_for(cache, n, one).exec, q->stream));
-    count -= n;
-  }
+  if (a.ctrl) a.ctrl += par;
+  const int grid = q->operate(in_bytes, a, q->stream);
+  if (a.do_err) n_partials = grid;
 }
 
 // fixed_step_size_solver::solve_1 (fixed_step_size_solver.h:29-52): steps of
 // dt, the last one shortened to end exactly at t1.  The step sequence is
-// computed on the host with the reference's arithmetic; the steps of the full
-// dt are replayed from graphs of kGraphSteps steps and of one step.
+// computed on the host with the reference's arithmetic.
 void Solver::fixed_steps(double t0, double t1, double dt, long long& n_full, double& dt_last) {
   double t = t0, dt_1 = dt;
   n_full = 0;
@@ -401,19 +396,11 @@ void Solver::rk4_interval(double t0, double t1, double dt) {
     stats.n_accepted += n_full + 1;
     return;
   }
-  long long done = 0;
-  if (use_graphs && n_full > 0) {
-    if (g_rk4_dt != dt) {
-      g_rk4.clear();
-      g_rk4_dt = dt;
-    }
-    replay(g_rk4, n_full, [&] {
-      for (int s = 0; s < 4; ++s) launch_stage(s, dt);
-      if (q->opt.renorm_rho0) renorm(false);
-    });
-    done = n_full;
-  }
-  for (; done < n_full; ++done) {
+  // Launched one by one: the host enqueues a stage in less time than the device
+  // takes for the smallest, and graphs of the same launches have to be
+  // instantiated for every solve (7-site Dormand-Prince, five intervals: 4.60 ms
+  // with graphs, 4.30 without; 4-site chain, 160 RK4 stages: 1.27 and 1.20).
+  for (long long n = 0; n < n_full; ++n) {
     for (int s = 0; s < 4; ++s) launch_stage(s, dt);
     if (q->opt.renorm_rho0) renorm(false);
   }
@@ -424,40 +411,107 @@ void Solver::rk4_interval(double t0, double t1, double dt) {
   stats.n_accepted += n_full + 1;
 }
 
-// adaptive_step_size_solver::solve_1 (adaptive_step_size_solver.h:32-56) with
-// the attempts of rkdp::solve_adaptive_step launched in batches.
-int Solver::rkdp_interval(double t0, double t1, double dt_first, int& batch) {
-  launch_ctrl_init(ctrl_dev(), t0, t1, dt_first, q->stream);
-  long long a0 = h_ctrl->attempts;
-  // the projection kernel runs after every attempt and acts only when the
-  // control block counts a new accepted step
-  const auto attempt = [&] {
-    for (int s = 0; s < 7; ++s) launch_stage(s, 0.0);
-    if (q->opt.renorm_rho0) renorm(true);
-  };
-  while (true) {
-    if (use_graphs) {
-      replay(g_dopri, batch, attempt);
-    } else {
-      for (int b = 0; b < batch; ++b) attempt();
-    }
-    HAMD_HIP(hipMemcpyAsync(h_ctrl, ctrl_dev(), sizeof(Ctrl), hipMemcpyDeviceToHost, q->stream));
-    HAMD_HIP(hipStreamSynchronize(q->stream));
-    if (h_ctrl->done) break;
-    // attempts still needed at the current step (attempts after the interval
-    // is done are no-ops of a few microseconds each; a short batch costs one
-    // more host round trip)
-    const double rem = (h_ctrl->t_bound - h_ctrl->t) / h_ctrl->dt;
-    const long long est =
-        (rem > 0.0 && rem < static_cast<double>(kMaxAttemptBatch)) ? static_cast<long long>(
-                                                                         std::ceil(rem))
-                                                                   : 2LL * batch;
-    batch = static_cast<int>(std::min<long long>(kMaxAttemptBatch, std::max<long long>(1, est)));
+// The pass between two attempts, see StepArgs
+void Solver::launch_step(int mode) {
+  StepArgs a{};
+  a.mode = mode;
+  if (mode & STEP_CONTROL) par ^= 1;
+  a.next = ctrl_dev() + par;
+  a.prev = (mode & STEP_CONTROL) ? ctrl_dev() + (par ^ 1) : a.next;
+  a.partials = partials_dev();
+  a.nparts = n_partials;
+  a.inv_n = 1.0 / static_cast<double>(ms);
+  a.t_list = step_t;
+  a.n_int = step_n_int;
+  a.rho_s = (mode & STEP_CONTROL) ? step_rho_s : nullptr;
+  a.n_rs = q->N2;
+  for (int cur = 0; cur < 2; ++cur) {
+    a.y[cur] = static_cast<const z128*>(slot_ptr(SL_Y, cur));
+    a.D[cur] = slot_ptr(SL_D, cur);
   }
-  // the next interval starts with as many attempts as this one took
-  const long long used = h_ctrl->attempts - a0;
-  batch = static_cast<int>(std::max<long long>(1, std::min<long long>(used, 4096)));
+  a.lo = in_bytes == 4 ? 1 : 0;
+  a.sa = sp[SL_SA];
+  a.a21 = kDpA[1][0];
+  a.n = ms;
+  a.mail = mail;
+  launch_dopri_step(a, q->stream);
+}
+
+// The device's progress word once it has moved past `seen` step passes.
+unsigned long long Solver::wait_mail(unsigned long long seen) {
+  for (unsigned n = 1;; ++n) {
+    const unsigned long long v = __atomic_load_n(mail, __ATOMIC_ACQUIRE);
+    if ((v >> 2) > seen) return v;
+    if (n % (1u << 14) == 0) std::this_thread::yield();
+    if (n % (1u << 20) == 0) {
+      const hipError_t e = hipStreamQuery(q->stream);
+      if (e == hipErrorNotReady) continue;
+      HAMD_HIP(e);
+      // the stream has drained: the word is final
+      const unsigned long long w = __atomic_load_n(mail, __ATOMIC_ACQUIRE);
+      if ((w >> 2) > seen) return w;
+      throw HeomError{HEOM_ERR_HIP, "rkdp: the step pass left no progress word"};
+    }
+  }
+}
+
+// Attempts of rkdp::solve_adaptive_step until the control block is done: one
+// output interval (adaptive_step_size_solver::solve_1,
+// adaptive_step_size_solver.h:32-56), or all of step_t.  While an attempt runs,
+// the next one is queued behind it, so the device never waits for the host; when
+// the running attempt can be the last, only its step pass is, so that nothing is
+// left over (attempts queued in batches left 3-4 idle ones per solve of 30).
+int Solver::run_attempts() {
+  const bool proj = q->opt.renorm_rho0 != 0;
+  __atomic_store_n(mail, 0ull, __ATOMIC_RELEASE);
+  // a projection of rho_0 after every attempt acts only on an accepted one and
+  // makes the stored D stale
+  const auto step = [&](bool first) {
+    launch_step(STEP_CONTROL | (first ? STEP_FIRST : 0) | (proj ? 0 : STEP_INPUT));
+    if (proj) {
+      if (!first) renorm(true);
+      launch_stage(0, 0.0);
+      launch_step(STEP_INPUT);
+    }
+  };
+  const auto evaluate = [&] {
+    for (int s = 1; s < 7; ++s) launch_stage(s, 0.0);
+  };
+  step(true);
+  evaluate();
+  unsigned long long steps = 1, attempts = 1, seen = 0;
+  while (true) {
+    const unsigned long long v = wait_mail(seen);
+    seen = v >> 2;
+    if (v & 1) break;
+    if (attempts < seen) {  // the attempt held back as possibly not needed
+      evaluate();
+      ++attempts;
+    }
+    if (steps < seen + 1) {
+      step(false);
+      ++steps;
+    }
+    if (!(v & 2) && attempts < seen + 1) {
+      evaluate();
+      ++attempts;
+    }
+  }
+  HAMD_HIP(hipMemcpyAsync(h_ctrl, ctrl_dev() + par, sizeof(Ctrl), hipMemcpyDeviceToHost,
+                          q->stream));
+  HAMD_HIP(hipStreamSynchronize(q->stream));
   return h_ctrl->gave_up;
+}
+
+void Solver::add_dopri_stats() {
+  // the scheme's seven stages per attempt (the first one taken from the attempt
+  // before it)
+  stats.n_rhs += 7 * h_ctrl->attempts;
+  stats.n_attempts += h_ctrl->attempts;
+  stats.n_accepted += h_ctrl->accepted;
+  stats.n_rejected += h_ctrl->rejected;
+  stats.last_err = h_ctrl->err;
+  stats.last_dt = dt_save;
 }
 
 int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
@@ -476,8 +530,7 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
   }
   HAMD_HIP(hipSetDevice(q->opt.device));
   build_stages(atol, rtol);
-  build_resident();  // nothing without graphs
-  if (!noalloc) reset_graphs();  // stage arguments (tolerances, closure) may have changed
+  build_resident();
   const size_t bytes = sizeof(z128) * ms;
   hipStream_t st = q->stream;
   // the caller's state enters the FP64 state slot
@@ -497,16 +550,11 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
     // wavefront holds the same ADOs as a workgroup of the stage kernels: the
     // error norm is then the same sum, so the steps are decided alike (spin-boson
     // depth 6, ten intervals: 4.7 ms with the stage kernels, 0.8 ms here).
-    const bool resident = use_graphs && in_bytes == 8 && !q->opt.renorm_rho0 &&
+    const bool resident = use_resident && in_bytes == 8 && !q->opt.renorm_rho0 &&
                           q->dev.kind == HEOM_HILB && (q->N == 1 || q->N == 2 || q->N == 4) &&
                           resident_dopri_ok(q->dev, q->dev.max_links);
     std::memset(h_ctrl, 0, sizeof(Ctrl));
-    if (!resident) {
-      HAMD_HIP(hipMemcpyAsync(ctrl_dev(), h_ctrl, sizeof(Ctrl), hipMemcpyHostToDevice, st));
-      HAMD_HIP(hipStreamSynchronize(st));
-    }
-    double first = dt_save > 0.0 ? dt_save : dt;
-    int batch = 4;
+    const double first = dt_save > 0.0 ? dt_save : dt;
     int cur = 0;
     bool started = false;
     for (int i = 0; i < n_t - 1; ++i) {
@@ -514,22 +562,21 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
       // a zero-length interval takes no attempt and keeps the step size (the
       // reference would clamp the step to 0 and never finish the next interval)
       if (!(t_list[i + 1] > t_list[i])) continue;
-      if (resident)
+      if (resident) {
         gave_up |= rkdp_interval_resident(t_list[i], t_list[i + 1], started ? h_ctrl->dt : first,
                                           atol, rtol);
-      else
-        gave_up |= rkdp_interval(t_list[i], t_list[i + 1], started ? -1.0 : first, batch);
+      } else {
+        launch_ctrl_init(ctrl_dev() + par, t_list[i], t_list[i + 1], started ? -1.0 : first, i,
+                         st);
+        if (!started && !q->opt.renorm_rho0) launch_stage(0, 0.0);
+        gave_up |= run_attempts();
+      }
       started = true;
       cur = h_ctrl->cur;
     }
     on_output(n_t - 1, P[cur].p);
     if (started) dt_save = h_ctrl->dt;
-    stats.n_rhs += 7 * h_ctrl->attempts;
-    stats.n_attempts += h_ctrl->attempts;
-    stats.n_accepted += h_ctrl->accepted;
-    stats.n_rejected += h_ctrl->rejected;
-    stats.last_err = h_ctrl->err;
-    stats.last_dt = dt_save;
+    add_dopri_stats();
     HAMD_HIP(hipMemcpyAsync(rho_dev, P[cur].p, bytes, hipMemcpyDeviceToDevice, st));
   }
   HAMD_HIP(hipStreamSynchronize(st));
@@ -543,9 +590,8 @@ int Solver::solve_gather(void* rho_dev, const double* t_list, int n_t, double dt
   check_qme();
   const size_t rs_bytes = sizeof(z128) * q->N2;
   hipStream_t st = q->stream;
-  if (kind == HEOM_RKDP && n_t >= 2 && use_graphs && in_bytes == 8 && !q->opt.renorm_rho0 &&
-      resident_dopri_ok(q->dev, q->dev.max_links))
-    return solve_resident_dopri(rho_dev, t_list, n_t, dt, atol, rtol, rho_s_dev);
+  if (kind == HEOM_RKDP && n_t >= 2 && !q->opt.renorm_rho0 && q->kind != kBatch)
+    return solve_dopri(rho_dev, t_list, n_t, dt, atol, rtol, rho_s_dev);
   if (kind == HEOM_RKDP || n_t < 2 || q->kind == kBatch) {
     return solve(rho_dev, t_list, n_t, dt, atol, rtol, [&](int i, const void* cur) {
       HAMD_HIP(hipMemcpyAsync(static_cast<char*>(rho_s_dev) + rs_bytes * i, cur, rs_bytes,
@@ -560,7 +606,6 @@ int Solver::solve_gather(void* rho_dev, const double* t_list, int n_t, double dt
   build_stages(atol, rtol);
   build_resident();
   if (res.scheme == 0) {
-    reset_graphs();
     return solve(rho_dev, t_list, n_t, dt, atol, rtol, [&](int i, const void* cur) {
       HAMD_HIP(hipMemcpyAsync(static_cast<char*>(rho_s_dev) + rs_bytes * i, cur, rs_bytes,
                               hipMemcpyDeviceToDevice, st));
@@ -595,51 +640,71 @@ int Solver::solve_gather(void* rho_dev, const double* t_list, int n_t, double dt
   return HEOM_OK;
 }
 
-// adaptive_step_size_solver::solve (adaptive_step_size_solver.h:32-56) for a
-// small problem: every interval, attempt and output in one resident launch.
-int Solver::solve_resident_dopri(void* rho_dev, const double* t_list, int n_t, double dt,
-                                 double atol, double rtol, void* rho_s_dev) {
+// adaptive_step_size_solver::solve (adaptive_step_size_solver.h:32-56) with the
+// device walking through the output times: a small problem in one resident
+// launch, others as a queue of attempts without a stop between the intervals.
+int Solver::solve_dopri(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
+                        double rtol, void* rho_s_dev) {
   check_qme();
-  for (int i = 0; i + 1 < n_t; ++i)
+  int first = -1;  // first interval of positive length
+  for (int i = 0; i + 1 < n_t; ++i) {
     if (!(t_list[i + 1] >= t_list[i]))
       throw HeomError{HEOM_ERR_ARG, "solve: t_list must be non-decreasing"};
+    if (first < 0 && t_list[i + 1] > t_list[i]) first = i;
+  }
   if (!(dt > 0.0) && dt_save <= 0.0) throw HeomError{HEOM_ERR_ARG, "rkdp: dt must be > 0"};
   if (!(atol >= 0.0) || !(rtol >= 0.0) || (atol == 0.0 && rtol == 0.0))
     throw HeomError{HEOM_ERR_ARG, "rkdp: atol/rtol must be >= 0 and not both 0"};
   HAMD_HIP(hipSetDevice(q->opt.device));
-  build_stages(atol, rtol);  // kept current for time_stages / stage_bytes
-  reset_graphs();
+  build_stages(atol, rtol);
   hipStream_t st = q->stream;
-  std::vector<double> t(t_list, t_list + n_t);
-  d_res_t.upload(t);
-  ResidentDopriArgs a{};
-  a.y = static_cast<z128*>(P[SL_Y].p);
-  a.n_int = n_t - 1;
-  a.t_list = d_res_t.as<double>();
-  a.dt_first = dt_save > 0.0 ? dt_save : dt;
-  a.atol = atol;
-  a.rtol = rtol;
-  a.inv_n = 1.0 / static_cast<double>(ms);
-  a.rho_s = static_cast<z128*>(rho_s_dev);
-  a.ctrl = d_ctrl.as<Ctrl>();
+  const bool resident =
+      use_resident && in_bytes == 8 && resident_dopri_ok(q->dev, q->dev.max_links);
+  upload_times(t_list, n_t);
+  const double dt_first = dt_save > 0.0 ? dt_save : dt;
   const size_t bytes = sizeof(z128) * ms;
   HAMD_HIP(hipMemcpyAsync(P[SL_Y].p, rho_dev, bytes, hipMemcpyDeviceToDevice, st));
-  launch_resident_dopri(q->dev, q->dev.max_links, a, st);
-  HAMD_HIP(hipMemcpyAsync(rho_dev, P[SL_Y].p, bytes, hipMemcpyDeviceToDevice, st));
-  HAMD_HIP(hipMemcpyAsync(h_ctrl, d_ctrl.p, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
+  std::memset(h_ctrl, 0, sizeof(Ctrl));
+  if (resident) {
+    ResidentDopriArgs a{};
+    a.y = static_cast<z128*>(P[SL_Y].p);
+    a.n_int = n_t - 1;
+    a.t_list = d_res_t.as<double>();
+    a.dt_first = dt_first;
+    a.atol = atol;
+    a.rtol = rtol;
+    a.inv_n = 1.0 / static_cast<double>(ms);
+    a.rho_s = static_cast<z128*>(rho_s_dev);
+    a.ctrl = d_ctrl.as<Ctrl>();
+    launch_resident_dopri(q->dev, q->dev.max_links, a, st);
+    HAMD_HIP(hipMemcpyAsync(rho_dev, P[SL_Y].p, bytes, hipMemcpyDeviceToDevice, st));
+    HAMD_HIP(hipMemcpyAsync(h_ctrl, d_ctrl.p, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
+  } else if (first < 0) {  // outputs only
+    for (int i = 0; i < n_t; ++i)
+      HAMD_HIP(hipMemcpyAsync(static_cast<z128*>(rho_s_dev) + static_cast<size_t>(i) * q->N2,
+                              P[SL_Y].p, sizeof(z128) * q->N2, hipMemcpyDeviceToDevice, st));
+  } else {
+    if (in_bytes == 4) launch_narrow(P[SL_Y32].p, P[SL_Y].p, ms, st);
+    launch_ctrl_init(ctrl_dev() + par, t_list[first], t_list[first + 1], dt_first, first, st);
+    launch_stage(0, 0.0);
+    step_t = d_res_t.as<double>();
+    step_n_int = n_t - 1;
+    step_rho_s = static_cast<z128*>(rho_s_dev);
+    try {
+      run_attempts();
+    } catch (...) {
+      step_t = nullptr;
+      step_rho_s = nullptr;
+      throw;
+    }
+    step_t = nullptr;
+    step_rho_s = nullptr;
+    HAMD_HIP(hipMemcpyAsync(rho_dev, P[h_ctrl->cur].p, bytes, hipMemcpyDeviceToDevice, st));
+  }
   HAMD_HIP(hipStreamSynchronize(st));
   // only intervals of positive length touch the step size (as in solve)
-  for (int i = 0; i + 1 < n_t; ++i)
-    if (t_list[i + 1] > t_list[i]) {
-      dt_save = h_ctrl->dt;
-      break;
-    }
-  stats.n_rhs += 7 * h_ctrl->attempts;
-  stats.n_attempts += h_ctrl->attempts;
-  stats.n_accepted += h_ctrl->accepted;
-  stats.n_rejected += h_ctrl->rejected;
-  stats.last_err = h_ctrl->err;
-  stats.last_dt = dt_save;
+  if (first >= 0) dt_save = h_ctrl->dt;
+  add_dopri_stats();
   stats.ado_stage_updates = stats.n_rhs * q->hs.n_hrchy;
   stats.gave_up |= h_ctrl->gave_up;
   return h_ctrl->gave_up ? HEOM_ERR_STEP_REJECTED : HEOM_OK;
@@ -652,9 +717,8 @@ int Solver::solve_noalloc(void* rho_dev, const double* t_list, int n_t, double d
   const bool batch = q->kind == kBatch;
   const size_t rs_bytes = sizeof(z128) * (batch ? q->batch_rs_size : q->N2);
   hipStream_t st = q->stream;
-  const bool graphs = use_graphs;
-  use_graphs = false;
-  noalloc = true;
+  const bool resident = use_resident;
+  use_resident = false;
   ext_ctrl = ctrl;
   ext_partials = partials;
   int rc = HEOM_OK;
@@ -667,14 +731,12 @@ int Solver::solve_noalloc(void* rho_dev, const double* t_list, int n_t, double d
         HAMD_HIP(hipMemcpyAsync(dst, cur, rs_bytes, hipMemcpyDeviceToDevice, st));
     });
   } catch (...) {
-    use_graphs = graphs;
-    noalloc = false;
+    use_resident = resident;
     ext_ctrl = nullptr;
     ext_partials = nullptr;
     throw;
   }
-  use_graphs = graphs;
-  noalloc = false;
+  use_resident = resident;
   ext_ctrl = nullptr;
   ext_partials = nullptr;
   return rc;
@@ -694,6 +756,7 @@ void Solver::time_stages(int reps, std::vector<double>& out) {
     c.dt = dt_save > 0.0 ? dt_save : 1e-3;
     c.cur = h_ctrl ? h_ctrl->cur : 0;
     std::memcpy(h_ctrl, &c, sizeof(Ctrl));
+    par = 0;
     HAMD_HIP(hipMemcpyAsync(d_ctrl.p, h_ctrl, sizeof(Ctrl), hipMemcpyHostToDevice, st));
   }
   hipEvent_t e0, e1;
@@ -701,11 +764,17 @@ void Solver::time_stages(int reps, std::vector<double>& out) {
   HAMD_HIP(hipEventCreate(&e1));
   for (int s = 0; s < ns; ++s) {
     StageArgs a = stages[s];
-    a.control = 0;
     a.a_re = 1e-3;
-    launch_operator(q->dev, in_bytes, a, st);  // warm-up
+    // the first of the seven Dormand-Prince passes is the step pass
+    const auto pass = [&] {
+      if (kind == HEOM_RKDP && s == 0)
+        launch_step(STEP_INPUT);
+      else
+        launch_operator(q->dev, in_bytes, a, st);
+    };
+    pass();  // warm-up
     HAMD_HIP(hipEventRecord(e0, st));
-    for (int r = 0; r < reps; ++r) launch_operator(q->dev, in_bytes, a, st);
+    for (int r = 0; r < reps; ++r) pass();
     HAMD_HIP(hipEventRecord(e1, st));
     HAMD_HIP(hipEventSynchronize(e1));
     float msf = 0.f;
@@ -758,6 +827,9 @@ void Solver::stage_bytes(std::vector<double>& out) {
     for (int r : rd) per += size_of(r);
     for (int w : wr) per += size_of(w);
     out[s] = per * static_cast<double>(ms) + tables;
+    // the step pass: y and D read, the next stage input written
+    if (kind == HEOM_RKDP && s == 0)
+      out[s] = (16.0 + size_of(SL_D) + size_of(SL_SA)) * static_cast<double>(ms);
   }
 }
 

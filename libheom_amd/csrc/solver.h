@@ -2,7 +2,6 @@
 #pragma once
 
 #include <functional>
-#include <map>
 #include <memory>
 #include <vector>
 
@@ -25,22 +24,8 @@ struct StageSpec {
   double ec[kMaxPre] = {};
   double ek = 0.0;
   int ynew_pre = -1, yold_pre = -1;
-  int control = 0;
   int pre_index(int slot);
   void combo(const std::vector<std::pair<int, double>>& terms, double ckv, int d, int d2 = -1);
-};
-
-// An instantiated HIP graph owned by the solver.
-struct GraphExec {
-  hipGraphExec_t exec = nullptr;
-  GraphExec() = default;
-  GraphExec(const GraphExec&) = delete;
-  GraphExec& operator=(const GraphExec&) = delete;
-  ~GraphExec() { reset(); }
-  void reset() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    exec = nullptr;
-  }
 };
 
 class Solver {
@@ -55,27 +40,33 @@ class Solver {
   long long ms;    // main_size
   double dt_save = -1.0;
   heom_stats stats{};
-  // replay fixed stage sequences from HIP graphs (RK4 steps of the full dt,
-  // Dormand-Prince attempts); 0 launches every kernel individually
-  bool use_graphs = true;
+  // small problems in the resident integrators; false launches every stage kernel
+  bool use_resident = true;
 
   // Propagate the FP64 device state rho_dev over t_list.  on_output(i, cur_ptr)
   // is called at every t_i with a device pointer to the FP64 state.
   int solve(void* rho_dev, const double* t_list, int n_t, double dt, double atol, double rtol,
             const std::function<void(int, const void*)>& on_output);
   // The same with rho_S of every output time gathered into rho_s_dev (n_t N^2
-  // complex128 in device memory) instead of a callback; a small fixed-step
-  // problem then runs the whole solve in one resident launch.
+  // complex128 in device memory) instead of a callback; a small problem then
+  // runs the whole solve in one resident launch, and Dormand-Prince passes from
+  // interval to interval on the device.
   int solve_gather(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
                    double rtol, void* rho_s_dev);
 
   // solve_gather without any device allocation, for callers that cannot
-  // allocate: every stage kernel is launched directly (no graphs, no resident
-  // integrator), the control block and the error-norm partials are the
+  // allocate: every stage kernel is launched (no resident
+  // integrator), the control blocks (two) and the error-norm partials are the
   // caller's (ctrl, partials: kMaxGrid doubles), and rho_S of every output time
   // is copied to rho_s_dev.  No closure may be bound.
   int solve_noalloc(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
                     double rtol, Ctrl* ctrl, double* partials, void* rho_s_dev);
+
+  // device workspace of one solve call: the solver's d_state / d_rho_s while it is
+  // at most kKeepWork bytes, else the caller's `own`
+  static constexpr size_t kKeepWork = size_t(64) << 20;
+  DevBuf d_state, d_rho_s;
+  void* workspace(DevBuf& kept, DevBuf& own, size_t bytes);
 
   // Average duration (ms) of each stage kernel over `reps` replays.
   void time_stages(int reps, std::vector<double>& ms_out);
@@ -93,11 +84,23 @@ class Solver {
   void* sp[kSlots] = {};
   int slo[kSlots] = {};  // 1: complex64 buffer
   DevBuf d_ctrl, d_partials;
-  // control block and partials of the current solve (the solver's own, or a
-  // caller's in solve_noalloc); noalloc: no graph, upload or resident launch
+  // control blocks and partials of the current solve (the solver's own, or a
+  // caller's in solve_noalloc); the step passes read one block and write the
+  // other, par is the one written last
   Ctrl* ext_ctrl = nullptr;
   double* ext_partials = nullptr;
-  bool noalloc = false;
+  int par = 0;
+  int n_partials = 0;  // partials of the last error-norm pass
+  unsigned long long* mail = nullptr;  // progress word in pinned memory (see StepArgs)
+  // output times the device walks through and where rho_S goes (null: one
+  // interval at a time)
+  const double* step_t = nullptr;
+  int step_n_int = 0;
+  z128* step_rho_s = nullptr;
+  void launch_step(int mode);
+  unsigned long long wait_mail(unsigned long long seen);
+  int run_attempts();
+  void add_dopri_stats();
   Ctrl* ctrl_dev() const { return ext_ctrl ? ext_ctrl : d_ctrl.as<Ctrl>(); }
   double* partials_dev() const { return ext_partials ? ext_partials : d_partials.as<double>(); }
   DevBuf d_tr0;  // Tr rho_0 at the start of the solve (renorm_rho0)
@@ -110,33 +113,20 @@ class Solver {
   StageArgs resolve(const StageSpec& s) const;
   std::vector<StageSpec> specs;
   void launch_stage(int s, double dt);
-  // graphs of 2^j full RK4 steps / Dormand-Prince attempts (j <= 8), by 2^j;
-  // a count is replayed as its binary decomposition
-  static constexpr int kMaxGraphSteps = 256;
-  // most Dormand-Prince attempts enqueued before the host reads the control block
-  static constexpr int kMaxAttemptBatch = 1 << 14;
-  static constexpr size_t kMaxGraphs = 9;
-  std::map<long long, std::unique_ptr<GraphExec>> g_rk4, g_dopri;
-  double g_rk4_dt = 0.0;
-  GraphExec& graph_for(std::map<long long, std::unique_ptr<GraphExec>>& cache, long long n,
-                       const std::function<void()>& one);
-  void replay(std::map<long long, std::unique_ptr<GraphExec>>& cache, long long count,
-              const std::function<void()>& one);
-  template <typename F>
-  void capture(GraphExec& g, F&& body);
-  void reset_graphs();
   void rk4_interval(double t0, double t1, double dt);
   // resident integrator (small problems): scheme != 0 when the problem qualifies
   ResidentArgs res{};
   DevBuf d_res_nf, d_res_dl, d_res_t;
+  double* h_times = nullptr;
+  int n_times = 0;
+  void upload_times(const double* t, int n);
   int rkdp_interval_resident(double t0, double t1, double dt_first, double atol, double rtol);
-  int solve_resident_dopri(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
-                           double rtol, void* rho_s_dev);
+  int solve_dopri(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
+                  double rtol, void* rho_s_dev);
   // fixed_step_size_solver::solve_1's step sequence over [t0, t1]: n_full steps
   // of dt, then one step of dt_last
   static void fixed_steps(double t0, double t1, double dt, long long& n_full, double& dt_last);
   void build_resident();
-  int rkdp_interval(double t0, double t1, double dt_first, int& batch);
 };
 
 }  // namespace hamd

@@ -138,13 +138,18 @@ __device__ __forceinline__ z128 combine(const PreT<KP>& p, const double* c, int 
   return v;
 }
 
+// k = -alpha * D
+__device__ __forceinline__ z128 scaled_k(z128 alpha, z128 D) {
+  return z128{-(alpha.re * D.re - alpha.im * D.im), -(alpha.re * D.im + alpha.im * D.re)};
+}
+
 // Epilogue shared by all operator kernels.  D is the operator applied to the
 // stage input at flat element gi; returns w^2 of the error norm (or 0).
 template <bool F64, typename R, int KP>
-__device__ __forceinline__ double epilogue(const PreT<KP>& p, const StageArgs& A, int cur, At gi,
+__device__ __forceinline__ double epilogue(PreT<KP> p, const StageArgs& A, int cur, At gi,
                                            cx<R> Dr, z128 alpha) {
   const z128 D = conv<double>(Dr);
-  const z128 k{-(alpha.re * D.re - alpha.im * D.im), -(alpha.re * D.im + alpha.im * D.re)};
+  const z128 k = scaled_k(alpha, D);
   if (A.mode == MODE_DIFF) {
     z128 v = k;
     if (A.npre > 0) {
@@ -154,7 +159,12 @@ __device__ __forceinline__ double epilogue(const PreT<KP>& p, const StageArgs& A
     stz(pick(A.dst[0], cur), F64 ? false : A.dst_lo[0], gi, v);
     return 0.0;
   }
-  if (void* kp = pick(A.k, cur)) stz(kp, F64 ? false : A.k_lo, gi, k);
+  if (void* kp = pick(A.k, cur)) stz(kp, F64 ? false : A.k_lo, gi, A.k_raw ? D : k);
+  if (A.d_pre) {
+    // k_1 of the stored derivative, rounded as a stored k_1 would be
+    const z128 k1 = scaled_k(alpha, p.v[1]);
+    p.v[1] = (F64 || !(A.pre_lo & 2u)) ? k1 : conv<double>(conv<float>(k1));
+  }
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     if (c < A.ncombo) {
@@ -226,7 +236,7 @@ __device__ inline void dopri_control(Ctrl* c, double err) {
 }
 
 // Block reduction of the error-norm partial sums: one value per workgroup,
-// written without atomics; err_finalize_kernel combines them.
+// written without atomics; dopri_step_kernel combines them.
 __device__ inline void write_partial(const StageArgs& A, double v) {
   __shared__ double s_red[16];
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
