@@ -183,6 +183,18 @@ struct alignas(16) BlockMap {
   int g, l0, l1, pad;
 };
 
+// The kernel that shares an ADO's links between groups of lanes (hilb_split.hip)
+// takes units of G groups of lanes: G ADOs, or one whose links the groups share.
+struct SplitUnit {
+  int g;       // the group's ADO, -1: none
+  int shared;  // every group of the unit has the same ADO
+};
+__host__ __device__ constexpr int split_groups(int N) { return N <= 11 ? 4 : 2; }
+// its dynamic LDS: the diagonals of V and a zero row
+inline size_t split_vd_lds(int n_noise, int N, bool real, size_t real_bytes) {
+  return static_cast<size_t>(n_noise + 1) * N * (real ? 1 : 2) * real_bytes;
+}
+
 // One member of a batch of independent Hilbert-form hierarchies packed into
 // one set of device tables (Qme::set_param_batch).
 struct BatchInst {
@@ -237,6 +249,12 @@ struct FormDev {
   int max_links;         // most links of any single ADO
   const LinkFlat* flat;  // links with inlined coefficients (same order as links)
   const BlockMap* bmap;  // n_hrchy work units, one per workgroup (single hierarchies)
+  // work units of the kernel that shares an ADO's links between groups of lanes
+  // (n_sunits workgroups, split_groups(N) records each) and every group's links in
+  // slink_n slots (neighbour -1: none); null where another kernel is used
+  const SplitUnit* sunits;
+  const Link* slinks;
+  int n_sunits, slink_n;
   // diagonal V: per noise u (plus one zero row) and element e = i*N+j the pair
   // (v_i - v_j, v_i + v_j); real V stores the pair as (re, im) of one z128,
   // complex V as two z128

@@ -11,6 +11,9 @@ namespace hamd {
 
 template <typename R, bool F64>
 int launch_hilb(const FormDev& d, const StageArgs& A, hipStream_t st);
+// 4 <= N <= 16, diagonal V, few ADOs with many links (d.slinks)
+template <typename R, bool F64>
+int launch_hilb_split(const FormDev& d, const StageArgs& A, hipStream_t st);
 // 16 < N <= 64 on matrix cores: diagonal V (d.mfma 1, 2), dense V (d.mfma 3)
 template <typename R, bool F64>
 int launch_hilb_mfma(const FormDev& d, const StageArgs& A, hipStream_t st);

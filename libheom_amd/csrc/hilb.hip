@@ -403,6 +403,7 @@ __global__ void __launch_bounds__(kBigBS) hilb_big_kernel(const FormDev d, const
 
 template <int N, typename R, bool F64>
 int launch_hilb_n(const FormDev& d, const StageArgs& A, hipStream_t st) {
+  if (N >= 4 && d.slinks != nullptr) return launch_hilb_split<R, F64>(d, A, st);
   const bool real = d.real_v && d.real_h;
   if (N >= 6 && d.diag_v && d.bmap != nullptr && d.n_hrchy <= kMaxGrid &&
       fast_vd_lds(d, real, sizeof(R)) <= 32 * 1024) {

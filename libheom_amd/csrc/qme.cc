@@ -372,12 +372,72 @@ std::vector<BlockMap> Qme::build_block_map() const {
   return map;
 }
 
+// Work units of hilb_split_kernel, from the work-unit map: unit b keeps to XCD
+// b mod 8, whose ADOs stay the ones of the map.  An ADO with more links than a
+// quarter (a half, N > 11) of the most any has is shared by a unit's groups, the
+// others fill units together, in the map's order.
+// Used while the ADOs are at most 4096 wavefronts (2048 with two groups) and some
+// ADO has more links than the one-group kernels take in two rounds.  RK4 stages
+// with launch, one group -> shared: 253 ADOs of 7x7 9.8 -> 5.6 us, 1820 of 4x4
+// 8.2 -> 5.6, 1771 of 10x10 (3542 wavefronts) 10.9 -> 9.8, 325 of 12x12 11.3 -> 8.7;
+// past the line the chip is full, and the shared kernel's registers and
+// workgroups cost more than its shorter chain: 4060 of 9x9 13.7 -> 18.3,
+// 969 of 16x16 11.1 -> 12.3, 12 650 of 7x7 17.4 -> 24.4.
+void Qme::build_split_units(const std::vector<BlockMap>& bm) {
+  dev.sunits = nullptr;
+  dev.slinks = nullptr;
+  dev.n_sunits = dev.slink_n = 0;
+  int most = 0;
+  for (const BlockMap& b : bm) most = std::max(most, b.l1 - b.l0);
+  const long long waves = static_cast<long long>(hs.n_hrchy) * ((N2 + 63) / 64);
+  const int G = split_groups(N);
+  if (dev.kind != HEOM_HILB || !dev.diag_v || N < 4 || N > 16 || most <= 8 ||
+      waves > 1024 * G || split_vd_lds(dev.n_noise, N, false, sizeof(double)) > 32 * 1024)
+    return;
+  constexpr int P = 8;
+  const int per = (most + G - 1) / G;
+  struct Group {
+    int g, l0, l1, step, shared;  // links l0, l0 + step, ... below l1
+  };
+  std::vector<Group> x[P];
+  for (int p = 0; p < P; ++p) {
+    std::vector<Group> few;
+    for (size_t b = p; b < bm.size(); b += P) {
+      if (bm[b].l1 - bm[b].l0 > per)
+        for (int q = 0; q < G; ++q) x[p].push_back({bm[b].g, bm[b].l0 + q, bm[b].l1, G, 1});
+      else
+        few.push_back({bm[b].g, bm[b].l0, bm[b].l1, 1, 0});
+    }
+    while (few.size() % G) few.push_back({-1, 0, 0, 1, 0});
+    x[p].insert(x[p].end(), few.begin(), few.end());
+  }
+  size_t n = 0;  // groups per XCD
+  for (auto& v : x) n = std::max(n, v.size());
+  std::vector<SplitUnit> units(n * P, SplitUnit{-1, 0});
+  std::vector<Link> slots(n * P * per, Link{-1, 0});
+  for (int p = 0; p < P; ++p)
+    for (size_t y = 0; y < x[p].size(); ++y) {
+      const Group& gr = x[p][y];
+      const size_t at = (y / G * P + p) * G + y % G;
+      units[at] = SplitUnit{gr.g, gr.shared};
+      size_t t = at * per;
+      for (int l = gr.l0; l < gr.l1; l += gr.step) slots[t++] = links[l];
+    }
+  d_sunits.upload(units);
+  d_slinks.upload(slots);
+  dev.sunits = d_sunits.as<SplitUnit>();
+  dev.slinks = d_slinks.as<Link>();
+  dev.n_sunits = static_cast<int>(n * P / G);
+  dev.slink_n = per;
+}
+
 void Qme::upload() {
   const int nn = static_cast<int>(noise_work_.size());
   HAMD_HIP(hipSetDevice(opt.device));
   d_link_ptr.upload(link_ptr);
   d_links.upload(links);
-  d_bmap.upload(build_block_map());
+  const std::vector<BlockMap> bm = build_block_map();
+  d_bmap.upload(bm);
   std::vector<LinkFlat> flat(links.size());
   for (size_t l = 0; l < links.size(); ++l) {
     const Coef& cf = coef[links[l].cid];
@@ -473,6 +533,7 @@ void Qme::upload() {
   dev.real_v = real_v ? 1 : 0;
   dev.flat = d_flat.as<LinkFlat>();
   dev.bmap = d_bmap.as<BlockMap>();
+  build_split_units(bm);
   dev.cmac_tab = d_cmac.as<z128>();
   dev.max_links = 0;
   for (int l = 0; l < hs.n_hrchy; ++l)
