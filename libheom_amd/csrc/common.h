@@ -195,6 +195,15 @@ inline size_t split_vd_lds(int n_noise, int N, bool real, size_t real_bytes) {
   return static_cast<size_t>(n_noise + 1) * N * (real ? 1 : 2) * real_bytes;
 }
 
+// Tile of the matrix-core kernels (16 < N <= 64), to which a block is zero-padded.
+// Tiles of 48 rows: dense V, where the products are the time (33..48 levels, 969
+// ADOs, FP64 430-470 -> 255 us), and diagonal V in FP64 (33 levels 75 -> 71 us, 48
+// levels 98 -> 85); with FP32 operands the smaller tile saves nothing and nine
+// waves hold fewer loads (complex64, 40 levels 70 -> 77 us; split-bf16 59 -> 77).
+constexpr int mfma_tile(int N, bool dense, bool lo) {
+  return N <= 32 ? 32 : N <= 48 && (dense || !lo) ? 48 : 64;
+}
+
 // One member of a batch of independent Hilbert-form hierarchies packed into
 // one set of device tables (Qme::set_param_batch).
 struct BatchInst {
@@ -264,12 +273,13 @@ struct FormDev {
   const int* R_col;
   const z128* R_val;
   // matrix-core path (heom_hilb, 16 < N <= 64): H as separate real / imaginary
-  // planes in FP64 and FP32, leading dimension 32 or 64 (the MFMA tile,
+  // planes in FP64 and FP32, leading dimension tile (the MFMA tile,
   // zero-padded); mfma = 0 off, 1 on for diagonal V (operands in the state
   // precision), 2 split-bf16x3 products with FP32 accumulation (diagonal V),
   // 3 dense V (operands in the state precision)
   int real_h;
   int mfma;
+  int tile;
   const double* Hre;
   const double* Him;
   const float* Hre32;

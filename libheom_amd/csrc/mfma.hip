@@ -35,7 +35,7 @@ struct Mfma<double> {
   static __device__ __forceinline__ acc mac(double a, double b, acc c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
+  static __host__ __device__ constexpr int row(int lk, int r) { return lk + 4 * r; }
   static __device__ __forceinline__ const double* re(const FormDev& d) { return d.Hre; }
   static __device__ __forceinline__ const double* im(const FormDev& d) { return d.Him; }
 };
@@ -45,7 +45,7 @@ struct Mfma<float> {
   static __device__ __forceinline__ acc mac(float a, float b, acc c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
+  static __host__ __device__ constexpr int row(int lk, int r) { return 4 * lk + r; }
   static __device__ __forceinline__ const float* re(const FormDev& d) { return d.Hre32; }
   static __device__ __forceinline__ const float* im(const FormDev& d) { return d.Him32; }
 };
@@ -75,8 +75,6 @@ __device__ __forceinline__ mf_f4 mac3(const Split8& a, const Split8& b, mf_f4 c)
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.hi, c, 0, 0, 0);
 }
 
-constexpr int kMfmaBS = 256;
-
 // Coefficient of a neighbour element at (i, j) with the diagonals of every V_u
 // in LDS (sv: n_noise + 1 rows of n, the last row zero; real V as R, complex V
 // as cx<R>): (v_i - v_j)*iphi + (v_i + v_j)*psi + dir.
@@ -104,10 +102,12 @@ struct MfmaCfg {
   static constexpr int N2 = N * N;
   static constexpr int LD = N + 1;                // LDS row stride
   static constexpr int NB = N / 16;               // 16-row bands
-  static constexpr int TPW = NB * NB / 4;         // output tiles per wave
+  // threads per ADO: N = 64 eight waves with two output tiles each, N = 48 nine
+  // and N = 32 four with one
+  static constexpr int BS = N == 64 ? 512 : N == 48 ? 576 : 256;
   static constexpr int KS = N / 4;                // k steps of the 16x16x4 products
   static constexpr int KB = N / 32;               // k steps of the bf16 products
-  static_assert(N == 32 || N == 64, "MFMA path: tiles of 32 or 64 rows");
+  static_assert(N == 32 || N == 48 || N == 64, "MFMA path: tiles of 32, 48 or 64 rows");
 };
 
 // H*rho - rho*H for the wave's tiles, operands in the state precision R
@@ -411,15 +411,26 @@ __global__ void __launch_bounds__(BS, BS / 128)
 // (heom_hilb.h:108-209): per ADO
 //   D = i[H, rho] + Gamma_n rho + sum_u (V_u X_u + Y_u V_u) + sum_direct dir rho_l
 //   X_u = i Phi_u + Psi_u + delta_u [V_u, rho],  Y_u = Psi_u - i Phi_u - delta_u [V_u, rho]
-// (i[V,Phi] + {V,Psi} + delta [V,[V,rho]] = V X + Y V).  D stays in the MFMA
-// accumulators from i[H, rho] + Gamma rho on; per noise [V_u, rho] goes to a
-// second accumulator set, X_u and then Y_u are built in an LDS workspace
-// (delta C at the accumulator positions, then the links of noise u added by
-// coalesced element-parallel passes) and multiplied on the matrix cores.
+// (i[V,Phi] + {V,Psi} + delta [V,[V,rho]] = V X + Y V).  A lane works on the
+// elements of its accumulators throughout: D stays in the accumulators from
+// i[H, rho] + Gamma rho on; per noise [V_u, rho] goes to a second accumulator set,
+// the links of noise u add to X_u and Y_u in registers (one read of each neighbour
+// for both), and the two are written to the LDS workspace one after the other as
+// operands of the next products.  The epilogue needs no exchange either.
+// Bound: the matrix pipe (18 real-operand products of N^3 per ADO with four
+// noises), 53% busy at N = 64: one workgroup per CU, phases between barriers.
+// 969 ADOs, four noises, FP64 / complex64, us: with X and Y accumulated in LDS by
+// separate passes over the links 64 levels 491 / 300, 20 levels 98 / 73; now 437 / 267
+// and 74 / 64; with tiles of 48 rows besides, 40 levels 440 / 276 -> 259 / 222.
 // ---------------------------------------------------------------------------
+constexpr int kCprodAhead = 4;
+
 // acc += sgn * (A B) for the wave's tiles.  A and B are complex; an operand in
 // LDS has leading dimension LD, a global one (a V_u plane pair) N, and a global
-// operand is real when GREAL (its imaginary plane is not read).
+// operand is real when GREAL (its imaginary plane is not read).  Global operands
+// come from L2, 500 cycles and more away, and a SIMD has two or three waves to
+// hide that: KG k steps are loaded ahead of their products (two at a time cost
+// 3% of the stage at N = 64, eight at a time as much in registers).
 template <int N, typename R, bool A_LDS, bool B_LDS, bool GREAL, int TPW>
 __device__ __forceinline__ void mfma_cprod(const R* ar, const R* ai, const R* br, const R* bi,
                                            R sgn, int band, int t0, int lr, int lk,
@@ -429,23 +440,48 @@ __device__ __forceinline__ void mfma_cprod(const R* ar, const R* ai, const R* br
   using Cfg = MfmaCfg<N>;
   constexpr int LDA = A_LDS ? Cfg::LD : N, LDB = B_LDS ? Cfg::LD : N;
   constexpr bool AR = !A_LDS && GREAL, BR = !B_LDS && GREAL;
+  constexpr int KG = !GREAL ? 2 : Cfg::KS % kCprodAhead == 0 ? kCprodAhead : Cfg::KS * kCprodAhead / 16;
+  static_assert(Cfg::KS % KG == 0, "k groups");
   const int row = band * 16 + lr;
-#pragma unroll 2
-  for (int ks = 0; ks < Cfg::KS; ++ks) {
-    const int kk = 4 * ks + lk;
-    const R a_r = sgn * ar[row * LDA + kk];
-    const R a_i = AR ? R(0) : sgn * ai[row * LDA + kk];
+  R ga_r[KG], ga_i[KG], gb_r[KG][TPW], gb_i[KG][TPW];
+  auto load = [&](int k0) {
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const int col = ((t0 + t) % Cfg::NB) * 16 + lr;
-      const R b_r = br[kk * LDB + col];
-      cre[t] = M::mac(a_r, b_r, cre[t]);
-      if (!BR) {
-        const R b_i = bi[kk * LDB + col];
-        cim[t] = M::mac(a_r, b_i, cim[t]);
-        if (!AR) cre[t] = M::mac(-a_i, b_i, cre[t]);
+    for (int s = 0; s < KG; ++s) {
+      const int kk = 4 * (k0 + s) + lk;
+      if (!A_LDS) {
+        ga_r[s] = ar[row * LDA + kk];
+        if (!AR) ga_i[s] = ai[row * LDA + kk];
       }
-      if (!AR) cim[t] = M::mac(a_i, b_r, cim[t]);
+      if (!B_LDS) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+          const int col = ((t0 + t) % Cfg::NB) * 16 + lr;
+          gb_r[s][t] = br[kk * LDB + col];
+          if (!BR) gb_i[s][t] = bi[kk * LDB + col];
+        }
+      }
+    }
+  };
+#pragma unroll 1
+  for (int k0 = 0; k0 < Cfg::KS; k0 += KG) {
+    load(k0);
+#pragma unroll
+    for (int s = 0; s < KG; ++s) {
+      const int kk = 4 * (k0 + s) + lk;
+      const R a_r = sgn * (A_LDS ? ar[row * LDA + kk] : ga_r[s]);
+      const R a_i = AR ? R(0) : sgn * (A_LDS ? ai[row * LDA + kk] : ga_i[s]);
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        const int col = ((t0 + t) % Cfg::NB) * 16 + lr;
+        const R b_r = B_LDS ? br[kk * LDB + col] : gb_r[s][t];
+        cre[t] = M::mac(a_r, b_r, cre[t]);
+        if (!BR) {
+          const R b_i = B_LDS ? bi[kk * LDB + col] : gb_i[s][t];
+          cim[t] = M::mac(a_r, b_i, cim[t]);
+          if (!AR) cre[t] = M::mac(-a_i, b_i, cre[t]);
+        }
+        if (!AR) cim[t] = M::mac(a_i, b_r, cim[t]);
+      }
     }
   }
 }
@@ -463,10 +499,16 @@ struct MfmaV<float> {
   static __device__ __forceinline__ const float* im(const FormDev& d) { return d.Vim32; }
 };
 
-constexpr int kDenseCh = 4;  // elements per thread whose loads are in flight together
+// elements per thread of rho_n whose loads are in flight together
+constexpr int kDenseCh = 4;
+// waves per SIMD the registers have to allow: one workgroup per CU at N = 64 in FP64
+// (133 KB of LDS), two in FP32
+template <int N, typename R>
+constexpr int kDenseWps = N == 64 ? (sizeof(R) == 8 ? 2 : 4)
+                          : N == 48 ? (sizeof(R) == 8 ? 3 : 4) : (sizeof(R) == 8 ? 3 : 4);
 
 template <int N, typename R, bool REALV, bool REALH, bool F64, int KP, bool PADDED, int BS>
-__global__ void __launch_bounds__(BS, BS / 256)
+__global__ void __launch_bounds__(BS, (kDenseWps<N, R>))
     hilb_mfma_dense_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
   using M = Mfma<R>;
@@ -474,7 +516,7 @@ __global__ void __launch_bounds__(BS, BS / 256)
   using acc_t = typename M::acc;
   constexpr int N2 = Cfg::N2, LD = Cfg::LD, NB = Cfg::NB;
   constexpr int TPW = NB * NB / (BS / 64);  // output tiles per wave
-  constexpr int EPT = N2 / BS;  // elements per thread (tile)
+  constexpr int EPT = N2 / BS;  // elements per thread when rho_n is staged
   extern __shared__ __align__(16) unsigned char s_dyn[];
   R* s_re = reinterpret_cast<R*>(s_dyn);  // rho_n, at the end D
   R* s_im = s_re + N * LD;
@@ -499,6 +541,19 @@ __global__ void __launch_bounds__(BS, BS / 256)
   const int band = t0 / NB;
   const R* Vr0 = MfmaV<R>::re(d);
   const R* Vi0 = MfmaV<R>::im(d);
+  // the lane's elements: those of its accumulators, (i0 + r RS, j0 + 16 t), all tiles in
+  // one band (padding: element 0, not stored)
+  constexpr int RS = M::row(0, 1);
+  const int i0 = band * 16 + M::row(lk, 0), j0 = (t0 % NB) * 16 + lr, off0 = i0 * n + j0;
+  bool in_block[TPW][4];
+  int at[TPW][4];
+#pragma unroll
+  for (int t = 0; t < TPW; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      in_block[t][r] = !PADDED || (i0 + r * RS < n && j0 + 16 * t < n);
+      at[t][r] = in_block[t][r] ? off0 + r * RS * n + 16 * t : 0;
+    }
   double err_acc = 0.0;
   for (int w = blockIdx.x; w < d.n_hrchy; w += gridDim.x) {
     BlockMap bm{w, 0, 0, 0};
@@ -573,91 +628,86 @@ __global__ void __launch_bounds__(BS, BS / 256)
       const int lu0 = l;
       while (l < bm.l1 && flat[l].u == u) ++l;
       const int lu1 = l;
-#pragma unroll 1
-      for (int pass = 0; pass < 2; ++pass) {
-        // workspace = +-delta C at the accumulator positions
-        const R sg = pass == 0 ? R(1) : R(-1);
+      // X = delta C + sum (iphi + psi) rho_l and Y = sum (psi - iphi) rho_l - delta C at the
+      // accumulator positions: the neighbours are read once for both
+      C xs[TPW][4], ys[TPW][4];
+#pragma unroll
+      for (int t = 0; t < TPW; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          xs[t][r] = dl * C{ccr[t][r], cci[t][r]};
+          ys[t][r] = C{-xs[t][r].re, -xs[t][r].im};
+        }
+      for (int lq = lu0; lq < lu1; ++lq) {
+        const LinkFlat q = ld_flat(flat + lq);
+        const C ip = conv<R>(q.iphi), ps = conv<R>(q.psi);
+        const C cx = ip + ps, cy = ps - ip;
+        const C* nb = in + static_cast<long long>(q.nbr) * n2;
+        C xv[TPW][4];
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) xv[t][r] = nb[at[t][r]];
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            cmac(xs[t][r], cx, xv[t][r]);
+            cmac(ys[t][r], cy, xv[t][r]);
+          }
+      }
+      auto put = [&](const C (&v)[TPW][4]) {
 #pragma unroll
         for (int t = 0; t < TPW; ++t) {
           const int col = ((t0 + t) % NB) * 16 + lr;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int i = band * 16 + M::row(lk, r);
-            if (i < n && col < n) {
-              const C cv{sg * ccr[t][r], sg * cci[t][r]};
-              const C x = dl * cv;
-              w_re[i * LD + col] = x.re;
-              w_im[i * LD + col] = x.im;
+            if (in_block[t][r]) {
+              w_re[i * LD + col] = v[t][r].re;
+              w_im[i * LD + col] = v[t][r].im;
             }
           }
         }
         __syncthreads();
-        // + sum_l coefficient * rho_l, element-parallel: X: iphi + psi, Y: psi - iphi
-        for (int lq = lu0; lq < lu1; ++lq) {
-          const LinkFlat q = ld_flat(flat + lq);
-          const C ip = conv<R>(q.iphi), ps = conv<R>(q.psi);
-          const C cf = pass == 0 ? ip + ps : ps - ip;
-          const C* nb = in + static_cast<long long>(q.nbr) * n2;
-#pragma unroll 1
-          for (int c0 = 0; c0 < EPT; c0 += kDenseCh) {
-            C xv[kDenseCh];
-#pragma unroll
-            for (int c = 0; c < kDenseCh; ++c) {
-              const int x = threadIdx.x + (c0 + c) * BS;
-              xv[c] = nb[x < n2 ? x : 0];
-            }
-#pragma unroll
-            for (int c = 0; c < kDenseCh; ++c) {
-              const int x = threadIdx.x + (c0 + c) * BS;
-              if (x < n2) {
-                const int i = x / n, j = x - (x / n) * n;
-                C wv{w_re[i * LD + j], w_im[i * LD + j]};
-                cmac(wv, cf, xv[c]);
-                w_re[i * LD + j] = wv.re;
-                w_im[i * LD + j] = wv.im;
-              }
-            }
-          }
-        }
-        __syncthreads();
-        if (pass == 0)  // D += V X
-          mfma_cprod<N, R, false, true, REALV, TPW>(Vr, Vi, w_re, w_im, R(1), band, t0, lr, lk,
-                                                    cre, cim);
-        else  // D += Y V
-          mfma_cprod<N, R, true, false, REALV, TPW>(w_re, w_im, Vr, Vi, R(1), band, t0, lr, lk,
-                                                    cre, cim);
-        __syncthreads();
-      }
+      };
+      put(xs);  // D += V X
+      mfma_cprod<N, R, false, true, REALV, TPW>(Vr, Vi, w_re, w_im, R(1), band, t0, lr, lk, cre,
+                                                cim);
+      __syncthreads();
+      put(ys);  // D += Y V
+      mfma_cprod<N, R, true, false, REALV, TPW>(w_re, w_im, Vr, Vi, R(1), band, t0, lr, lk, cre,
+                                                cim);
+      __syncthreads();
     }
-    // D to LDS (every wave has finished reading rho and the workspace)
+    // direct links (off-diagonal gamma) and the Runge-Kutta epilogue
+    const int ld0 = l;
+    C D[TPW][4];
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const int col = ((t0 + t) % NB) * 16 + lr;
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) D[t][r] = C{cre[t][r], cim[t][r]};
+    for (int lq = ld0; lq < bm.l1; ++lq) {
+      const LinkFlat q = ld_flat(flat + lq);
+      const C dir = conv<R>(q.dir);
+      const C* nb = in + static_cast<long long>(q.nbr) * n2;
+#pragma unroll
+      for (int t = 0; t < TPW; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) cmac(D[t][r], dir, nb[at[t][r]]);
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = band * 16 + M::row(lk, r);
-        if (i < n && col < n) {
-          s_re[i * LD + col] = cre[t][r];
-          s_im[i * LD + col] = cim[t][r];
+        PreT<KP> pv;
+        prefetch<F64, KP>(pv, A, cur, base + at[t][r], true);
+        if (in_block[t][r]) {
+          add_closure(d, base + at[t][r], D[t][r]);
+          err_acc += epilogue<F64, R, KP>(pv, A, cur, base + at[t][r], D[t][r], pg.alpha);
         }
       }
-    }
-    __syncthreads();
-    // direct (off-diagonal gamma) links and the Runge-Kutta epilogue, coalesced
-    const int ld0 = l, ld1 = bm.l1;
-    for (int x0 = threadIdx.x; x0 < n2; x0 += BS) {
-      const int i = x0 / n, j = x0 - (x0 / n) * n;
-      C Dc{s_re[i * LD + j], s_im[i * LD + j]};
-      PreT<KP> pv;
-      prefetch<F64, KP>(pv, A, cur, base + x0, true);
-      for (int lq = ld0; lq < ld1; ++lq) {
-        const LinkFlat q = ld_flat(flat + lq);
-        cmac(Dc, conv<R>(q.dir), in[static_cast<long long>(q.nbr) * n2 + x0]);
-      }
-      add_closure(d, base + x0, Dc);
-      err_acc += epilogue<F64, R, KP>(pv, A, cur, base + x0, Dc, pg.alpha);
-    }
-    __syncthreads();
+    __syncthreads();  // every wave has finished reading rho
   }
   if (A.do_err) write_partial(A, err_acc);
 }
@@ -676,7 +726,7 @@ int launch_hilb_mfma_n(const FormDev& d, const StageArgs& A, hipStream_t st) {
   // measured at 969 ADOs per Dormand-Prince stage: FP64 135 against 158 us,
   // split-bf16 99 against 138 us, complex64 with the links outer 112 against
   // 126 us)
-  constexpr int BS = N == 64 ? 512 : kMfmaBS;
+  constexpr int BS = MfmaCfg<N>::BS;
 #define HAMD_MFMA(REALH, KP, PAD)                                                \
   {                                                                              \
     auto k = hilb_mfma_kernel<N, R, REALH, F64, KP, BF16X3, PAD, BS>;            \
@@ -708,7 +758,7 @@ int launch_hilb_mfma_dense_n(const FormDev& d, const StageArgs& A, hipStream_t s
   const bool small = A.npre <= 4;
   // N = 64: eight waves per ADO (measured at 969 ADOs: 497 against 715 us per
   // FP64 stage, 309 against 364 us complex64)
-  constexpr int BS = N == 64 ? 512 : kMfmaBS;
+  constexpr int BS = MfmaCfg<N>::BS;
 #define HAMD_MD(REALV, REALH, KP, PAD)                                                 \
   {                                                                                    \
     auto k = hilb_mfma_dense_kernel<N, R, REALV, REALH, F64, KP, PAD, BS>;             \
@@ -741,20 +791,23 @@ template <typename R, bool F64>
 int launch_hilb_mfma(const FormDev& d, const StageArgs& A, hipStream_t st) {
   if (d.mfma == 2) {
     if constexpr (std::is_same<R, float>::value) {
-      return d.N <= 32 ? launch_hilb_mfma_n<32, float, false, true>(d, A, st)
-                       : launch_hilb_mfma_n<64, float, false, true>(d, A, st);
+      return d.tile == 32 ? launch_hilb_mfma_n<32, float, false, true>(d, A, st)
+                          : launch_hilb_mfma_n<64, float, false, true>(d, A, st);
     } else {
       throw HeomError{HEOM_ERR_UNSUPPORTED, "bf16x3 products need the FP32 state"};
     }
   }
-  return d.N <= 32 ? launch_hilb_mfma_n<32, R, F64, false>(d, A, st)
-                   : launch_hilb_mfma_n<64, R, F64, false>(d, A, st);
+  if constexpr (std::is_same<R, double>::value)
+    if (d.tile == 48) return launch_hilb_mfma_n<48, R, F64, false>(d, A, st);
+  return d.tile == 32 ? launch_hilb_mfma_n<32, R, F64, false>(d, A, st)
+                      : launch_hilb_mfma_n<64, R, F64, false>(d, A, st);
 }
 
 template <typename R, bool F64>
 int launch_hilb_mfma_dense(const FormDev& d, const StageArgs& A, hipStream_t st) {
-  return d.N <= 32 ? launch_hilb_mfma_dense_n<32, R, F64>(d, A, st)
-                   : launch_hilb_mfma_dense_n<64, R, F64>(d, A, st);
+  return d.tile == 32   ? launch_hilb_mfma_dense_n<32, R, F64>(d, A, st)
+         : d.tile == 48 ? launch_hilb_mfma_dense_n<48, R, F64>(d, A, st)
+                        : launch_hilb_mfma_dense_n<64, R, F64>(d, A, st);
 }
 
 HAMD_FORM_INSTANCES(launch_hilb_mfma)

@@ -538,12 +538,13 @@ void Qme::upload() {
   dev.max_links = 0;
   for (int l = 0; l < hs.n_hrchy; ++l)
     dev.max_links = std::max(dev.max_links, link_ptr[l + 1] - link_ptr[l]);
-  // matrix-core commutator: heom_hilb, 16 < N <= 64, diagonal V (tiles of 32 or
-  // 64 rows; H is zero-padded to the tile in its planes)
+  // matrix-core commutator: heom_hilb, 16 < N <= 64, diagonal V (tiles of 32, 48
+  // or 64 rows; H is zero-padded to the tile in its planes)
   const bool big = hilb && N > 16 && N <= 64;
   const bool mfma_ok = big && diag_v;
   const bool mfma_dense = big && !diag_v;
   dev.mfma = 0;
+  dev.tile = mfma_tile(N, mfma_dense, lo());
   if (opt.matrix_cores && mfma_ok) dev.mfma = dtype == HEOM_C64_BF16X3 ? 2 : 1;
   if (opt.matrix_cores && mfma_dense && dtype != HEOM_C64_BF16X3) dev.mfma = 3;
   if (kind != HEOM_HILB) {
@@ -562,7 +563,7 @@ void Qme::upload() {
   {
     // real / imaginary planes of H with leading dimension P (the MFMA tile,
     // zero-padded), P = N outside the matrix-core path
-    const int P = (mfma_ok || mfma_dense) ? (N <= 32 ? 32 : 64) : N;
+    const int P = (mfma_ok || mfma_dense) ? dev.tile : N;
     std::vector<double> hr(static_cast<size_t>(P) * P, 0.0), hi(hr.size(), 0.0);
     std::vector<float> hr32(hr.size(), 0.f), hi32(hr.size(), 0.f);
     for (int i = 0; i < N; ++i)
@@ -583,7 +584,7 @@ void Qme::upload() {
   dev.real_vd = 1;
   if (dev.mfma == 3) {
     // every V_u zero-padded to the tile, as real / imaginary planes
-    const int P = N <= 32 ? 32 : 64;
+    const int P = dev.tile;
     const size_t pl = static_cast<size_t>(P) * P;
     std::vector<double> vr(pl * nn, 0.0), vi(vr.size(), 0.0);
     std::vector<float> vr32(vr.size(), 0.f), vi32(vr.size(), 0.f);
