@@ -606,20 +606,34 @@ int heom_solve(heom_solver_handle s, double* rho_host, const double* t_list, int
     void* d = sv.workspace(sv.d_state, own, bytes);
     HAMD_HIP(hipMemcpy(d, rho_host, bytes, hipMemcpyHostToDevice));
     std::vector<double> rs(2 * N2);
+    const size_t rs_bytes = sizeof(hamd::z128) * N2;
+    // the first output is the caller's state; later ones may already be in host memory
     auto out = [&](int i, const void* cur) {
-      if (full_copy) {
-        HAMD_HIP(hipMemcpyAsync(rho_host, cur, bytes, hipMemcpyDeviceToHost, sv.q->stream));
-        HAMD_HIP(hipStreamSynchronize(sv.q->stream));
-        if (cb) cb(t_list[i], rho_host, rho_host, user);
+      void* dst = full_copy ? static_cast<void*>(rho_host) : rs.data();
+      const size_t n = full_copy ? bytes : rs_bytes;
+      if (i == 0) {
+        if (!full_copy) std::memcpy(dst, rho_host, n);
+      } else if (sv.host_state) {
+        std::memcpy(dst, sv.host_state, n);
       } else {
-        HAMD_HIP(hipMemcpyAsync(rs.data(), cur, sizeof(hamd::z128) * N2, hipMemcpyDeviceToHost,
-                                sv.q->stream));
+        HAMD_HIP(hipMemcpyAsync(dst, cur, n, hipMemcpyDeviceToHost, sv.q->stream));
         HAMD_HIP(hipStreamSynchronize(sv.q->stream));
-        if (cb) cb(t_list[i], rs.data(), nullptr, user);
       }
+      if (cb) cb(t_list[i], full_copy ? rho_host : rs.data(), full_copy ? rho_host : nullptr, user);
     };
-    int rc = sv.solve(d, t_list, n_t, dt, atol, rtol, out);
-    HAMD_HIP(hipMemcpy(rho_host, d, bytes, hipMemcpyDeviceToHost));
+    sv.to_host = true;
+    int rc;
+    try {
+      rc = sv.solve(d, t_list, n_t, dt, atol, rtol, out);
+    } catch (...) {
+      sv.to_host = false;
+      throw;
+    }
+    sv.to_host = false;
+    if (sv.host_state)
+      std::memcpy(rho_host, sv.host_state, bytes);
+    else
+      HAMD_HIP(hipMemcpy(rho_host, d, bytes, hipMemcpyDeviceToHost));
     if (rc != HEOM_OK)
       hamd::set_error(rc, "rkdp: step rejected 1000 times; interval skipped as in the reference");
     return rc;

@@ -368,6 +368,15 @@ constexpr ResidentProg kResidentLsrk4{
      {0, 2, {0, 2, 0, 0}, 2, {{1.0, 2.0 / 3.0 * -1.0, 0, 0}, {0.0, -1.0, 0, 0}}, {2.0 / 3.0, 1.0}, {1, 2}},
      {1, 2, {1, 2, 0, 0}, 2, {{1.0, 1.0 / 4.0 * -1.0, 0, 0}, {0.0, -1.0, 0, 0}}, {1.0 / 4.0, 1.0}, {0, 2}}}};
 
+// Host copy of a resident launch's results in pinned memory (all null: none): the
+// state, the control block (Dormand-Prince), then the progress word (1 << 2),
+// so that the host needs neither copies nor a synchronisation.
+struct ResidentHost {
+  z128* y;
+  Ctrl* ctrl;
+  unsigned long long* mail;
+};
+
 struct ResidentArgs {
   z128* y;          // the FP64 state in HBM (read at the start, written at the end)
   long long n_full; // steps of dt, then one step of dt_last
@@ -380,6 +389,7 @@ struct ResidentArgs {
   const double* dt_last_i;
   z128* rho_s;
   int scheme;  // 0: none (the problem does not qualify); 1: kResidentRk4; 2: kResidentLsrk4
+  ResidentHost host;
 };
 
 // Resident Dormand-Prince: the whole solve of a small problem in one launch
@@ -397,6 +407,7 @@ struct ResidentDopriArgs {
   double atol, rtol, inv_n;
   z128* rho_s;           // rho_S at the n_int + 1 output times (may be null)
   Ctrl* ctrl;            // the final control block (counters, dt_save, any give-up)
+  ResidentHost host;
 };
 
 // ---------------------------------------------------------------------------

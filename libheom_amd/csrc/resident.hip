@@ -174,6 +174,17 @@ constexpr int res_buf(const ResidentProg& P, int slot) {
   return -1;
 }
 
+// The results to the host: every lane's element is in host memory before the
+// progress word is.
+__device__ __forceinline__ void post_host(const ResidentHost& h, bool ok, int e, z128 y) {
+  if (h.mail == nullptr) return;
+  if (ok) h.y[e] = y;
+  __threadfence_system();
+  __syncthreads();
+  if (e == 0)
+    __hip_atomic_store(h.mail, 1ull << 2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // What bounds it: one workgroup, a barrier per stage, and between two barriers
 // the LDS reads (own row and column, up to MAXL neighbours), the chain of FP64
 // sums and one LDS write.  With the level count compiled in and every operand
@@ -239,6 +250,7 @@ __global__ void __launch_bounds__(BS) resident_kernel(const FormDev d, const Res
   }
   if (a.n_int > 0 && e < N2) a.rho_s[static_cast<size_t>(a.n_int) * N2 + e] = r[0];
   if (ok) a.y[e] = r[0];
+  post_host(a.host, ok, e, r[0]);
 }
 
 // Resident Dormand-Prince: the adaptive solve of a small heom_hilb problem
@@ -288,6 +300,10 @@ __global__ void __launch_bounds__(BS)
   z128* SA = buf + 2 * static_cast<size_t>(ms);
   z128* SB = buf + 3 * static_cast<size_t>(ms);
   z128* KL = buf + 4 * static_cast<size_t>(ms);  // k1..k6 beyond 512 elements
+  // D of the current state: the first evaluation of an attempt is the last one of
+  // the attempt that produced the state (a rejected one keeps its own)
+  z128 dy{0.0, 0.0};
+  if (ok) dy = el.template op<REG>(buf, s_H, y, N, N2);
   for (int iv = 0; iv < a.n_int; ++iv) {
     // ctrl_init_kernel: dt carries over from the last attempt
     const double t0 = a.t_list ? a.t_list[iv] : a.t0, t1 = a.t_list ? a.t_list[iv + 1] : a.t1;
@@ -318,7 +334,8 @@ __global__ void __launch_bounds__(BS)
         const z128* in = st == 0 ? Y : ((st & 1) ? SA : SB);
         z128* out = st == 5 ? YN : ((st & 1) ? SB : SA);
         if (ok) {
-          const z128 D = el.template op<REG>(in, s_H, REG ? x : in[e], N, N2);
+          const z128 D =
+              st == 0 ? dy : el.template op<REG>(in, s_H, REG ? x : in[e], N, N2);
           const z128 k{-(dt * D.re - 0.0 * D.im), -(dt * D.im + 0.0 * D.re)};
           K(st) = k;
           const z128 y0 = REG ? y : Y[e];
@@ -341,9 +358,10 @@ __global__ void __launch_bounds__(BS)
         __syncthreads();
       }
       double w2 = 0.0;
+      z128 D{0.0, 0.0};
       if (ok) {
         const z128 yn = REG ? x : YN[e], yo = REG ? y : Y[e];
-        const z128 D = el.template op<REG>(YN, s_H, yn, N, N2);
+        D = el.template op<REG>(YN, s_H, yn, N, N2);
         const z128 k{-(dt * D.re - 0.0 * D.im), -(dt * D.im + 0.0 * D.re)};
         z128 er{0.0, 0.0};
 #pragma unroll
@@ -393,7 +411,10 @@ __global__ void __launch_bounds__(BS)
       }
       if (!REG) __syncthreads();
       if (c.gave_up) gave_up = 1;
-      if (REG && c.cur != cur) y = x;
+      if (c.cur != cur) {
+        dy = D;
+        if (REG) y = x;
+      }
     }
     if (!REG && ok) y = buf[(c.cur ? ms : 0) + e];
     if (a.rho_s && e < N2) a.rho_s[static_cast<size_t>(iv + 1) * N2 + e] = y;
@@ -405,7 +426,9 @@ __global__ void __launch_bounds__(BS)
     Ctrl out = c;
     out.gave_up = gave_up;
     *a.ctrl = out;
+    if (a.host.mail) *a.host.ctrl = out;
   }
+  post_host(a.host, ok, e, y);
 }
 
 }  // namespace

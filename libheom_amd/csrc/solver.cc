@@ -111,6 +111,7 @@ Solver::Solver(std::shared_ptr<Qme> q_, int kind_)
 Solver::~Solver() {
   if (h_ctrl) (void)hipHostFree(h_ctrl);
   if (h_times) (void)hipHostFree(h_times);
+  if (h_state) (void)hipHostFree(h_state);
 }
 
 // Output times to device memory by way of pinned memory: no allocation, and no
@@ -129,6 +130,12 @@ void Solver::upload_times(const double* t, int n) {
   std::memcpy(h_times, t, sizeof(double) * n);
   HAMD_HIP(hipMemcpyAsync(d_res_t.p, h_times, sizeof(double) * n, hipMemcpyHostToDevice,
                           q->stream));
+}
+
+// A small list to a device buffer that is kept while the lists fit (idle, as above)
+void Solver::upload_kept(DevBuf& b, const void* src, size_t bytes) {
+  if (b.bytes < bytes) b.alloc(bytes);
+  HAMD_HIP(hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, q->stream));
 }
 
 // Workspace of a solve call (its state or rho_S in device memory): kept up to
@@ -319,6 +326,15 @@ void Solver::build_resident() {
   res.scheme = kind == HEOM_RK4 ? 1 : 2;
 }
 
+// Where a resident launch leaves its results in host memory (see ResidentHost)
+ResidentHost Solver::resident_host() {
+  if (h_state == nullptr)
+    HAMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_state), sizeof(z128) * kResidentMax,
+                           hipHostMallocCoherent));
+  __atomic_store_n(mail, 0ull, __ATOMIC_RELEASE);
+  return ResidentHost{h_state, h_ctrl, mail};
+}
+
 // One Dormand-Prince interval of a small problem in one resident launch, as
 // rkdp_interval: the state stays in slot SL_Y, the control block's counters add
 // up over the intervals.
@@ -335,10 +351,11 @@ int Solver::rkdp_interval_resident(double t0, double t1, double dt_first, double
   a.rtol = rtol;
   a.inv_n = 1.0 / static_cast<double>(ms);
   a.ctrl = d_ctrl.as<Ctrl>();
-  launch_resident_dopri(q->dev, q->dev.max_links, a, q->stream);
   const Ctrl before = *h_ctrl;
-  HAMD_HIP(hipMemcpyAsync(h_ctrl, d_ctrl.p, sizeof(Ctrl), hipMemcpyDeviceToHost, q->stream));
-  HAMD_HIP(hipStreamSynchronize(q->stream));
+  a.host = resident_host();
+  launch_resident_dopri(q->dev, q->dev.max_links, a, q->stream);
+  (void)wait_mail(0);
+  host_state = h_state;
   h_ctrl->cur = 0;
   h_ctrl->attempts += before.attempts;
   h_ctrl->accepted += before.accepted;
@@ -390,7 +407,12 @@ void Solver::rk4_interval(double t0, double t1, double dt) {
     a.n_full = n_full;
     a.dt = dt;
     a.dt_last = dt_1;
+    if (to_host) a.host = resident_host();
     launch_resident(q->dev, q->dev.max_links, a, q->stream);
+    if (to_host) {
+      (void)wait_mail(0);
+      host_state = h_state;
+    }
     stats.n_rhs += 4 * (n_full + 1);
     stats.n_attempts += n_full + 1;
     stats.n_accepted += n_full + 1;
@@ -531,6 +553,7 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
   HAMD_HIP(hipSetDevice(q->opt.device));
   build_stages(atol, rtol);
   build_resident();
+  host_state = nullptr;
   const size_t bytes = sizeof(z128) * ms;
   hipStream_t st = q->stream;
   // the caller's state enters the FP64 state slot
@@ -549,7 +572,7 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
     // Small problems: an interval per resident launch.  The levels for which a
     // wavefront holds the same ADOs as a workgroup of the stage kernels: the
     // error norm is then the same sum, so the steps are decided alike (spin-boson
-    // depth 6, ten intervals: 4.7 ms with the stage kernels, 0.8 ms here).
+    // depth 6, ten intervals: 4.6 ms with the stage kernels, 0.52 ms here).
     const bool resident = use_resident && in_bytes == 8 && !q->opt.renorm_rho0 &&
                           q->dev.kind == HEOM_HILB && (q->N == 1 || q->N == 2 || q->N == 4) &&
                           resident_dopri_ok(q->dev, q->dev.max_links);
@@ -619,8 +642,8 @@ int Solver::solve_gather(void* rho_dev, const double* t_list, int n_t, double dt
     fixed_steps(t_list[i], t_list[i + 1], dt, nf[i], dl[i]);
     steps += nf[i] + 1;
   }
-  d_res_nf.upload(nf);
-  d_res_dl.upload(dl);
+  upload_kept(d_res_nf, nf.data(), sizeof(long long) * nf.size());
+  upload_kept(d_res_dl, dl.data(), sizeof(double) * dl.size());
   ResidentArgs a = res;
   a.y = static_cast<z128*>(P[SL_Y].p);
   a.dt = dt;

@@ -62,6 +62,11 @@ class Solver {
   int solve_noalloc(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
                     double rtol, Ctrl* ctrl, double* partials, void* rho_s_dev);
 
+  // heom_solve: the resident launches leave the state in host memory as well.
+  // host_state: the current state there, null when the output has to copy it
+  bool to_host = false;
+  const z128* host_state = nullptr;
+
   // device workspace of one solve call: the solver's d_state / d_rho_s while it is
   // at most kKeepWork bytes, else the caller's `own`
   static constexpr size_t kKeepWork = size_t(64) << 20;
@@ -120,6 +125,9 @@ class Solver {
   double* h_times = nullptr;
   int n_times = 0;
   void upload_times(const double* t, int n);
+  void upload_kept(DevBuf& b, const void* src, size_t bytes);
+  z128* h_state = nullptr;  // pinned copy of a resident launch's state
+  ResidentHost resident_host();
   int rkdp_interval_resident(double t0, double t1, double dt_first, double atol, double rtol);
   int solve_dopri(void* rho_dev, const double* t_list, int n_t, double dt, double atol,
                   double rtol, void* rho_s_dev);
