@@ -448,9 +448,8 @@ int heom_mlp_loss_grad(heom_mlp_handle m, const float* X, const float* Y, int n_
                        double* loss, float* grad_host) {
   return guard([&] {
     if (!X || !Y || n_rows < 1) throw hamd::HeomError{HEOM_ERR_ARG, "heom_mlp_loss_grad: bad input"};
-    const double l = M(m).loss_grad(X, Y, n_rows, nullptr);
+    const double l = M(m).loss_grad(X, Y, n_rows, nullptr, grad_host);
     if (loss) *loss = l;
-    if (grad_host) M(m).get_grad(grad_host);
     return HEOM_OK;
   });
 }

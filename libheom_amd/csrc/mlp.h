@@ -33,9 +33,10 @@ class Mlp {
   void fit_scaling(const float* X, const float* Y, long long n_rows);
   // raw inputs -> raw outputs (normalisation applied inside)
   void forward(const float* X, float* Y, int n_rows);
-  // MSE of normalised outputs; gradient left in the device gradient buffer
-  double loss_grad(const float* X, const float* Y, int n_rows, const int* perm_dev);
-  void get_grad(float* host) const;
+  // MSE of normalised outputs; gradient left in the device gradient buffer and, with
+  // grad_host, copied there
+  double loss_grad(const float* X, const float* Y, int n_rows, const int* perm_dev,
+                   float* grad_host = nullptr);
   void adam_step(double lr, double beta1, double beta2, double eps);
   void train(const float* X, const float* Y, long long n_rows, int batch, int epochs, double lr,
              uint64_t seed, double* epoch_loss);
@@ -46,7 +47,9 @@ class Mlp {
   DevBuf params, grads, adam_m, adam_v;
   DevBuf xm_, xs_, ym_, ys_;  // normalisation: x' = (x - xm)/xs, y = y'*ys + ym
   DevBuf xb, h1, h2, yb, dh1, dh2, dyb, partials, perm;
-  DevBuf gparts, loss_;  // gradient slices of the k parts (n_par each), the loss
+  DevBuf gparts;  // gradient slices of the k parts (n_par each)
+  double* h_loss = nullptr;  // pinned: the loss, the gradient
+  float* h_grad = nullptr;
   int cap_rows = 0;
   long long t_adam = 0;
   void ensure_rows(int rows);

@@ -19,8 +19,8 @@ typedef float mf_f4 __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------
 // FP32 matrix products of the network on the f32 matrix cores (16x16x4, FP32
 // accumulation): a 64 x 64 output tile per workgroup of four waves (2 x 2
-// accumulators each), k in slices of 32 staged in LDS while the next slice is
-// in flight in registers.  LDS strides 36 (k contiguous) and 80 (m or n
+// accumulators each), k in slices of 32 staged in two LDS buffers while the next
+// four (weight gradients: two) are in flight in registers.  LDS strides 36 (k contiguous) and 80 (m or n
 // contiguous): the 64 lanes of an operand read hit 64 distinct banks.
 //
 // The sizes are small (4096 rows x 256 units: 256 tiles, one per CU; 0.5 GFLOP,
@@ -30,8 +30,9 @@ typedef float mf_f4 __attribute__((ext_vector_type(4)));
 // partial buffer that grad_reduce_kernel adds up in order.
 // Loss and gradient of 4096 rows of a 49-256-256-32 network: 4850 us with
 // unsplit 64 x 64 vector-ALU products (820 us per weight gradient, 880 us per
-// serial column sum), 180 us here (19 us per layer product, 18 us the three
-// weight gradients, 10 us their sum).
+// serial column sum); 203 us with one slice ahead (19 us per layer product, 10 us
+// the sum of the gradient's parts) and the results copied back, 126 us here (16 us,
+// 9 us, results written to pinned memory).
 // ---------------------------------------------------------------------------
 constexpr int kT = 64, kK = 32;
 constexpr int kLdK = kK + 4, kLdM = kT + 16;
@@ -98,8 +99,8 @@ struct Slice {
 
 template <bool TA, bool TB>
 __device__ void gemm_tile(const GemmArgs& g, int bx, int by, int bz, int wg) {
-  __shared__ __align__(16) float As[TA ? kK * kLdM : kT * kLdK];
-  __shared__ __align__(16) float Bs[TB ? kT * kLdK : kK * kLdM];
+  __shared__ __align__(16) float s_a[2][TA ? kK * kLdM : kT * kLdK];
+  __shared__ __align__(16) float s_b[2][TB ? kT * kLdK : kK * kLdM];
   __shared__ double s_loss[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lk = lane >> 4;
@@ -110,37 +111,50 @@ __device__ void gemm_tile(const GemmArgs& g, int bx, int by, int bz, int wg) {
   const bool vb = g.ldb % 4 == 0 && (reinterpret_cast<uintptr_t>(g.B) & 15) == 0;
   mf_f4 acc[2][2] = {};
   float asum = 0.f;
-  Slice<TA> a;
-  Slice<!TB> b;
-  a.load(g.A, g.lda, m0, g.M, k0, k1, va);
-  b.load(g.B, g.ldb, n0, g.N, k0, k1, vb);
-  for (int k = k0; k < k1; k += kK) {
-    __syncthreads();
-    a.store(As);
-    b.store(Bs);
-    __syncthreads();
-    if (k + kK < k1) {
-      a.load(g.A, g.lda, m0, g.M, k + kK, k1, va);
-      b.load(g.B, g.ldb, n0, g.N, k + kK, k1, vb);
-    }
+  // k slices in flight in registers (even: two LDS buffers); a part of a weight
+  // gradient has three workgroups per CU, which hide their loads already (four slices:
+  // 17.5 -> 20 us)
+  constexpr int kAhead = TA ? 2 : 4;
+  Slice<TA> a[kAhead];
+  Slice<!TB> b[kAhead];
+  auto load = [&](int p, int k) {
+    if (k >= k1) return;
+    a[p].load(g.A, g.lda, m0, g.M, k, k1, va);
+    b[p].load(g.B, g.ldb, n0, g.N, k, k1, vb);
+  };
 #pragma unroll
-    for (int s = 0; s < kK / 4; ++s) {
-      const int kk = 4 * s + lk;
-      float av[2], bv[2];
+  for (int p = 0; p < kAhead; ++p) load(p, k0 + p * kK);
+  for (int kb = k0; kb < k1; kb += kAhead * kK) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int m = wm + 16 * t + lr, n = wn + 16 * t + lr;
-        av[t] = TA ? As[kk * kLdM + m] : As[m * kLdK + kk];
-        bv[t] = TB ? Bs[n * kLdK + kk] : Bs[kk * kLdM + n];
+    for (int p = 0; p < kAhead; ++p) {
+      const int k = kb + p * kK;
+      if (k >= k1) break;
+      // two LDS buffers, one barrier: the slice before the last was read by
+      // every wave before it reached the last barrier
+      float *As = s_a[p & 1], *Bs = s_b[p & 1];
+      a[p].store(As);
+      b[p].store(Bs);
+      __syncthreads();
+      load(p, k + kAhead * kK);
+#pragma unroll
+      for (int s = 0; s < kK / 4; ++s) {
+        const int kk = 4 * s + lk;
+        float av[2], bv[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int m = wm + 16 * t + lr, n = wn + 16 * t + lr;
+          av[t] = TA ? As[kk * kLdM + m] : As[m * kLdK + kk];
+          bv[t] = TB ? Bs[n * kLdK + kk] : Bs[kk * kLdM + n];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
       }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+      if (TA && g.asum && bx == 0 && threadIdx.x < kT)
+        for (int kk = 0; kk < kK; ++kk) asum += As[kk * kLdM + threadIdx.x];
     }
-    if (TA && g.asum && bx == 0 && threadIdx.x < kT)
-      for (int kk = 0; kk < kK; ++kk) asum += As[kk * kLdM + threadIdx.x];
   }
   if (TA && g.asum && bx == 0 && threadIdx.x < kT && m0 + static_cast<int>(threadIdx.x) < g.M)
     g.asum[bz * g.part_stride + m0 + threadIdx.x] = asum;
@@ -204,15 +218,26 @@ __global__ void __launch_bounds__(256) grad_kernel(const GradArgs a) {
 
 // grads[i] = sum over the parts, in order; workgroup 0 also adds up the loss
 // partials (fixed order) and divides by their element count
+// (out: host memory); host (may be null): the gradient in pinned host memory too
 __global__ void __launch_bounds__(256) grad_reduce_kernel(const float* parts, int n_parts,
                                                           long long n, float* grads,
                                                           const double* loss, int n_loss,
-                                                          double count, double* out) {
+                                                          double count, double* out,
+                                                          float* host) {
   const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
   if (i < n) {
     float s = 0.f;
-    for (int p = 0; p < n_parts; ++p) s += parts[p * n + i];
+    int p = 0;
+    for (; p + 8 <= n_parts; p += 8) {  // eight parts in flight, added in order
+      float v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = parts[(p + q) * n + i];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s += v[q];
+    }
+    for (; p < n_parts; ++p) s += parts[p * n + i];
     grads[i] = s;
+    if (host) host[i] = s;
   }
   if (blockIdx.x != 0) return;
   __shared__ double sd[256];
@@ -401,6 +426,8 @@ Mlp::Mlp(int n_in_, int n_hidden, int n_out_, uint64_t seed, int device_)
 
 Mlp::~Mlp() {
   if (stream) (void)hipStreamDestroy(stream);
+  if (h_loss) (void)hipHostFree(h_loss);
+  if (h_grad) (void)hipHostFree(h_grad);
 }
 
 float* Mlp::W1() const { return params.as<float>(); }
@@ -416,10 +443,6 @@ void Mlp::get_params(float* host) const {
 
 void Mlp::set_params(const float* host) {
   HAMD_HIP(hipMemcpy(params.p, host, sizeof(float) * n_par, hipMemcpyHostToDevice));
-}
-
-void Mlp::get_grad(float* host) const {
-  HAMD_HIP(hipMemcpy(host, grads.p, sizeof(float) * n_par, hipMemcpyDeviceToHost));
 }
 
 void Mlp::set_scaling(const float* xm, const float* xs, const float* ym, const float* ys) {
@@ -476,7 +499,6 @@ void Mlp::ensure_rows(int rows) {
   yb.alloc(sizeof(float) * rows * static_cast<size_t>(n_out));
   dyb.alloc(sizeof(float) * rows * static_cast<size_t>(n_out));
   partials.alloc(sizeof(double) * gemm_tiles(n_out) * gemm_tiles(rows));
-  loss_.alloc(sizeof(double));
   cap_rows = rows;
 }
 
@@ -508,9 +530,17 @@ void Mlp::forward(const float* X, float* Y, int n_rows) {
 // Forward, loss and gradient in eight launches (the gather, three layers with
 // the loss in the last one's epilogue, two backward products with the
 // derivative of tanh in theirs, the weight and bias gradients, their sum).
-double Mlp::loss_grad(const float* X, const float* Y, int rows, const int* perm_dev) {
+// Loss and, on request, gradient come back through pinned host memory that the last
+// kernel writes: one synchronisation and no copy commands.
+double Mlp::loss_grad(const float* X, const float* Y, int rows, const int* perm_dev,
+                      float* grad_host) {
   HAMD_HIP(hipSetDevice(device));
   ensure_rows(rows);
+  if (h_loss == nullptr)
+    HAMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_loss), 64, hipHostMallocCoherent));
+  if (grad_host && h_grad == nullptr)
+    HAMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_grad), sizeof(float) * n_par,
+                           hipHostMallocCoherent));
   const long long ni = static_cast<long long>(rows) * n_in, no = static_cast<long long>(rows) * n_out;
   hipLaunchKernelGGL(gather_norm_kernel, dim3(grid_for(ni)), dim3(256), 0, stream, X, perm_dev,
                      rows, n_in, xm_.as<float>(), xs_.as<float>(), xb.as<float>());
@@ -565,12 +595,11 @@ double Mlp::loss_grad(const float* X, const float* Y, int rows, const int* perm_
   hipLaunchKernelGGL(grad_kernel, dim3(ga.wg0[3]), dim3(256), 0, stream, ga);
   hipLaunchKernelGGL(grad_reduce_kernel, dim3(static_cast<int>((n_par + 255) / 256)), dim3(256), 0,
                      stream, gp, n_parts, n_par, grads.as<float>(), partials.as<double>(), n_loss,
-                     static_cast<double>(no), loss_.as<double>());
+                     static_cast<double>(no), h_loss, grad_host ? h_grad : nullptr);
   HAMD_HIP(hipGetLastError());
-  double loss = 0.0;
-  HAMD_HIP(hipMemcpyAsync(&loss, loss_.p, sizeof(double), hipMemcpyDeviceToHost, stream));
   HAMD_HIP(hipStreamSynchronize(stream));
-  return loss;
+  if (grad_host) std::memcpy(grad_host, h_grad, sizeof(float) * n_par);
+  return *h_loss;
 }
 
 void Mlp::adam_step(double lr, double beta1, double beta2, double eps) {
