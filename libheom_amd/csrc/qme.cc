@@ -423,10 +423,15 @@ void Qme::build_split_units(const std::vector<BlockMap>& bm) {
       size_t t = at * per;
       for (int l = gr.l0; l < gr.l1; l += gr.step) slots[t++] = links[l];
     }
-  d_sunits.upload(units);
-  d_slinks.upload(slots);
+  // one buffer for both: an allocation and a copy are 25 us each of the set-up
+  std::vector<char> all(sizeof(SplitUnit) * units.size() + sizeof(Link) * slots.size());
+  static_assert(sizeof(SplitUnit) % alignof(Link) == 0, "slots follow the units");
+  std::memcpy(all.data(), units.data(), sizeof(SplitUnit) * units.size());
+  std::memcpy(all.data() + sizeof(SplitUnit) * units.size(), slots.data(),
+              sizeof(Link) * slots.size());
+  d_sunits.upload(all);
   dev.sunits = d_sunits.as<SplitUnit>();
-  dev.slinks = d_slinks.as<Link>();
+  dev.slinks = reinterpret_cast<const Link*>(d_sunits.as<SplitUnit>() + units.size());
   dev.n_sunits = static_cast<int>(n * P / G);
   dev.slink_n = per;
 }

@@ -89,7 +89,7 @@ class Qme {
   FormDev dev{};
   hipStream_t stream = nullptr;
   DevBuf d_link_ptr, d_links, d_flat, d_cmac, d_coef, d_gam, d_H, d_V, d_Vd, d_dterm, d_sdelta;
-  DevBuf d_bmap, d_sunits, d_slinks;
+  DevBuf d_bmap, d_sunits;
   DevBuf d_R_ptr, d_R_col, d_R_val;
   long long csr_nnz = 0;  // redfield_liou
 
