@@ -748,6 +748,9 @@ def main():
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
             "kernel": "hilb_fast_kernel<7,double> (fused Dormand-Prince stage pass)",
+            "note": "mean of the seven passes of an attempt: the first is the step pass "
+                    "(dopri_step_kernel: k_1 comes from the last stage of the attempt before), "
+                    "six are operator passes; value counts the scheme's seven stages",
             "bytes_per_ado_stage": unit_bytes, "ados_per_launch": qme.n_hrchy,
             "bytes_per_launch": avg_bytes, "avg_launch_ms": avg_ms,
             "stage_ms": [float(x) for x in ms[:n]],

@@ -74,7 +74,8 @@ typedef struct heom_options {
 } heom_options;
 
 typedef struct heom_stats {
-  long long n_rhs;          /* calc_diff evaluations (RK stages) */
+  long long n_rhs;          /* Runge-Kutta stages (7 per rkdp attempt, whose first is
+                             * the last evaluation of the attempt before) */
   long long n_attempts;     /* rkdp attempts / rk4 steps */
   long long n_accepted;
   long long n_rejected;
