@@ -239,8 +239,10 @@ int heom_closure_rows(heom_handle deep, heom_handle shallow, const void* rho_dee
 /* solver_base::init via qme_solver (qme_solver.h:26-35).  The solver shares
  * ownership of the QME: heom_destroy(h) leaves it usable until
  * heom_solver_destroy.  If set_param is called again on h, the solver follows
- * the new parameters; a solve returns HEOM_ERR_STATE when h is not set up or
- * its main_size differs from the one the solver was created for. */
+ * the new parameters, also from a callback during heom_solve (from the interval
+ * that follows on; the same for a closure bound or unbound there); a solve
+ * returns HEOM_ERR_STATE when h is not set up or its main_size differs from the
+ * one the solver was created for. */
 int heom_solver_create(heom_handle h, int solver_kind, heom_solver_handle* out);
 int heom_solver_destroy(heom_solver_handle s);
 

@@ -119,7 +119,9 @@ Qme::~Qme() {
 
 using namespace supop;
 
+// Every change of the operator begins here (set_param, binding, unbinding).
 void Qme::clear_closure() {
+  ++generation;
   closure.reset();
   dev.clos = nullptr;
   dev.clos_lo = dev.clos_n = 0;
@@ -160,8 +162,10 @@ void Qme::set_param() {
   for (int u = 0; u < nn; ++u)
     if (!noise[u].set)
       throw HeomError{HEOM_ERR_ARG, "set_param: noise " + std::to_string(u) + " not set"};
+  uploaded = false;
   if (redfield()) {
     set_param_redfield();
+    uploaded = true;
     return;
   }
 
@@ -247,6 +251,7 @@ void Qme::set_param() {
   if ((kind == HEOM_LIOU || kind == HEOM_ADO) && N > 32)
     throw HeomError{HEOM_ERR_UNSUPPORTED, "heom_liou/heom_ado: n_level > 32"};
   upload();
+  uploaded = true;
   ready = true;
 }
 

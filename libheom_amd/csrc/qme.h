@@ -69,6 +69,10 @@ class Qme {
   bool H_set = false;
   std::vector<NoiseParams> noise;
   bool ready = false;
+  // Set-ups and closure (un)bindings so far: the operator of a solve changes when this
+  // does (in a callback), and a derivative stored before is stale.
+  unsigned long long generation = 0;
+  bool uploaded = false;  // the device tables are those of one whole set-up
   heom_hrchy_filter hrchy_filter = nullptr;
   void* hrchy_filter_user = nullptr;
 

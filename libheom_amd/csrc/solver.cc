@@ -159,6 +159,15 @@ void Solver::check_qme() const {
                                     "created; create a new solver"};
 }
 
+bool Solver::operator_changed(unsigned long long& gen) const {
+  if (q->generation == gen) return false;
+  gen = q->generation;
+  if (!q->uploaded || q->main_size() != ms)
+    throw HeomError{HEOM_ERR_STATE, "solver: set_param failed or changed the main_size during a "
+                                    "solve"};
+  return true;
+}
+
 // Physical buffer of a slot for ping-pong parity `cur` (slots 0..3 and the D
 // pair swap within their pair when cur == 1).
 void* Solver::slot_ptr(int s, int cur) const {
@@ -335,8 +344,17 @@ ResidentHost Solver::resident_host() {
   return ResidentHost{h_state, h_ctrl, mail};
 }
 
+// Small problems: an interval per resident launch.  The levels for which a
+// wavefront holds the same ADOs as a workgroup of the stage kernels: the
+// error norm is then the same sum, so the steps are decided alike (spin-boson
+// depth 6, ten intervals: 4.6 ms with the stage kernels, 0.52 ms here).
+bool Solver::dopri_interval_resident() const {
+  return use_resident && in_bytes == 8 && !q->opt.renorm_rho0 && q->dev.kind == HEOM_HILB &&
+         (q->N == 1 || q->N == 2 || q->N == 4) && resident_dopri_ok(q->dev, q->dev.max_links);
+}
+
 // One Dormand-Prince interval of a small problem in one resident launch, as
-// rkdp_interval: the state stays in slot SL_Y, the control block's counters add
+// run_attempts: the state stays in slot SL_Y, the control block's counters add
 // up over the intervals.
 int Solver::rkdp_interval_resident(double t0, double t1, double dt_first, double atol,
                                    double rtol) {
@@ -561,27 +579,38 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
   if (in_bytes == 4) launch_narrow(P[SL_Y32].p, P[SL_Y].p, ms, st);
   if (q->opt.renorm_rho0) launch_rho0_trace(P[SL_Y].p, q->N, d_tr0.as<double>(), st);
   int gave_up = 0;
+  unsigned long long gen = q->generation;
   if (kind != HEOM_RKDP) {  // fixed step: rk4, lsrk4
     for (int i = 0; i < n_t - 1; ++i) {
       on_output(i, P[SL_Y].p);
+      if (operator_changed(gen)) {
+        build_resident();
+        if (res.scheme == 0) host_state = nullptr;
+      }
       rk4_interval(t_list[i], t_list[i + 1], dt);
     }
     on_output(n_t - 1, P[SL_Y].p);
     HAMD_HIP(hipMemcpyAsync(rho_dev, P[SL_Y].p, bytes, hipMemcpyDeviceToDevice, st));
   } else {
-    // Small problems: an interval per resident launch.  The levels for which a
-    // wavefront holds the same ADOs as a workgroup of the stage kernels: the
-    // error norm is then the same sum, so the steps are decided alike (spin-boson
-    // depth 6, ten intervals: 4.6 ms with the stage kernels, 0.52 ms here).
-    const bool resident = use_resident && in_bytes == 8 && !q->opt.renorm_rho0 &&
-                          q->dev.kind == HEOM_HILB && (q->N == 1 || q->N == 2 || q->N == 4) &&
-                          resident_dopri_ok(q->dev, q->dev.max_links);
+    bool resident = dopri_interval_resident();
     std::memset(h_ctrl, 0, sizeof(Ctrl));
-    const double first = dt_save > 0.0 ? dt_save : dt;
+    double first = dt_save > 0.0 ? dt_save : dt;
+    Ctrl before{};  // counters of resident intervals that stage launches continue
     int cur = 0;
     bool started = false;
+    bool on_device = false;  // the device's control block carries the step size and counters
+    bool stale = true;       // SL_D is not D of the current state and operator
     for (int i = 0; i < n_t - 1; ++i) {
       on_output(i, P[cur].p);
+      if (operator_changed(gen)) {
+        stale = true;
+        if (resident && !dopri_interval_resident()) {
+          resident = false;
+          host_state = nullptr;
+          if (started) first = h_ctrl->dt;
+          before = *h_ctrl;
+        }
+      }
       // a zero-length interval takes no attempt and keeps the step size (the
       // reference would clamp the step to 0 and never finish the next interval)
       if (!(t_list[i + 1] > t_list[i])) continue;
@@ -589,13 +618,20 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
         gave_up |= rkdp_interval_resident(t_list[i], t_list[i + 1], started ? h_ctrl->dt : first,
                                           atol, rtol);
       } else {
-        launch_ctrl_init(ctrl_dev() + par, t_list[i], t_list[i + 1], started ? -1.0 : first, i,
+        launch_ctrl_init(ctrl_dev() + par, t_list[i], t_list[i + 1], on_device ? -1.0 : first, i,
                          st);
-        if (!started && !q->opt.renorm_rho0) launch_stage(0, 0.0);
+        if (stale && !q->opt.renorm_rho0) launch_stage(0, 0.0);
         gave_up |= run_attempts();
+        on_device = true;
+        stale = false;
       }
       started = true;
       cur = h_ctrl->cur;
+    }
+    if (on_device) {
+      h_ctrl->attempts += before.attempts;
+      h_ctrl->accepted += before.accepted;
+      h_ctrl->rejected += before.rejected;
     }
     on_output(n_t - 1, P[cur].p);
     if (started) dt_save = h_ctrl->dt;

@@ -78,6 +78,9 @@ class Solver {
   // throws HEOM_ERR_STATE unless the QME is set up with the size the solver's
   // buffers were allocated for (set_param may have been called again)
   void check_qme() const;
+  // whether a callback has changed the operator since `gen` (then moved on); the new
+  // one must fit this solver's buffers
+  bool operator_changed(unsigned long long& gen) const;
   void stage_bytes(std::vector<double>& bytes_out);
   int n_stages() const { return kind == HEOM_RKDP ? 7 : 4; }
 
@@ -135,6 +138,8 @@ class Solver {
   // of dt, then one step of dt_last
   static void fixed_steps(double t0, double t1, double dt, long long& n_full, double& dt_last);
   void build_resident();
+  // whether heom_solve runs Dormand-Prince intervals of this problem in resident launches
+  bool dopri_interval_resident() const;
 };
 
 }  // namespace hamd
