@@ -85,10 +85,13 @@ Solver::Solver(std::shared_ptr<Qme> q_, int kind_)
   if (kind == HEOM_RK4 || kind == HEOM_LSRK4) {
     mk(SL_ACC, z128b, 0);  // rk4: the accumulator; lsrk4: buff
   } else {
-    for (int k = 1; k < 5; ++k) mk(SL_K1 + k, sinb, lo);
+    // the error sum takes the buffer of k_2, which no stage reads any more when it is
+    // written (B_2 = E_2 = 0): ten state blocks (complex64: 7.5) in all
+    mk(SL_K1 + 1, z128b, lo);
+    sp[SL_E] = P[SL_K1 + 1].p;
+    for (int k = 2; k < 5; ++k) mk(SL_K1 + k, sinb, lo);
     mk(SL_D, sinb, lo);
     mk(SL_DNEW, sinb, lo);
-    mk(SL_E, z128b, 0);
   }
   if (q->opt.renorm_rho0) {
     if (q->kind == kBatch)
