@@ -107,7 +107,7 @@ class Solver {
   z128* step_rho_s = nullptr;
   void launch_step(int mode);
   unsigned long long wait_mail(unsigned long long seen);
-  int run_attempts();
+  int run_attempts(bool stale);
   void add_dopri_stats();
   Ctrl* ctrl_dev() const { return ext_ctrl ? ext_ctrl : d_ctrl.as<Ctrl>(); }
   double* partials_dev() const { return ext_partials ? ext_partials : d_partials.as<double>(); }
