@@ -195,7 +195,7 @@ __device__ __forceinline__ cx<R> batch_compute(const FormDev& d, const cx<R>* in
 // LOOP: a persistent grid (fewer workgroups than item groups).  With one group
 // per workgroup the loop is compiled out: around a loop the compiler keeps every
 // kernel argument in scalar registers and spills them (400 lane reads per item).
-template <typename R, bool F64, int KP, int IPW, int WPB, bool LOOP>
+template <typename R, bool F64, int KP, Epi E, int IPW, int WPB, bool LOOP>
 __global__ void __launch_bounds__(64 * WPB) batch_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
   __shared__ C s_rho[WPB][IPW][64];
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(64 * WPB) batch_kernel(const FormDev d, const 
       else
         D = batch_compute<0, false>(d, in, s_rho[w][q], s_H[w][q], b[q]);
       if (b[q].ok)
-        err_acc += epilogue<F64, R, KP>(b[q].pv, A, cur, At(b[q].I.elem, b[q].off), D, pg.alpha);
+        err_acc += epilogue<F64, R, KP, E>(b[q].pv, A, cur, At(b[q].I.elem, b[q].off), D, pg.alpha);
     }
     if constexpr (LOOP) {
       if constexpr (WPB > 1)
@@ -247,11 +247,13 @@ __global__ void __launch_bounds__(64 * WPB) batch_kernel(const FormDev d, const 
       g += gridDim.x;
     }
   } while (LOOP && g < 8 * per);
-  if (A.do_err) {
-    if constexpr (WPB > 1)
-      write_partial_wave(A, err_acc, static_cast<int>(blockIdx.x) * WPB + w);
-    else
-      write_partial(A, err_acc);
+  if constexpr (E == EPI_D) {
+    if (A.do_err) {
+      if constexpr (WPB > 1)
+        write_partial_wave(A, err_acc, static_cast<int>(blockIdx.x) * WPB + w);
+      else
+        write_partial(A, err_acc);
+    }
   }
 }
 
@@ -270,30 +272,42 @@ int launch_batch(const FormDev& d, const StageArgs& A, hipStream_t st) {
   const int ipw = d.batch_ipw == 2 ? 2 : 1;
   const int groups = 8 * ((d.n_items + 8 * wpb * ipw - 1) / (8 * wpb * ipw));
   const int grid = std::max(1, std::min({d.batch_grid, groups, kMaxGrid / wpb}));
-  const bool small = A.npre <= kBatchPre && A.pre_lo == 0;
-#define HAMD_BATCH_L(IPW, WPB, KP)                                                            \
-  {                                                                                           \
-    if (grid < groups)                                                                        \
-      hipLaunchKernelGGL((batch_kernel<R, F64, KP, IPW, WPB, true>), dim3(grid),              \
-                         dim3(64 * WPB), 0, st, d, A);                                        \
-    else                                                                                      \
-      hipLaunchKernelGGL((batch_kernel<R, F64, KP, IPW, WPB, false>), dim3(groups),           \
-                         dim3(64 * WPB), 0, st, d, A);                                        \
+  const auto run = [&](auto kp, auto epi) {
+    constexpr int KP = decltype(kp)::value;
+    constexpr Epi E = decltype(epi)::value;
+#define HAMD_BATCH(IPW, WPB)                                                                   \
+  {                                                                                            \
+    if (grid < groups)                                                                         \
+      hipLaunchKernelGGL((batch_kernel<R, F64, KP, E, IPW, WPB, true>), dim3(grid),           \
+                         dim3(64 * WPB), 0, st, d, A);                                         \
+    else                                                                                       \
+      hipLaunchKernelGGL((batch_kernel<R, F64, KP, E, IPW, WPB, false>), dim3(groups),        \
+                         dim3(64 * WPB), 0, st, d, A);                                         \
   }
-#define HAMD_BATCH(IPW, WPB)                                          \
-  {                                                                   \
-    if (small) HAMD_BATCH_L(IPW, WPB, kBatchPre) else HAMD_BATCH_L(IPW, WPB, kMaxPre) \
+#define HAMD_BATCH_W(IPW)                \
+  {                                      \
+    if (wpb == 4) HAMD_BATCH(IPW, 4)     \
+    else if (wpb == 2) HAMD_BATCH(IPW, 2) \
+    else HAMD_BATCH(IPW, 1)              \
   }
-#define HAMD_BATCH_W(IPW)                   \
-{                                         \
-  if (wpb == 4) HAMD_BATCH(IPW, 4)        \
-  else if (wpb == 2) HAMD_BATCH(IPW, 2)   \
-  else HAMD_BATCH(IPW, 1)                 \
-}
-  if (ipw == 2) HAMD_BATCH_W(2) else HAMD_BATCH_W(1)
+    if (ipw == 2) HAMD_BATCH_W(2) else HAMD_BATCH_W(1)
 #undef HAMD_BATCH_W
 #undef HAMD_BATCH
-#undef HAMD_BATCH_L
+  };
+  if (A.npre <= kBatchPre && A.pre_lo == 0 && A.epi != EPI_D) {
+    if (A.epi == EPI_RK)
+      run(KpTag<kBatchPre>{}, EpiTag<EPI_RK>{});
+    else
+      run(KpTag<kBatchPre>{}, EpiTag<EPI_K>{});
+  } else if (A.epi == EPI_K) {
+    run(KpTag<kMaxPre>{}, EpiTag<EPI_K>{});
+  } else if (A.epi == EPI_D) {
+    run(KpTag<4>{}, EpiTag<EPI_D>{});  // three operands at most
+  } else if constexpr (!F64) {  // a derivative added to a complex64 one
+    run(KpTag<kMaxPre>{}, EpiTag<EPI_RK>{});
+  } else {
+    throw HeomError{HEOM_ERR_STATE, "batch: operands of the pass"};
+  }
   return grid * wpb;  // error-norm partials: one per wavefront
 }
 

@@ -125,6 +125,13 @@ enum SlotType { ST_C128 = 0, ST_C64 = 1 };
 
 enum Mode { MODE_DIFF = 0, MODE_STAGE = 1 };
 
+// What a kernel's epilogue is compiled for: RK4 and lsrk4 stages and derivatives; the
+// Dormand-Prince stages that store k, with D of the current state as operand 1; and
+// those that store D, one of them with the error norm.  (One epilogue for all, told
+// apart at run time, took an 81st register in hilb_fast_kernel<7,double>, five waves per
+// SIMD instead of six, and private memory in 200 kernels: 7-site RK4 pass 15.7 us, 14.8 without.)
+enum Epi { EPI_RK = 0, EPI_K = 1, EPI_D = 2 };
+
 constexpr int kMaxPre = 8;  // state-sized operands an epilogue may read per element
 
 // Epilogue of one operator pass, applied per element after D is known.  All
@@ -134,12 +141,12 @@ constexpr int kMaxPre = 8;  // state-sized operands an epilogue may read per ele
 //   pv[s] = pre[cur][s] at this element (loaded before the operator work)
 // MODE_DIFF : dst[0] = beta*pv[0] - alpha*D      (pv[0] = old drho when beta != 0)
 // MODE_STAGE: k = -dt*D (dt from the control block when attached, else a_re)
-//             k[cur] <- k, or D itself with k_raw (optional)
-//             d_pre: operand 1 holds a stored D; it stands for k_1 = -dt*D
+//             k[cur] <- k (null: not stored), or D itself, by epi
+//             EPI_K: operand 1 holds a stored D; it stands for k_1 = -dt*D
 //             dst[c] (and dst2[c]) <- sum_s cc[c][s]*pv[s] + ck[c]*k, summed in s order
 //             with zero coefficients skipped (so the order follows the reference)
-//   error norm (rkdp.h:142-153): e = sum_s ec[s]*pv[s] + ek*k,
-//             w = |e| / (atol + rtol*max(|pv[ynew]|, |pv[yold]|)); sum of w^2 per workgroup
+//   error norm (rkdp.h:142-153): e = pv[0] + ek*k, w = |e| / (atol + rtol*max(|pv[1]|, |pv[2]|))
+//             with y_new and y_old in pv[1], pv[2]; sum of w^2 per workgroup
 struct StageArgs {
   int mode;
   const void* in[2];  // operator input (neighbour reads)
@@ -150,8 +157,7 @@ struct StageArgs {
   unsigned pre_lo;
   void* k[2];  // null: k not stored
   int k_lo;
-  int k_raw;
-  int d_pre;
+  Epi epi;
   int ncombo;
   double cc[2][kMaxPre];
   double ck[2];
@@ -159,9 +165,7 @@ struct StageArgs {
   void* dst2[2][2];  // null: none
   int dst_lo[2], dst2_lo[2];
   int do_err;
-  double ec[kMaxPre];
   double ek;
-  int ynew_pre, yold_pre;
   double atol, rtol;
   Ctrl* ctrl;
   double* partials;

@@ -30,7 +30,7 @@ inline size_t fast_vd_lds(const FormDev& d, bool real, int real_bytes) {
   const size_t rows = static_cast<size_t>(d.n_noise + 1) * d.N;
   return rows * (real ? 1 : 2) * static_cast<size_t>(real_bytes);
 }
-template <int N, typename R, bool REAL, bool F64, int KP>
+template <int N, typename R, bool REAL, bool F64, int KP, Epi E>
 __global__ void __launch_bounds__(WaveCfg<N>::BS, 1)
     hilb_fast_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
@@ -152,14 +152,17 @@ __global__ void __launch_bounds__(WaveCfg<N>::BS, 1)
   double w2 = 0.0;
   if (lane_ok) {
     add_closure(d, gi, D);
-    w2 = epilogue<F64, R, KP>(pv, A, cur, gi, D, pg.alpha);
+    w2 = epilogue<F64, R, KP, E>(pv, A, cur, gi, D, pg.alpha);
   }
-  if (A.do_err) write_partial(A, w2);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, w2);
 }
 
 // ---------------------------------------------------------------------------
 // heom_hilb, general path: any V, N <= 16; N <= 8 packs 64/N^2 ADOs per
-// wavefront (heom_hilb.h:96-212)
+// wavefront (heom_hilb.h:96-212).  N = 16 in FP32 is held to four waves per SIMD: with
+// dense V the compiler otherwise takes 137 registers (924 ADOs, RK4 pass: 32.5 us, 24.4 us
+// bounded); other sizes are as fast or faster unbounded.
 // ---------------------------------------------------------------------------
 template <int N>
 struct HilbCfg {
@@ -168,8 +171,8 @@ struct HilbCfg {
   static constexpr int APB = BS / N2;  // ADOs per workgroup
 };
 
-template <int N, typename R, bool DIAGV, bool F64, int KP>
-__global__ void __launch_bounds__(HilbCfg<N>::BS)
+template <int N, typename R, bool DIAGV, bool F64, int KP, Epi E>
+__global__ void __launch_bounds__(HilbCfg<N>::BS, N == 16 && sizeof(R) == 4 ? 4 : 1)
     hilb_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
   constexpr int N2 = N * N, APB = HilbCfg<N>::APB, BS = HilbCfg<N>::BS;
@@ -297,11 +300,12 @@ __global__ void __launch_bounds__(HilbCfg<N>::BS)
     }
     if (ok) {
       add_closure(d, gi, D);
-      err_acc += epilogue<F64, R, KP>(pv, A, cur, gi, D, pg.alpha);
+      err_acc += epilogue<F64, R, KP, E>(pv, A, cur, gi, D, pg.alpha);
     }
     __syncthreads();
   }
-  if (A.do_err) write_partial(A, err_acc);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, err_acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -313,7 +317,7 @@ __global__ void __launch_bounds__(HilbCfg<N>::BS)
 constexpr int kBigBS = 256;
 constexpr int kBigTile = 4;
 
-template <typename R, bool HLDS, bool F64, int KP>
+template <typename R, bool HLDS, bool F64, int KP, Epi E>
 __global__ void __launch_bounds__(kBigBS) hilb_big_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
   extern __shared__ __align__(16) unsigned char s_dyn[];
@@ -393,12 +397,13 @@ __global__ void __launch_bounds__(kBigBS) hilb_big_kernel(const FormDev d, const
           PreT<KP> pv;
           prefetch<F64, KP>(pv, A, cur, base + e, true);
           add_closure(d, base + e, D);
-          err_acc += epilogue<F64, R, KP>(pv, A, cur, base + e, D, pg.alpha);
+          err_acc += epilogue<F64, R, KP, E>(pv, A, cur, base + e, D, pg.alpha);
         }
     }
     __syncthreads();
   }
-  if (A.do_err) write_partial(A, err_acc);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, err_acc);
 }
 
 template <int N, typename R, bool F64>
@@ -410,49 +415,34 @@ int launch_hilb_n(const FormDev& d, const StageArgs& A, hipStream_t st) {
     constexpr int BS = WaveCfg<N>::BS;
     const int grid = d.n_hrchy;
     const size_t lds = fast_vd_lds(d, real, sizeof(R));
-    // four prefetched operands cover every stage except the last Dormand-Prince one
-    const bool small = A.npre <= 4;
-    const bool mid = A.npre <= 6;  // Dormand-Prince stages 5 and 6
-    if (real) {
-      if (small)
-        hipLaunchKernelGGL((hilb_fast_kernel<N, R, true, F64, 4>), dim3(grid), dim3(BS), lds, st,
-                           d, A);
-      else if (mid)
-        hipLaunchKernelGGL((hilb_fast_kernel<N, R, true, F64, 6>), dim3(grid), dim3(BS), lds, st,
-                           d, A);
-      else
-        hipLaunchKernelGGL((hilb_fast_kernel<N, R, true, F64, kMaxPre>), dim3(grid), dim3(BS),
-                           lds, st, d, A);
-      return grid;
-    } else {
-      if (small)
-        hipLaunchKernelGGL((hilb_fast_kernel<N, R, false, F64, 4>), dim3(grid), dim3(BS), lds,
-                           st, d, A);
-      else
-        hipLaunchKernelGGL((hilb_fast_kernel<N, R, false, F64, kMaxPre>), dim3(grid), dim3(BS),
-                           lds, st, d, A);
-      return grid;
-    }
+    // four prefetched operands cover every stage but Dormand-Prince's fifth and sixth
+    const auto run = [&](auto real_, auto kp, auto epi) {
+      hipLaunchKernelGGL(
+          (hilb_fast_kernel<N, R, decltype(real_)::value, F64, decltype(kp)::value,
+                            decltype(epi)::value>),
+          dim3(grid), dim3(BS), lds, st, d, A);
+    };
+    if (real)
+      with_epilogue<4, 6>(A, [&](auto kp, auto epi) { run(std::true_type{}, kp, epi); });
+    else
+      with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) { run(std::false_type{}, kp, epi); });
+    return grid;
   }
   constexpr int APB = HilbCfg<N>::APB, BS = HilbCfg<N>::BS;
   const int grid = cap_grid((d.n_hrchy + APB - 1) / APB);
-  const bool small = A.npre <= 4;
-  if (d.diag_v) {
-    const size_t lds = sizeof(cx<R>) * (d.n_noise + 1) * N;
-    if (lds > 48 * 1024)
-      throw HeomError{HEOM_ERR_UNSUPPORTED, "heom_hilb: too many noises for the LDS tables"};
-    if (small)
-      hipLaunchKernelGGL((hilb_kernel<N, R, true, F64, 4>), dim3(grid), dim3(BS), lds, st, d, A);
-    else
-      hipLaunchKernelGGL((hilb_kernel<N, R, true, F64, kMaxPre>), dim3(grid), dim3(BS), lds, st,
-                         d, A);
-  } else {
-    if (small)
-      hipLaunchKernelGGL((hilb_kernel<N, R, false, F64, 4>), dim3(grid), dim3(BS), 0, st, d, A);
-    else
-      hipLaunchKernelGGL((hilb_kernel<N, R, false, F64, kMaxPre>), dim3(grid), dim3(BS), 0, st, d,
+  const size_t lds = d.diag_v ? sizeof(cx<R>) * (d.n_noise + 1) * N : 0;
+  if (lds > 48 * 1024)
+    throw HeomError{HEOM_ERR_UNSUPPORTED, "heom_hilb: too many noises for the LDS tables"};
+  with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) {
+    constexpr int KP = decltype(kp)::value;
+    constexpr Epi E = decltype(epi)::value;
+    if (d.diag_v)
+      hipLaunchKernelGGL((hilb_kernel<N, R, true, F64, KP, E>), dim3(grid), dim3(BS), lds, st, d,
                          A);
-  }
+    else
+      hipLaunchKernelGGL((hilb_kernel<N, R, false, F64, KP, E>), dim3(grid), dim3(BS), 0, st, d,
+                         A);
+  });
   return grid;
 }
 template <typename R, bool F64>
@@ -465,23 +455,18 @@ int launch_hilb_big(const FormDev& d, const StageArgs& A, hipStream_t st) {
                     "heom_hilb: n_level > 16 is provided for diagonal coupling operators V"};
   const size_t one = sizeof(cx<R>) * static_cast<size_t>(d.N2);
   const int grid = cap_grid(d.n_hrchy);
-  if (2 * one <= 64 * 1024) {
-    if (A.npre <= 4)
-      hipLaunchKernelGGL((hilb_big_kernel<R, true, F64, 4>), dim3(grid), dim3(kBigBS), 2 * one,
-                         st, d, A);
-    else
-      hipLaunchKernelGGL((hilb_big_kernel<R, true, F64, kMaxPre>), dim3(grid), dim3(kBigBS),
-                         2 * one, st, d, A);
-  } else if (one <= 64 * 1024) {
-    if (A.npre <= 4)
-      hipLaunchKernelGGL((hilb_big_kernel<R, false, F64, 4>), dim3(grid), dim3(kBigBS), one, st,
-                         d, A);
-    else
-      hipLaunchKernelGGL((hilb_big_kernel<R, false, F64, kMaxPre>), dim3(grid), dim3(kBigBS), one,
-                         st, d, A);
-  } else {
+  if (one > 64 * 1024)
     throw HeomError{HEOM_ERR_UNSUPPORTED, "heom_hilb: one ADO block exceeds 64 KB of LDS"};
-  }
+  with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) {
+    constexpr int KP = decltype(kp)::value;
+    constexpr Epi E = decltype(epi)::value;
+    if (2 * one <= 64 * 1024)
+      hipLaunchKernelGGL((hilb_big_kernel<R, true, F64, KP, E>), dim3(grid), dim3(kBigBS),
+                         2 * one, st, d, A);
+    else
+      hipLaunchKernelGGL((hilb_big_kernel<R, false, F64, KP, E>), dim3(grid), dim3(kBigBS), one,
+                         st, d, A);
+  });
   return grid;
 }
 

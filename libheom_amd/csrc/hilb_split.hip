@@ -31,7 +31,7 @@ struct SplitCfg {
   static constexpr int BS = lanes * G;
 };
 
-template <int N, typename R, bool REAL, bool F64, int KP>
+template <int N, typename R, bool REAL, bool F64, int KP, Epi E>
 __global__ void __launch_bounds__(SplitCfg<N>::BS)
     hilb_split_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
@@ -188,9 +188,10 @@ __global__ void __launch_bounds__(SplitCfg<N>::BS)
   if (own) {
     cmac(D, gd, r);
     add_closure(d, gi, D);
-    w2 = epilogue<F64, R, KP>(pv, A, cur, gi, D, pg.alpha);
+    w2 = epilogue<F64, R, KP, E>(pv, A, cur, gi, D, pg.alpha);
   }
-  if (A.do_err) write_partial(A, w2);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, w2);
 }
 
 template <int N, typename R, bool F64>
@@ -198,12 +199,14 @@ int launch_split_n(const FormDev& d, const StageArgs& A, hipStream_t st) {
   const bool real = d.real_v && d.real_h;
   const size_t lds = split_vd_lds(d.n_noise, N, real, sizeof(R));
   const dim3 grid(d.n_sunits), block(SplitCfg<N>::BS);
-  if (real && A.npre <= 4)
-    hipLaunchKernelGGL((hilb_split_kernel<N, R, true, F64, 4>), grid, block, lds, st, d, A);
-  else if (real)
-    hipLaunchKernelGGL((hilb_split_kernel<N, R, true, F64, 6>), grid, block, lds, st, d, A);
-  else
-    hipLaunchKernelGGL((hilb_split_kernel<N, R, false, F64, 6>), grid, block, lds, st, d, A);
+  with_epilogue<4, 6>(A, [&](auto kp, auto epi) {
+    constexpr Epi E = decltype(epi)::value;
+    if (real)
+      hipLaunchKernelGGL((hilb_split_kernel<N, R, true, F64, decltype(kp)::value, E>), grid,
+                         block, lds, st, d, A);
+    else
+      hipLaunchKernelGGL((hilb_split_kernel<N, R, false, F64, 6, E>), grid, block, lds, st, d, A);
+  });
   return d.n_sunits;
 }
 
@@ -211,7 +214,6 @@ int launch_split_n(const FormDev& d, const StageArgs& A, hipStream_t st) {
 
 template <typename R, bool F64>
 int launch_hilb_split(const FormDev& d, const StageArgs& A, hipStream_t st) {
-  if (A.npre > 6) throw HeomError{HEOM_ERR_STATE, "hilb_split: more than six operands"};
   switch (d.N) {
 #define HAMD_CASE(n) \
   case n:            \

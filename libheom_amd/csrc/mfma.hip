@@ -214,7 +214,8 @@ __device__ __forceinline__ void mfma_commutator_bf16x3(const FormDev& d, const f
 // (32 or 64); the ADO block is n x n with n = d.N in (N/2, N] for N = 64, in
 // (16, 32] for N = 32, zero-padded in LDS (and H in its planes), so that the
 // padded rows and columns of the products are exactly zero.
-template <int N, typename R, bool REALH, bool F64, int KP, bool BF16X3, bool PADDED, int BS>
+template <int N, typename R, bool REALH, bool F64, int KP, Epi E, bool BF16X3, bool PADDED,
+          int BS>
 __global__ void __launch_bounds__(BS, BS / 128)
     hilb_mfma_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
@@ -397,13 +398,18 @@ __global__ void __launch_bounds__(BS, BS / 128)
         const int x = x0 + c * BS;
         if (x < n2) {
           add_closure(d, base + x, Dc[c]);
-          err_acc += epilogue<F64, R, KP>(pv[c], A, cur, base + x, Dc[c], pg.alpha);
+          // FP64 at N = 64 reads the coefficients ahead of its eight passes: Dormand-Prince
+          // pass of 969 ADOs 117.1 us on average, 121.2 read in each pass (RK4 and the
+          // other sizes and types are 1-6% faster with the latter)
+          err_acc += epilogue<F64, R, KP, E, sizeof(R) == 8 && N == 64 && E == EPI_K>(
+              pv[c], A, cur, base + x, Dc[c], pg.alpha);
         }
       }
     }
     __syncthreads();
   }
-  if (A.do_err) write_partial(A, err_acc);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, err_acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -507,7 +513,7 @@ template <int N, typename R>
 constexpr int kDenseWps = N == 64 ? (sizeof(R) == 8 ? 2 : 4)
                           : N == 48 ? (sizeof(R) == 8 ? 3 : 4) : (sizeof(R) == 8 ? 3 : 4);
 
-template <int N, typename R, bool REALV, bool REALH, bool F64, int KP, bool PADDED, int BS>
+template <int N, typename R, bool REALV, bool REALH, bool F64, int KP, Epi E, bool PADDED, int BS>
 __global__ void __launch_bounds__(BS, (kDenseWps<N, R>))
     hilb_mfma_dense_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
@@ -704,12 +710,13 @@ __global__ void __launch_bounds__(BS, (kDenseWps<N, R>))
         prefetch<F64, KP>(pv, A, cur, base + at[t][r], true);
         if (in_block[t][r]) {
           add_closure(d, base + at[t][r], D[t][r]);
-          err_acc += epilogue<F64, R, KP>(pv, A, cur, base + at[t][r], D[t][r], pg.alpha);
+          err_acc += epilogue<F64, R, KP, E>(pv, A, cur, base + at[t][r], D[t][r], pg.alpha);
         }
       }
     __syncthreads();  // every wave has finished reading rho
   }
-  if (A.do_err) write_partial(A, err_acc);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, err_acc);
 }
 
 template <int N, typename R, bool F64, bool BF16X3>
@@ -720,31 +727,32 @@ int launch_hilb_mfma_n(const FormDev& d, const StageArgs& A, hipStream_t st) {
   if (lds > kMfmaLdsCap)
     throw HeomError{HEOM_ERR_UNSUPPORTED, "matrix-core path: too many noises for LDS"};
   const int grid = cap_grid(d.n_hrchy);
-  const bool small = A.npre <= 4;
   // N = 64: eight waves per ADO, each with half the output tiles (two
   // workgroups per CU either way, so twice the waves work on the same ADOs;
   // measured at 969 ADOs per Dormand-Prince stage: FP64 135 against 158 us,
   // split-bf16 99 against 138 us, complex64 with the links outer 112 against
   // 126 us)
   constexpr int BS = MfmaCfg<N>::BS;
-#define HAMD_MFMA(REALH, KP, PAD)                                                \
-  {                                                                              \
-    auto k = hilb_mfma_kernel<N, R, REALH, F64, KP, BF16X3, PAD, BS>;            \
-    static bool once = (allow_lds(k, kMfmaLdsCap), true);                        \
-    (void)once;                                                                  \
-    hipLaunchKernelGGL(k, dim3(grid), dim3(BS), lds, st, d, A);                  \
+  const auto run = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(BS), lds, st, d, A);
+  };
+  with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) {
+    constexpr int KP = decltype(kp)::value;
+    constexpr Epi E = decltype(epi)::value;
+#define HAMD_MFMA(REALH, PAD)                                             \
+  {                                                                       \
+    auto k = hilb_mfma_kernel<N, R, REALH, F64, KP, E, BF16X3, PAD, BS>; \
+    static bool once = (allow_lds(k, kMfmaLdsCap), true);                 \
+    (void)once;                                                           \
+    run(k);                                                               \
   }
-#define HAMD_MFMA_P(REALH, KP)                          \
-  {                                                     \
-    if (d.N == N) HAMD_MFMA(REALH, KP, false) else HAMD_MFMA(REALH, KP, true) \
-  }
-  if (d.real_h) {
-    if (small) HAMD_MFMA_P(true, 4) else HAMD_MFMA_P(true, kMaxPre)
-  } else {
-    if (small) HAMD_MFMA_P(false, 4) else HAMD_MFMA_P(false, kMaxPre)
-  }
-#undef HAMD_MFMA_P
+    if (d.real_h) {
+      if (d.N == N) HAMD_MFMA(true, false) else HAMD_MFMA(true, true)
+    } else {
+      if (d.N == N) HAMD_MFMA(false, false) else HAMD_MFMA(false, true)
+    }
 #undef HAMD_MFMA
+  });
   return grid;
 }
 
@@ -755,33 +763,34 @@ int launch_hilb_mfma_dense_n(const FormDev& d, const StageArgs& A, hipStream_t s
   if (lds > kMfmaLdsCap)
     throw HeomError{HEOM_ERR_UNSUPPORTED, "matrix-core path: the blocks exceed LDS"};
   const int grid = cap_grid(d.n_hrchy);
-  const bool small = A.npre <= 4;
   // N = 64: eight waves per ADO (measured at 969 ADOs: 497 against 715 us per
   // FP64 stage, 309 against 364 us complex64)
   constexpr int BS = MfmaCfg<N>::BS;
-#define HAMD_MD(REALV, REALH, KP, PAD)                                                 \
-  {                                                                                    \
-    auto k = hilb_mfma_dense_kernel<N, R, REALV, REALH, F64, KP, PAD, BS>;             \
-    static bool once = (allow_lds(k, kMfmaLdsCap), true);                              \
-    (void)once;                                                                        \
-    hipLaunchKernelGGL(k, dim3(grid), dim3(BS), lds, st, d, A);                        \
+  const auto run = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(BS), lds, st, d, A);
+  };
+  with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) {
+    constexpr int KP = decltype(kp)::value;
+    constexpr Epi E = decltype(epi)::value;
+#define HAMD_MD(REALV, REALH, PAD)                                             \
+  {                                                                            \
+    auto k = hilb_mfma_dense_kernel<N, R, REALV, REALH, F64, KP, E, PAD, BS>; \
+    static bool once = (allow_lds(k, kMfmaLdsCap), true);                      \
+    (void)once;                                                                \
+    run(k);                                                                    \
   }
-#define HAMD_MD_P(REALV, REALH, KP) \
-  {                                 \
-    if (d.N == N) HAMD_MD(REALV, REALH, KP, false) else HAMD_MD(REALV, REALH, KP, true) \
-  }
-#define HAMD_MD_K(REALV, REALH) \
+#define HAMD_MD_P(REALV, REALH) \
   {                             \
-    if (small) HAMD_MD_P(REALV, REALH, 4) else HAMD_MD_P(REALV, REALH, kMaxPre) \
+    if (d.N == N) HAMD_MD(REALV, REALH, false) else HAMD_MD(REALV, REALH, true) \
   }
-  if (d.real_vd) {
-    if (d.real_h) HAMD_MD_K(true, true) else HAMD_MD_K(true, false)
-  } else {
-    if (d.real_h) HAMD_MD_K(false, true) else HAMD_MD_K(false, false)
-  }
-#undef HAMD_MD_K
+    if (d.real_vd) {
+      if (d.real_h) HAMD_MD_P(true, true) else HAMD_MD_P(true, false)
+    } else {
+      if (d.real_h) HAMD_MD_P(false, true) else HAMD_MD_P(false, false)
+    }
 #undef HAMD_MD_P
 #undef HAMD_MD
+  });
   return grid;
 }
 

@@ -136,7 +136,6 @@ StageArgs Qme::diff_args(void* drho, const void* rho, z128 alpha, z128 beta) con
   A.in_lo = l;
   A.dst[0][0] = A.dst[0][1] = drho;
   A.dst_lo[0] = l;
-  A.ynew_pre = A.yold_pre = -1;
   if (beta.re != 0.0 || beta.im != 0.0) {
     A.npre = 1;
     A.pre[0][0] = A.pre[1][0] = drho;

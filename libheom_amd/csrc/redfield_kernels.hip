@@ -21,7 +21,7 @@ namespace {
 //     into LDS, a barrier, and D += [V_u, T_u].
 // LDS (cx<R> elements): rho, H or HL, HR (DIAG), per noise Lambda_u, Lambda_u^+
 // and V_u (dense), then v_u (DIAG) or T (dense).
-template <typename R, bool F64, int KP, bool DIAG>
+template <typename R, bool F64, int KP, Epi E, bool DIAG>
 __global__ void __launch_bounds__(256) redfield_small_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
   extern __shared__ __align__(16) unsigned char rf_lds[];
@@ -109,8 +109,9 @@ __global__ void __launch_bounds__(256) redfield_small_kernel(const FormDev d, co
     }
   }
   double err = 0.0;
-  if (ok) err = epilogue<F64, R, KP>(pv, A, cur, e, D, pg.alpha);
-  if (A.do_err) write_partial(A, err);
+  if (ok) err = epilogue<F64, R, KP, E>(pv, A, cur, e, D, pg.alpha);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, err);
 }
 
 // Larger problems, first pass: T_u = Lambda_u rho - rho Lambda_u^+ for every
@@ -143,7 +144,7 @@ __global__ void __launch_bounds__(256) redfield_t_kernel(const FormDev d, const 
 
 // Larger problems, second pass: D = i[H, rho] + sum_u [V_u, T_u] (diagonal V:
 // (v_i - v_j) T_u[i][j]) and the stage epilogue, one lane per element.
-template <typename R, bool F64, int KP>
+template <typename R, bool F64, int KP, Epi E>
 __global__ void __launch_bounds__(256) redfield_d_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
   const Prologue pg = prologue(A);
@@ -176,16 +177,17 @@ __global__ void __launch_bounds__(256) redfield_d_kernel(const FormDev d, const 
         }
       }
     }
-    err_acc += epilogue<F64, R, KP>(pv, A, cur, e, D, pg.alpha);
+    err_acc += epilogue<F64, R, KP, E>(pv, A, cur, e, D, pg.alpha);
   }
-  if (A.do_err) write_partial(A, err_acc);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, err_acc);
 }
 
 // Sparse superoperator times the state, one 64-lane wavefront per row: the
 // lanes stride over the row's entries (coalesced) and reduce with shuffles;
 // lane 0 runs the epilogue.  Used for redfield_liou, whose rows hold up to
 // N^2 entries (R = L - sum_u Phi_u Theta_u).
-template <typename R, bool F64, int KP>
+template <typename R, bool F64, int KP, Epi E>
 __global__ void __launch_bounds__(256) csr_wave_kernel(const FormDev d, const StageArgs A) {
   using C = cx<R>;
   const Prologue pg = prologue(A);
@@ -206,36 +208,37 @@ __global__ void __launch_bounds__(256) csr_wave_kernel(const FormDev d, const St
       D.re += __shfl_down(D.re, off, 64);
       D.im += __shfl_down(D.im, off, 64);
     }
-    if (lane == 0) err_acc += epilogue<F64, R, KP>(pv, A, cur, r, D, pg.alpha);
+    if (lane == 0) err_acc += epilogue<F64, R, KP, E>(pv, A, cur, r, D, pg.alpha);
   }
-  if (A.do_err) write_partial(A, err_acc);
+  if constexpr (E == EPI_D)
+    if (A.do_err) write_partial(A, err_acc);
 }
 
 }  // namespace
 
 template <typename R, bool F64>
 int launch_redfield(const FormDev& d, const StageArgs& A, hipStream_t st) {
-  const bool small = A.npre <= 4;
   if (d.kind == HEOM_REDFIELD_LIOU) {
     const int grid = cap_grid((d.main_size + 3) / 4);  // four rows per workgroup
-    if (small)
-      hipLaunchKernelGGL((csr_wave_kernel<R, F64, 4>), dim3(grid), dim3(256), 0, st, d, A);
-    else
-      hipLaunchKernelGGL((csr_wave_kernel<R, F64, kMaxPre>), dim3(grid), dim3(256), 0, st, d, A);
+    with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) {
+      hipLaunchKernelGGL((csr_wave_kernel<R, F64, decltype(kp)::value, decltype(epi)::value>),
+                         dim3(grid), dim3(256), 0, st, d, A);
+    });
     return grid;
   }
   const bool diag = d.rf_HL != nullptr;
   const size_t lds = redfield_lds_elems(d.N2, d.N, d.n_noise, diag) * sizeof(cx<R>);
   if (d.N <= 16 && lds <= kRedfieldLds) {
-#define HAMD_RF(DG, KPV)                                                                    \
-  hipLaunchKernelGGL((redfield_small_kernel<R, F64, KPV, DG>), dim3(1), dim3(256), lds, st, d, \
-                     A)
-    if (diag) {
-      if (small) HAMD_RF(true, 4); else HAMD_RF(true, kMaxPre);
-    } else {
-      if (small) HAMD_RF(false, 4); else HAMD_RF(false, kMaxPre);
-    }
-#undef HAMD_RF
+    with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) {
+      constexpr int KP = decltype(kp)::value;
+      constexpr Epi E = decltype(epi)::value;
+      if (diag)
+        hipLaunchKernelGGL((redfield_small_kernel<R, F64, KP, E, true>), dim3(1), dim3(256), lds,
+                           st, d, A);
+      else
+        hipLaunchKernelGGL((redfield_small_kernel<R, F64, KP, E, false>), dim3(1), dim3(256), lds,
+                           st, d, A);
+    });
     return 1;
   }
   if (d.rf_T == nullptr) throw HeomError{HEOM_ERR_STATE, "redfield_hilb: scratch missing"};
@@ -243,10 +246,10 @@ int launch_redfield(const FormDev& d, const StageArgs& A, hipStream_t st) {
   hipLaunchKernelGGL((redfield_t_kernel<R>), dim3(cap_grid((nt + 255) / 256)), dim3(256), 0, st,
                      d, A);
   const int grid = cap_grid((d.N2 + 255) / 256);
-  if (small)
-    hipLaunchKernelGGL((redfield_d_kernel<R, F64, 4>), dim3(grid), dim3(256), 0, st, d, A);
-  else
-    hipLaunchKernelGGL((redfield_d_kernel<R, F64, kMaxPre>), dim3(grid), dim3(256), 0, st, d, A);
+  with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) {
+    hipLaunchKernelGGL((redfield_d_kernel<R, F64, decltype(kp)::value, decltype(epi)::value>),
+                       dim3(grid), dim3(256), 0, st, d, A);
+  });
   return grid;
 }
 

@@ -199,8 +199,9 @@ StageArgs Solver::resolve(const StageSpec& s) const {
   for (size_t j = 0; j < s.pre.size(); ++j)
     if (s.pre[j] >= 0 && slo[s.pre[j]]) a.pre_lo |= 1u << j;
   a.k_lo = s.k_slot >= 0 ? slo[s.k_slot] : 0;
-  a.k_raw = s.k_slot >= SL_D ? 1 : 0;
-  a.d_pre = s.pre.size() > 1 && s.pre[1] == SL_D ? 1 : 0;
+  a.epi = kind != HEOM_RKDP ? EPI_RK : s.k_slot >= SL_D ? EPI_D : EPI_K;
+  if (a.epi == EPI_K && (s.pre.size() < 2 || s.pre[1] != SL_D))
+    throw HeomError{HEOM_ERR_STATE, "Dormand-Prince stage without D as operand 1"};
   a.ncombo = s.ncombo;
   std::memcpy(a.cc, s.cc, sizeof(a.cc));
   std::memcpy(a.ck, s.ck, sizeof(a.ck));
@@ -209,10 +210,7 @@ StageArgs Solver::resolve(const StageSpec& s) const {
     a.dst2_lo[k] = s.dst2[k] >= 0 ? slo[s.dst2[k]] : 0;
   }
   a.do_err = s.do_err;
-  std::memcpy(a.ec, s.ec, sizeof(a.ec));
   a.ek = s.ek;
-  a.ynew_pre = s.ynew_pre;
-  a.yold_pre = s.yold_pre;
   if (kind == HEOM_RKDP) a.ctrl = ctrl_dev();
   a.partials = partials_dev();
   return a;
@@ -311,13 +309,8 @@ void Solver::build_stages(double atol, double rtol) {
     a.in_slot = lo ? SL_YNEW32 : SL_YNEW;
     a.k_slot = SL_DNEW;
     a.do_err = 1;
-    a.ec[a.pre_index(SL_E)] = 1.0;
     a.ek = kDpE[6];
-    // the error weights read y_new / y_old from the last two operand positions
-    a.pre.push_back(SL_YNEW);
-    a.pre.push_back(SL_Y);
-    a.ynew_pre = 1;
-    a.yold_pre = 2;
+    a.pre = {SL_E, SL_YNEW, SL_Y};  // as the epilogue takes them
     specs.push_back(a);
   }
   for (auto& s : specs) {

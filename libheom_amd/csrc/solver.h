@@ -21,9 +21,7 @@ struct StageSpec {
   int dst[2] = {-1, -1};
   int dst2[2] = {-1, -1};
   int do_err = 0;
-  double ec[kMaxPre] = {};
   double ek = 0.0;
-  int ynew_pre = -1, yold_pre = -1;
   int pre_index(int slot);
   void combo(const std::vector<std::pair<int, double>>& terms, double ckv, int d, int d2 = -1);
 };

@@ -121,16 +121,17 @@ __device__ __forceinline__ void prefetch(PreT<KP>& p, const StageArgs& A, int cu
 
 // Linear combination sum_s c[s]*p[s] + ck*k, accumulated in s order.  Terms
 // with a zero coefficient add an exact zero, so the result equals the
-// sequential sum over the non-zero terms (reference order).
-template <int KP>
-__device__ __forceinline__ z128 combine(const PreT<KP>& p, const double* c, int npre, double ck,
-                                        z128 k) {
+// sequential sum over the non-zero terms (reference order).  P1: operand 1 is p1.
+template <bool P1, int KP, class C>
+__device__ __forceinline__ z128 combine(const PreT<KP>& p, z128 p1, const C& c, int npre,
+                                        double ck, z128 k) {
   z128 v{0.0, 0.0};
 #pragma unroll
   for (int s = 0; s < KP; ++s) {
     if (s < npre) {
-      v.re = fma(c[s], p.v[s].re, v.re);
-      v.im = fma(c[s], p.v[s].im, v.im);
+      const z128 q = P1 && s == 1 ? p1 : p.v[s];
+      v.re = fma(c[s], q.re, v.re);
+      v.im = fma(c[s], q.im, v.im);
     }
   }
   v.re = fma(ck, k.re, v.re);
@@ -145,49 +146,81 @@ __device__ __forceinline__ z128 scaled_k(z128 alpha, z128 D) {
 
 // Epilogue shared by all operator kernels.  D is the operator applied to the
 // stage input at flat element gi; returns w^2 of the error norm (or 0).
-template <bool F64, typename R, int KP>
-__device__ __forceinline__ double epilogue(PreT<KP> p, const StageArgs& A, int cur, At gi,
+// AHEAD: the coefficients as the compiler schedules them (see below).
+template <bool F64, typename R, int KP, Epi E, bool AHEAD = false>
+__device__ __forceinline__ double epilogue(const PreT<KP>& p, const StageArgs& A, int cur, At gi,
                                            cx<R> Dr, z128 alpha) {
   const z128 D = conv<double>(Dr);
   const z128 k = scaled_k(alpha, D);
-  if (A.mode == MODE_DIFF) {
-    z128 v = k;
-    if (A.npre > 0) {
-      const z128 o = p.v[0];
-      v = z128{A.b_re * o.re - A.b_im * o.im + k.re, A.b_re * o.im + A.b_im * o.re + k.im};
+  z128 p1{0.0, 0.0};
+  if constexpr (E == EPI_RK) {
+    if (A.mode == MODE_DIFF) {
+      z128 v = k;
+      if (A.npre > 0) {
+        const z128 o = p.v[0];
+        v = z128{A.b_re * o.re - A.b_im * o.im + k.re, A.b_re * o.im + A.b_im * o.re + k.im};
+      }
+      stz(pick(A.dst[0], cur), F64 ? false : A.dst_lo[0], gi, v);
+      return 0.0;
     }
-    stz(pick(A.dst[0], cur), F64 ? false : A.dst_lo[0], gi, v);
-    return 0.0;
-  }
-  if (void* kp = pick(A.k, cur)) stz(kp, F64 ? false : A.k_lo, gi, A.k_raw ? D : k);
-  if (A.d_pre) {
+  } else if constexpr (E == EPI_K) {
+    if (void* kp = pick(A.k, cur)) stz(kp, !F64, gi, k);
     // k_1 of the stored derivative, rounded as a stored k_1 would be
-    const z128 k1 = scaled_k(alpha, p.v[1]);
-    p.v[1] = (F64 || !(A.pre_lo & 2u)) ? k1 : conv<double>(conv<float>(k1));
+    p1 = scaled_k(alpha, p.v[1]);
+    if (!F64) p1 = conv<double>(conv<float>(p1));
+  } else {
+    stz(pick(A.k, cur), !F64, gi, D);
   }
+  // The coefficients are read from the kernel's arguments (FormDev, StageArgs) where they
+  // are used: read as A.cc, the compiler loads them ahead of the operator work and spills
+  // scalar registers across it (20 levels, FP64: RK4 pass 22.4 us, 21.4 here).  With more
+  // than four operands that takes a barrier besides (7-site stages 5 and 6: 36 spills, 20.4
+  // and 20.8 us; 0 and 19.2 and 19.6 us).
+  static_assert(sizeof(FormDev) % alignof(StageArgs) == 0, "second kernel argument");
+  auto ca = reinterpret_cast<cptr<StageArgs>>(
+      (cptr<char>)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(FormDev));
+  if constexpr (E == EPI_K && KP > 4 && !AHEAD) asm volatile("" : "+s"(ca));
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     if (c < A.ncombo) {
-      const z128 v = combine(p, A.cc[c], A.npre, A.ck[c], k);
+      const z128 v = AHEAD ? combine<E == EPI_K>(p, p1, A.cc[c], A.npre, A.ck[c], k)
+                           : combine<E == EPI_K>(p, p1, ca->cc[c], A.npre, ca->ck[c], k);
       stz(pick(A.dst[c], cur), F64 ? false : A.dst_lo[c], gi, v);
       if (void* d2 = pick(A.dst2[c], cur)) stz(d2, F64 ? false : A.dst2_lo[c], gi, v);
     }
   }
-  if (A.do_err) {
-    // the last two operands hold y_new / y_old (zero weights in ec)
-    const int np = A.npre;
-    const z128 e = combine(p, A.ec, np - 2, A.ek, k);
-    z128 yn{0.0, 0.0}, yo{0.0, 0.0};
-#pragma unroll
-    for (int s = 0; s < KP; ++s) {
-      if (s == np - 2) yn = p.v[s];
-      if (s == np - 1) yo = p.v[s];
+  if constexpr (E == EPI_D) {
+    if (A.do_err) {
+      // operands: the error sum of the six stages before, y_new, y_old
+      const z128 e{fma(A.ek, k.re, p.v[0].re), fma(A.ek, k.im, p.v[0].im)};
+      const double a1 = zabs(p.v[1]), a0 = zabs(p.v[2]);
+      const double w = zabs(e) / (A.atol + A.rtol * (a1 > a0 ? a1 : a0));
+      return w * w;
     }
-    const double a1 = zabs(yn), a0 = zabs(yo);
-    const double w = zabs(e) / (A.atol + A.rtol * (a1 > a0 ? a1 : a0));
-    return w * w;
   }
   return 0.0;
+}
+
+template <int KP>
+using KpTag = std::integral_constant<int, KP>;
+template <Epi E>
+using EpiTag = std::integral_constant<Epi, E>;
+
+// f(KP, epilogue) of a pass: at most KS operands, or (Dormand-Prince stages that store
+// k) KW.
+template <int KS, int KW, class F>
+void with_epilogue(const StageArgs& A, F&& f) {
+  const bool wide = A.npre > KS;
+  if (A.npre > KW || (wide && A.epi != EPI_K))
+    throw HeomError{HEOM_ERR_STATE, "operator pass: more operands than its kernel takes"};
+  if (A.epi == EPI_RK)
+    f(KpTag<KS>{}, EpiTag<EPI_RK>{});
+  else if (A.epi == EPI_D)
+    f(KpTag<KS>{}, EpiTag<EPI_D>{});
+  else if (!wide)
+    f(KpTag<KS>{}, EpiTag<EPI_K>{});
+  else
+    f(KpTag<KW>{}, EpiTag<EPI_K>{});
 }
 
 // Step control of rkdp::solve_adaptive_step (rkdp.h:97-177) for the attempt
