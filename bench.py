@@ -31,7 +31,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-GRAPHS = True  # small problems in resident launches (--no-graphs: every stage launched)
+GRAPHS = True  # resident launches and graph replay (--no-graphs: every stage launched)
 
 
 def alg_bytes_per_ado_stage(n_level, n_dim, method, sc=16):

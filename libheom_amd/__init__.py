@@ -522,6 +522,7 @@ class qme_solver:
         _capi.check(_capi.load().heom_solver_reset(self._s))
 
     def set_graphs(self, enable):
-        """Small problems in resident launches (default) or every stage kernel launched."""
+        """Small problems in resident launches and long runs from HIP graphs (default), or
+        every stage kernel launched."""
         self._graphs = bool(enable)
         _capi.check(_capi.load().heom_solver_set_graphs(self._s, int(bool(enable))))

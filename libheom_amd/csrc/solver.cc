@@ -112,6 +112,8 @@ Solver::Solver(std::shared_ptr<Qme> q_, int kind_)
 }
 
 Solver::~Solver() {
+  graphs.clear();
+  if (rec_stream) (void)hipStreamDestroy(rec_stream);
   if (h_ctrl) (void)hipHostFree(h_ctrl);
   if (h_times) (void)hipHostFree(h_times);
   if (h_state) (void)hipHostFree(h_state);
@@ -162,9 +164,11 @@ void Solver::check_qme() const {
                                     "created; create a new solver"};
 }
 
-bool Solver::operator_changed(unsigned long long& gen) const {
+bool Solver::operator_changed(unsigned long long& gen) {
   if (q->generation == gen) return false;
   gen = q->generation;
+  graphs.clear();
+  graph_warm = false;
   if (!q->uploaded || q->main_size() != ms)
     throw HeomError{HEOM_ERR_STATE, "solver: set_param failed or changed the main_size during a "
                                     "solve"};
@@ -219,6 +223,9 @@ StageArgs Solver::resolve(const StageSpec& s) const {
 void Solver::build_stages(double atol, double rtol) {
   specs.clear();
   stages.clear();
+  graphs.clear();
+  graph_warm = false;
+  direct_attempts = 0;
   const bool lo = in_bytes == 4;
   const int y_in = lo ? SL_Y32 : SL_Y;
   if (kind == HEOM_RK4) {
@@ -385,15 +392,49 @@ void Solver::renorm(bool with_ctrl) {
   launch_rho0_renorm(slot_ptr(SL_Y, 0), slot_ptr(SL_Y, with_ctrl ? 1 : 0),
                      lo ? slot_ptr(SL_Y32, 0) : nullptr,
                      lo ? slot_ptr(SL_Y32, with_ctrl ? 1 : 0) : nullptr,
-                     with_ctrl ? ctrl_dev() + par : nullptr, q->N, d_tr0.as<double>(), q->stream);
+                     with_ctrl ? ctrl_dev() + par : nullptr, q->N, d_tr0.as<double>(), stream());
 }
 
 void Solver::launch_stage(int s, double dt) {
   StageArgs a = stages[s];
   a.a_re = dt;
   if (a.ctrl) a.ctrl += par;
-  const int grid = q->operate(in_bytes, a, q->stream);
+  const int grid = q->operate(in_bytes, a, stream());
   if (a.do_err) n_partials = grid;
+}
+
+// A run of many short stages waits longer between its kernels when the host launches
+// them one by one (RK4, 16 000 stages of 364 ADOs of 2x2: 5.30 us per stage, 4.6 from
+// graphs), but a graph costs its instantiation, some 100 us, on every solve: fixed steps
+// are replayed in graphs of up to kGraphSteps steps when the solve takes kGraphMin of
+// them, Dormand-Prince attempts one at a time after kGraphAttempts of them.
+constexpr int kGraphSteps = 16, kGraphMin = 512, kGraphIntervals = 8, kGraphAttempts = 128;
+
+// Launch `body` from graph `key`, which is recorded the first time.  The body launches
+// kernels only (no copy or memset: replays of memset nodes have gone wrong).
+void Solver::replay(int key, const std::function<void()>& body) {
+  GraphExec& g = graphs[key];
+  if (g.exec == nullptr) {
+    if (rec_stream == nullptr)
+      HAMD_HIP(hipStreamCreateWithFlags(&rec_stream, hipStreamNonBlocking));
+    HAMD_HIP(hipStreamBeginCapture(rec_stream, hipStreamCaptureModeThreadLocal));
+    hipGraph_t graph = nullptr;
+    recording = true;
+    try {
+      body();
+    } catch (...) {
+      recording = false;
+      (void)hipStreamEndCapture(rec_stream, &graph);
+      if (graph) (void)hipGraphDestroy(graph);
+      throw;
+    }
+    recording = false;
+    HAMD_HIP(hipStreamEndCapture(rec_stream, &graph));
+    const hipError_t e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    HAMD_HIP(e);
+  }
+  HAMD_HIP(hipGraphLaunch(g.exec, q->stream));
 }
 
 // fixed_step_size_solver::solve_1 (fixed_step_size_solver.h:29-52): steps of
@@ -434,13 +475,21 @@ void Solver::rk4_interval(double t0, double t1, double dt) {
     stats.n_accepted += n_full + 1;
     return;
   }
-  // Launched one by one: the host enqueues a stage in less time than the device
-  // takes for the smallest, and graphs of the same launches have to be
-  // instantiated for every solve (7-site Dormand-Prince, five intervals: 4.60 ms
-  // with graphs, 4.30 without; 4-site chain, 160 RK4 stages: 1.27 and 1.20).
-  for (long long n = 0; n < n_full; ++n) {
+  const auto step = [&] {
     for (int s = 0; s < 4; ++s) launch_stage(s, dt);
     if (q->opt.renorm_rho0) renorm(false);
+  };
+  for (long long n = 0; n < n_full;) {
+    int size = graph_steps && graph_warm ? kGraphSteps : 1;
+    while (size > n_full - n) size = graph_parts ? size / 2 : 1;
+    if (size > 1)
+      replay(size, [&] {
+        for (int k = 0; k < size; ++k) step();
+      });
+    else
+      step();
+    graph_warm = true;
+    n += size;
   }
   for (int s = 0; s < 4; ++s) launch_stage(s, dt_1);  // the last (shortened) step
   if (q->opt.renorm_rho0) renorm(false);
@@ -472,7 +521,7 @@ void Solver::launch_step(int mode) {
   a.a21 = kDpA[1][0];
   a.n = ms;
   a.mail = mail;
-  launch_dopri_step(a, q->stream);
+  launch_dopri_step(a, stream());
 }
 
 // The device's progress word once it has moved past `seen` step passes.
@@ -526,6 +575,18 @@ int Solver::run_attempts(bool stale) {
     if (attempts < seen) {  // the attempt held back as possibly not needed
       evaluate();
       ++attempts;
+      ++direct_attempts;
+    }
+    if (use_resident && direct_attempts >= kGraphAttempts && !(v & 2) && steps < seen + 1 &&
+        attempts == steps) {
+      const int from = par;  // the step pass writes the other control block
+      replay(from, [&] {
+        step(false);
+        evaluate();
+      });
+      par = from ^ 1;
+      ++steps;
+      ++attempts;
     }
     if (steps < seen + 1) {
       step(false);
@@ -534,6 +595,7 @@ int Solver::run_attempts(bool stale) {
     if (!(v & 2) && attempts < seen + 1) {
       evaluate();
       ++attempts;
+      ++direct_attempts;
     }
   }
   HAMD_HIP(hipMemcpyAsync(h_ctrl, ctrl_dev() + par, sizeof(Ctrl), hipMemcpyDeviceToHost,
@@ -580,6 +642,17 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
   int gave_up = 0;
   unsigned long long gen = q->generation;
   if (kind != HEOM_RKDP) {  // fixed step: rk4, lsrk4
+    graph_steps = graph_parts = false;
+    if (use_resident && res.scheme == 0) {
+      long long total = 0, n = 0;
+      double last = 0.0;
+      for (int i = 0; i + 1 < n_t; ++i) {
+        fixed_steps(t_list[i], t_list[i + 1], dt, n, last);
+        total += n;
+      }
+      graph_steps = total >= kGraphMin;
+      graph_parts = graph_steps && n_t > kGraphIntervals;
+    }
     for (int i = 0; i < n_t - 1; ++i) {
       on_output(i, P[SL_Y].p);
       if (operator_changed(gen)) {
@@ -637,6 +710,7 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
     HAMD_HIP(hipMemcpyAsync(rho_dev, P[cur].p, bytes, hipMemcpyDeviceToDevice, st));
   }
   HAMD_HIP(hipStreamSynchronize(st));
+  graphs.clear();
   stats.ado_stage_updates = stats.n_rhs * q->hs.n_hrchy;
   stats.gave_up |= gave_up;
   return gave_up ? HEOM_ERR_STEP_REJECTED : HEOM_OK;
@@ -758,6 +832,7 @@ int Solver::solve_dopri(void* rho_dev, const double* t_list, int n_t, double dt,
     HAMD_HIP(hipMemcpyAsync(rho_dev, P[h_ctrl->cur].p, bytes, hipMemcpyDeviceToDevice, st));
   }
   HAMD_HIP(hipStreamSynchronize(st));
+  graphs.clear();
   // only intervals of positive length touch the step size (as in solve)
   if (first >= 0) dt_save = h_ctrl->dt;
   add_dopri_stats();

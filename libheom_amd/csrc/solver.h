@@ -2,6 +2,7 @@
 #pragma once
 
 #include <functional>
+#include <map>
 #include <memory>
 #include <vector>
 
@@ -26,6 +27,17 @@ struct StageSpec {
   void combo(const std::vector<std::pair<int, double>>& terms, double ckv, int d, int d2 = -1);
 };
 
+// An instantiated graph, destroyed with the object.
+struct GraphExec {
+  hipGraphExec_t exec = nullptr;
+  GraphExec() = default;
+  GraphExec(const GraphExec&) = delete;
+  GraphExec& operator=(const GraphExec&) = delete;
+  ~GraphExec() {
+    if (exec) (void)hipGraphExecDestroy(exec);
+  }
+};
+
 class Solver {
  public:
   Solver(std::shared_ptr<Qme> q, int kind);
@@ -38,7 +50,8 @@ class Solver {
   long long ms;    // main_size
   double dt_save = -1.0;
   heom_stats stats{};
-  // small problems in the resident integrators; false launches every stage kernel
+  // small problems in the resident integrators and long runs from graphs; false
+  // launches every stage kernel
   bool use_resident = true;
 
   // Propagate the FP64 device state rho_dev over t_list.  on_output(i, cur_ptr)
@@ -78,7 +91,7 @@ class Solver {
   void check_qme() const;
   // whether a callback has changed the operator since `gen` (then moved on); the new
   // one must fit this solver's buffers
-  bool operator_changed(unsigned long long& gen) const;
+  bool operator_changed(unsigned long long& gen);
   void stage_bytes(std::vector<double>& bytes_out);
   int n_stages() const { return kind == HEOM_RKDP ? 7 : 4; }
 
@@ -119,6 +132,19 @@ class Solver {
   StageArgs resolve(const StageSpec& s) const;
   std::vector<StageSpec> specs;
   void launch_stage(int s, double dt);
+  // Graphs of a long run's repeated launches (cleared when a solve begins and ends and
+  // when the operator changes).  stream(): where launches go, the QME's stream or the one
+  // that records a graph: a stream of its own that other threads' work on the default
+  // stream does not wait for
+  std::map<int, GraphExec> graphs;
+  hipStream_t rec_stream = nullptr;
+  bool recording = false;
+  hipStream_t stream() const { return recording ? rec_stream : q->stream; }
+  void replay(int key, const std::function<void()>& body);
+  bool graph_steps = false;  // fixed steps: this solve is long enough
+  bool graph_warm = false;   // a step of this operator has been launched (its kernels are loaded)
+  bool graph_parts = false;  // and has enough intervals for graphs of less than kGraphSteps
+  long long direct_attempts = 0;  // Dormand-Prince: attempts of this solve launched one by one
   void rk4_interval(double t0, double t1, double dt);
   // resident integrator (small problems): scheme != 0 when the problem qualifies
   ResidentArgs res{};
