@@ -293,7 +293,9 @@ int heom_solver_set_graphs(heom_solver_handle s, int enable);
 
 /* measurement helpers: average device duration (ms, HIP events on the
  * library stream) of each RK stage kernel, replayed `reps` times on the
- * current state; n_stage receives 4 (rk4) or 7 (rkdp). */
+ * current state; n_stage receives 4 (rk4) or 7 (rkdp, whose first pass is the
+ * one between two attempts -- error norm, step control, next stage input -- or,
+ * with renorm_rho0, the first stage). */
 int heom_solver_time_stages(heom_solver_handle s, int reps, double* ms_per_stage,
                             int* n_stage);
 /* algorithmic HBM bytes moved by each stage kernel (same order) */

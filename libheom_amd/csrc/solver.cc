@@ -499,10 +499,9 @@ void Solver::rk4_interval(double t0, double t1, double dt) {
 }
 
 // The pass between two attempts, see StepArgs
-void Solver::launch_step(int mode) {
+StepArgs Solver::step_args(int mode) const {
   StepArgs a{};
   a.mode = mode;
-  if (mode & STEP_CONTROL) par ^= 1;
   a.next = ctrl_dev() + par;
   a.prev = (mode & STEP_CONTROL) ? ctrl_dev() + (par ^ 1) : a.next;
   a.partials = partials_dev();
@@ -521,7 +520,12 @@ void Solver::launch_step(int mode) {
   a.a21 = kDpA[1][0];
   a.n = ms;
   a.mail = mail;
-  launch_dopri_step(a, stream());
+  return a;
+}
+
+void Solver::launch_step(int mode) {
+  if (mode & STEP_CONTROL) par ^= 1;
+  launch_dopri_step(step_args(mode), stream());
 }
 
 // The device's progress word once it has moved past `seen` step passes.
@@ -880,7 +884,7 @@ void Solver::time_stages(int reps, std::vector<double>& out) {
   const int ns = n_stages();
   out.assign(ns, 0.0);
   if (kind == HEOM_RKDP) {
-    // a control block that never finishes; the last stage only reduces the norm
+    // a control block that never finishes: every pass, the step pass too, starts from it
     Ctrl c{};
     c.t = 0.0;
     c.t_bound = 1e300;
@@ -889,6 +893,7 @@ void Solver::time_stages(int reps, std::vector<double>& out) {
     std::memcpy(h_ctrl, &c, sizeof(Ctrl));
     par = 0;
     HAMD_HIP(hipMemcpyAsync(d_ctrl.p, h_ctrl, sizeof(Ctrl), hipMemcpyHostToDevice, st));
+    n_partials = launch_operator(q->dev, in_bytes, stages[6], st);  // what the step pass adds up
   }
   hipEvent_t e0, e1;
   HAMD_HIP(hipEventCreate(&e0));
@@ -896,13 +901,17 @@ void Solver::time_stages(int reps, std::vector<double>& out) {
   for (int s = 0; s < ns; ++s) {
     StageArgs a = stages[s];
     a.a_re = 1e-3;
-    // the first of the seven Dormand-Prince passes is the step pass (with a
-    // projection of rho_0: stage 0)
+    // the first of the seven Dormand-Prince passes is the step pass with its decision
+    // (with a projection of rho_0: stage 0); the decision goes to the other control block
     const auto pass = [&] {
-      if (kind == HEOM_RKDP && s == 0 && !q->opt.renorm_rho0)
-        launch_step(STEP_INPUT);
-      else
+      if (kind == HEOM_RKDP && s == 0 && !q->opt.renorm_rho0) {
+        StepArgs sa = step_args(STEP_CONTROL | STEP_INPUT);
+        sa.prev = ctrl_dev();
+        sa.next = ctrl_dev() + 1;
+        launch_dopri_step(sa, st);
+      } else {
         launch_operator(q->dev, in_bytes, a, st);
+      }
     };
     pass();  // warm-up
     HAMD_HIP(hipEventRecord(e0, st));

@@ -116,6 +116,7 @@ class Solver {
   const double* step_t = nullptr;
   int step_n_int = 0;
   z128* step_rho_s = nullptr;
+  StepArgs step_args(int mode) const;
   void launch_step(int mode);
   unsigned long long wait_mail(unsigned long long seen);
   int run_attempts(bool stale);
