@@ -284,7 +284,8 @@ int heom_solver_reset(heom_solver_handle s); /* forget dt_save (adaptive_step_si
  * output interval (RK4, lsrk4; Dormand-Prince for a heom_hilb problem of 1, 2 or
  * 4 levels), or one per heom_solve_dev call (RK4, lsrk4 and Dormand-Prince with
  * the step control on the device), and replay the launches of long runs from HIP
- * graphs (512 steps, 128 attempts and more); 0: launch every stage kernel.
+ * graphs (512 steps, 128 attempts and more, hierarchies of up to 2^17 and 2^16
+ * elements); 0: launch every stage kernel.
  * Fixed-step results are identical either way; Dormand-Prince
  * sums its error norm in another order, so a borderline attempt may be decided
  * differently (the states agree within the tolerance).  No counterpart in the

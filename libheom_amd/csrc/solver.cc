@@ -404,11 +404,16 @@ void Solver::launch_stage(int s, double dt) {
 }
 
 // A run of many short stages waits longer between its kernels when the host launches
-// them one by one (RK4, 16 000 stages of 364 ADOs of 2x2: 5.30 us per stage, 4.6 from
+// them one by one (RK4, 16 000 stages of 364 ADOs of 2x2: 4.80 us per stage, 4.41 from
 // graphs), but a graph costs its instantiation, some 100 us, on every solve: fixed steps
 // are replayed in graphs of up to kGraphSteps steps when the solve takes kGraphMin of
-// them, Dormand-Prince attempts one at a time after kGraphAttempts of them.
+// them, Dormand-Prince attempts one at a time after kGraphAttempts of them.  Longer stages
+// hide the host's launches, and then a graph's start costs more than it saves: RK4 step and
+// attempt of 253 ADOs of 7x7 18.7 -> 17.7 and 42.3 -> 39.0 us, 2024 ADOs (99 000 elements)
+// 21.5 and 44.8 -> 21.4 and 45.3, 12 650 ADOs 60.9 and 122.4 -> 61.6 and 126.9; RK4 step of
+// 80 000 elements in 4x4 31.2 -> 30.1, of 167 000 in 3x3 42.3 -> 42.9.
 constexpr int kGraphSteps = 16, kGraphMin = 512, kGraphIntervals = 8, kGraphAttempts = 128;
+constexpr long long kGraphStepSize = 1 << 17, kGraphAttemptSize = 1 << 16;  // elements
 
 // Launch `body` from graph `key`, which is recorded the first time.  The body launches
 // kernels only (no copy or memset: replays of memset nodes have gone wrong).
@@ -581,8 +586,8 @@ int Solver::run_attempts(bool stale) {
       ++attempts;
       ++direct_attempts;
     }
-    if (use_resident && direct_attempts >= kGraphAttempts && !(v & 2) && steps < seen + 1 &&
-        attempts == steps) {
+    if (use_resident && ms <= kGraphAttemptSize && direct_attempts >= kGraphAttempts &&
+        !(v & 2) && steps < seen + 1 && attempts == steps) {
       const int from = par;  // the step pass writes the other control block
       replay(from, [&] {
         step(false);
@@ -647,7 +652,7 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
   unsigned long long gen = q->generation;
   if (kind != HEOM_RKDP) {  // fixed step: rk4, lsrk4
     graph_steps = graph_parts = false;
-    if (use_resident && res.scheme == 0) {
+    if (use_resident && res.scheme == 0 && ms <= kGraphStepSize) {
       long long total = 0, n = 0;
       double last = 0.0;
       for (int i = 0; i + 1 < n_t; ++i) {
