@@ -7,14 +7,16 @@ Workload (one "step" = one full propagation, the time-to-rho_S(t) job):
   plain FP64 (complex128) Hilbert form.  Inputs are synthetic (seeded).
 The state is resident in HBM when the timed region starts.
 
-Metric: ADO-stage updates/s = n_hrchy * (RHS evaluations performed) / s.
+Metric: ADO-stage updates/s = n_hrchy * (RHS evaluations performed) / s.  A
+Dormand-Prince attempt has seven stages; the first is the last one of the attempt
+before, so six evaluations are performed (evaluations()).
 Also reported: the roofline of the dominant kernel (the fused Hilbert-form
-stage pass; algorithmic bytes per launch / average launch duration measured
-with HIP events on the library stream) and the CPU oracle timed on the host
-cores on a bounded sample of the same workload.  The algorithmic bytes are
-those of the reference's step per ADO-stage (alg_bytes_per_ado_stage) times
-the ADOs of one launch; the bytes the fused kernel itself must move (fewer:
-stage 6 forms the error sum) are reported beside them.
+stage pass; the bytes the pass itself must move per launch / average launch
+duration measured with HIP events on the library stream, over the six operator
+passes of an attempt) and the CPU oracle timed on the host cores on a bounded
+sample of the same workload.  Beside it the same attempt, step pass included,
+against the bytes of the reference's step (alg_bytes_per_ado_stage, seven
+evaluations without fusion of the error sum).
 
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W]
 """
@@ -44,6 +46,14 @@ def alg_bytes_per_ado_stage(n_level, n_dim, method, sc=16):
     Neighbour ADOs count once (another ADO's compulsory read)."""
     m = 47.0 / 7.0 if method == "rkdp" else 5.0
     return m * n_level * n_level * sc + 8.0 * n_dim + 8.0
+
+
+def evaluations(st, solves=1, projected=False):
+    """Operator evaluations of `solves` Dormand-Prince solves: six per attempt and one
+    at the start of each, or seven per attempt where rho_0 is projected (the stored
+    derivative is stale then).  stats()["n_rhs"] counts the scheme's stages, seven per
+    attempt."""
+    return 7 * st["n_attempts"] if projected else 6 * st["n_attempts"] + solves
 
 
 def mk_solver(H, eng, q, method):
@@ -380,14 +390,15 @@ def bench_dense64(H, L, reps):
         flops = q.n_hrchy * 4 * 2 * 64 ** 3
         unit = q.n_hrchy * alg_bytes_per_ado_stage(
             q.n_level, q.n_dim, "rkdp", 16 if dtype in ("complex128", "valu") else 8)
-        res[dtype] = {"value": st["ado_stage_updates"] / el, "time_to_rho_s_ms": 1e3 * el,
+        evals = evaluations(st)
+        res[dtype] = {"value": q.n_hrchy * evals / el, "time_to_rho_s_ms": 1e3 * el,
                       "stage_ms": stage_ms,
                       "hbm_frac": unit / (stage_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
                       "alg_bytes_per_stage": unit,
                       "hbm_frac_kernel_bytes": float(sby[:n].mean()) / (stage_ms * 1e-3)
                       / 1e9 / HBM_PEAK_GBS,
                       "commutator_tflops": flops / (stage_ms * 1e-3) / 1e12,
-                      "rhs_evals": st["n_rhs"], "rs": rs}
+                      "rhs_evals": evals, "rs": rs}
     f64 = res["complex128"]
 
     def variant(r):
@@ -479,7 +490,8 @@ def bench_redfield(H, L, reps, cpu=True):
         el = time.perf_counter() - t0
         st = sv.stats()
         st_ms, st_b = _stage_stats(L, sv, reps)
-        r = {"time_to_rho_s_ms": 1e3 * el, "rhs_evals": st["n_rhs"], "stage_us": 1e3 * st_ms,
+        r = {"time_to_rho_s_ms": 1e3 * el, "stage_us": 1e3 * st_ms,
+             "rhs_evals": evaluations(st) if isinstance(solver, H.rkdp) else st["n_rhs"],
              "bytes_per_stage": st_b}
         if cpu:
             o = O.Oracle(okind, m["N"], 0, n_threads=1).load(m)
@@ -651,8 +663,8 @@ def main():
     for _ in range(args.steps):
         el, st = one_step()
         times.append(el)
-        updates += st["ado_stage_updates"]
-        rhs += st["n_rhs"]
+        updates += qme.n_hrchy * evaluations(st)
+        rhs += evaluations(st)
     total = sum(times)
     value = updates / total
 
@@ -665,7 +677,7 @@ def main():
     for _ in range(args.steps):
         el, st = one_step(solver32, rs32)
         t32 += el
-        u32 += st["ado_stage_updates"]
+        u32 += qme32.n_hrchy * evaluations(st)
     variant32 = {
         "dtype": "f32 operator / f64 combination", "value": u32 / t32,
         "ms_per_step": 1e3 * t32 / args.steps,
@@ -687,7 +699,7 @@ def main():
     for _ in range(args.steps):
         el, st = one_step(solver32p, rs32p)
         t32p += el
-        u32p += st["ado_stage_updates"]
+        u32p += qme32p.n_hrchy * evaluations(st, projected=True)
     trace_err = lambda r: float(np.abs(np.trace(r, axis1=1, axis2=2) - 1.0).max())
     variant32["trace_err"] = trace_err(rs32)
     variant32p = {
@@ -718,11 +730,12 @@ def main():
     _capi.check(L.heom_solver_time_stages(solver._s, args.reps, p(ms), ctypes.byref(ns)))
     _capi.check(L.heom_solver_stage_bytes(solver._s, p(by), ctypes.byref(ns)))
     n = ns.value
-    kernel_bytes = float(by[:n].mean())
-    avg_ms = float(ms[:n].mean())
-    unit_bytes = alg_bytes_per_ado_stage(qme.n_level, qme.n_dim, "rkdp")
-    avg_bytes = unit_bytes * qme.n_hrchy
+    # the six operator passes (pass 0 is the step pass)
+    avg_bytes = float(by[1:n].mean())
+    avg_ms = float(ms[1:n].mean())
     achieved = avg_bytes / (avg_ms * 1e-3) / 1e9
+    unit_bytes = alg_bytes_per_ado_stage(qme.n_level, qme.n_dim, "rkdp")
+    ref_gbs = 7 * unit_bytes * qme.n_hrchy / (float(ms[:n].sum()) * 1e-3) / 1e9
     L.heom_dev_free(d)
     # measured HBM bytes per stage dispatch (rocprofv3 FETCH_SIZE + WRITE_SIZE,
     # calibrated on a copy of known size), recorded by --summarize-pmc
@@ -748,14 +761,16 @@ def main():
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
             "kernel": "hilb_fast_kernel<7,double> (fused Dormand-Prince stage pass)",
-            "note": "mean of the seven passes of an attempt: the first is the step pass "
-                    "(dopri_step_kernel: k_1 comes from the last stage of the attempt before), "
-                    "six are operator passes; value counts the scheme's seven stages",
-            "bytes_per_ado_stage": unit_bytes, "ados_per_launch": qme.n_hrchy,
+            "note": "the six operator passes of an attempt, the bytes they must move; stage_ms "
+                    "lists the step pass (dopri_step_kernel) first",
             "bytes_per_launch": avg_bytes, "avg_launch_ms": avg_ms,
+            "ados_per_launch": qme.n_hrchy,
             "stage_ms": [float(x) for x in ms[:n]],
-            "kernel_bytes_per_launch": kernel_bytes,
-            "frac_kernel_bytes": kernel_bytes / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
+            "reference_step": {
+                "note": "the bytes of the reference's seven evaluations over the time of the "
+                        "attempt's seven passes",
+                "bytes_per_ado_stage": unit_bytes, "gbs": ref_gbs,
+                "frac": ref_gbs / HBM_PEAK_GBS},
         },
         "rho_s_max_abs_err_vs_oracle": (float(np.abs(rs - gold).max())
                                         if gold is not None else None),
