@@ -278,18 +278,19 @@ int heom_solve_dev_noalloc(heom_solver_handle s, void* rho_dev, const double* t_
                            double dt, double atol, double rtol, double* rho_s_out);
 int heom_solver_stats(heom_solver_handle s, heom_stats* out);
 int heom_solver_reset(heom_solver_handle s); /* forget dt_save (adaptive_step_size_solver.h:28) */
-/* 1 (default): run a small heom_hilb problem (diagonal V, FP64, at most 1024
- * elements -- 960 for Dormand-Prince -- and at most 8 links per ADO) or a small redfield_hilb problem (diagonal V, FP64,
- * its tables within LDS) in resident launches with the state in LDS: one per
- * output interval (RK4, lsrk4; Dormand-Prince for a heom_hilb problem of 1, 2 or
- * 4 levels), or one per heom_solve_dev call (RK4, lsrk4 and Dormand-Prince with
- * the step control on the device), and replay the launches of long runs from HIP
- * graphs (512 steps, 128 attempts and more, hierarchies of up to 2^17 and 2^16
- * elements); 0: launch every stage kernel.
- * Fixed-step results are identical either way; Dormand-Prince
- * sums its error norm in another order, so a borderline attempt may be decided
- * differently (the states agree within the tolerance).  No counterpart in the
- * reference. */
+/* 1 (default): run a small heom_hilb, heom_liou or heom_ado problem (diagonal V,
+ * FP64, at most 1024 elements -- 960 for Dormand-Prince -- and at most 8 links per
+ * ADO) or a small redfield_hilb problem (diagonal V, FP64, its tables within LDS)
+ * in resident launches with the state in LDS: one per output interval (RK4, lsrk4;
+ * Dormand-Prince for 1, 2 or 4 levels, not redfield_hilb), or one per heom_solve_dev
+ * call (RK4, lsrk4 and Dormand-Prince with the step control on the device), and
+ * replay the launches of long runs from HIP graphs (512 steps, 128 attempts and
+ * more, hierarchies of up to 2^17 and 2^16 elements); 0: launch every stage kernel.
+ * Graph replay gives the same bits.  Resident fixed-step launches do for up to 5
+ * levels and real parameters, and else agree to rounding; resident Dormand-Prince
+ * sums its error norm in another order in heom_solve_dev, so a borderline attempt may
+ * be decided differently (the states agree within the tolerance).  No counterpart in
+ * the reference. */
 int heom_solver_set_graphs(heom_solver_handle s, int enable);
 
 /* measurement helpers: average device duration (ms, HIP events on the

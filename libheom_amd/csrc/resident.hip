@@ -100,7 +100,13 @@ struct ResidentElem {
     cmac(D, diag, x);
 #pragma unroll
     for (int l = 0; l < MAXL; ++l)
-      if (l < nl) cmac(D, cf[l], AHEAD ? xn[l] : X[nbr[l]]);
+      if (l < nl) {
+        // the product that is not rounded is the one of the stage kernels, whose bits
+        // a fixed-step solve with real parameters keeps
+        const z128 c = cf[l], v = AHEAD ? xn[l] : X[nbr[l]];
+        D.re += fma(c.re, v.re, -(c.im * v.im));
+        D.im += fma(c.im, v.re, c.re * v.im);
+      }
     return D;
   }
 };
