@@ -409,24 +409,24 @@ __global__ void __launch_bounds__(kBigBS) hilb_big_kernel(const FormDev d, const
 template <int N, typename R, bool F64>
 int launch_hilb_n(const FormDev& d, const StageArgs& A, hipStream_t st) {
   if (N >= 4 && d.slinks != nullptr) return launch_hilb_split<R, F64>(d, A, st);
-  const bool real = d.real_v && d.real_h;
-  if (N >= 6 && d.diag_v && d.bmap != nullptr && d.n_hrchy <= kMaxGrid &&
-      fast_vd_lds(d, real, sizeof(R)) <= 32 * 1024) {
-    constexpr int BS = WaveCfg<N>::BS;
-    const int grid = d.n_hrchy;
+  if constexpr (N >= 6) {
+    const bool real = d.real_v && d.real_h;
     const size_t lds = fast_vd_lds(d, real, sizeof(R));
-    // four prefetched operands cover every stage but Dormand-Prince's fifth and sixth
-    const auto run = [&](auto real_, auto kp, auto epi) {
-      hipLaunchKernelGGL(
-          (hilb_fast_kernel<N, R, decltype(real_)::value, F64, decltype(kp)::value,
-                            decltype(epi)::value>),
-          dim3(grid), dim3(BS), lds, st, d, A);
-    };
-    if (real)
-      with_epilogue<4, 6>(A, [&](auto kp, auto epi) { run(std::true_type{}, kp, epi); });
-    else
-      with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) { run(std::false_type{}, kp, epi); });
-    return grid;
+    if (d.diag_v && d.bmap != nullptr && d.n_hrchy <= kMaxGrid && lds <= 32 * 1024) {
+      const int grid = d.n_hrchy;
+      // four prefetched operands cover every stage but Dormand-Prince's fifth and sixth
+      const auto run = [&](auto real_, auto kp, auto epi) {
+        hipLaunchKernelGGL(
+            (hilb_fast_kernel<N, R, decltype(real_)::value, F64, decltype(kp)::value,
+                              decltype(epi)::value>),
+            dim3(grid), dim3(WaveCfg<N>::BS), lds, st, d, A);
+      };
+      if (real)
+        with_epilogue<4, 6>(A, [&](auto kp, auto epi) { run(std::true_type{}, kp, epi); });
+      else
+        with_epilogue<4, kMaxPre>(A, [&](auto kp, auto epi) { run(std::false_type{}, kp, epi); });
+      return grid;
+    }
   }
   constexpr int APB = HilbCfg<N>::APB, BS = HilbCfg<N>::BS;
   const int grid = cap_grid((d.n_hrchy + APB - 1) / APB);

@@ -211,9 +211,9 @@ __device__ __forceinline__ void mfma_commutator_bf16x3(const FormDev& d, const f
 // CU (LDS holds two FP64 workgroups per CU), i.e. BS / 128 waves per SIMD:
 // 256 threads leave 256 registers per lane, 512 threads 128.
 // BF16X3: R = float, products via mfma_commutator_bf16x3.  N is the tile size
-// (32 or 64); the ADO block is n x n with n = d.N in (N/2, N] for N = 64, in
-// (16, 32] for N = 32, zero-padded in LDS (and H in its planes), so that the
-// padded rows and columns of the products are exactly zero.
+// (mfma_tile: 32, 48 or 64); the ADO block is n x n with n = d.N <= N, zero-padded in
+// LDS (and H in its planes), so that the padded rows and columns of the products are
+// exactly zero.
 template <int N, typename R, bool REALH, bool F64, int KP, Epi E, bool BF16X3, bool PADDED,
           int BS>
 __global__ void __launch_bounds__(BS, BS / 128)
@@ -446,7 +446,7 @@ __device__ __forceinline__ void mfma_cprod(const R* ar, const R* ai, const R* br
   using Cfg = MfmaCfg<N>;
   constexpr int LDA = A_LDS ? Cfg::LD : N, LDB = B_LDS ? Cfg::LD : N;
   constexpr bool AR = !A_LDS && GREAL, BR = !B_LDS && GREAL;
-  constexpr int KG = !GREAL ? 2 : Cfg::KS % kCprodAhead == 0 ? kCprodAhead : Cfg::KS * kCprodAhead / 16;
+  constexpr int KG = GREAL ? kCprodAhead : 2;
   static_assert(Cfg::KS % KG == 0, "k groups");
   const int row = band * 16 + lr;
   R ga_r[KG], ga_i[KG], gb_r[KG][TPW], gb_i[KG][TPW];
@@ -510,8 +510,7 @@ constexpr int kDenseCh = 4;
 // waves per SIMD the registers have to allow: one workgroup per CU at N = 64 in FP64
 // (133 KB of LDS), two in FP32
 template <int N, typename R>
-constexpr int kDenseWps = N == 64 ? (sizeof(R) == 8 ? 2 : 4)
-                          : N == 48 ? (sizeof(R) == 8 ? 3 : 4) : (sizeof(R) == 8 ? 3 : 4);
+constexpr int kDenseWps = sizeof(R) == 4 ? 4 : N == 64 ? 2 : 3;
 
 template <int N, typename R, bool REALV, bool REALH, bool F64, int KP, Epi E, bool PADDED, int BS>
 __global__ void __launch_bounds__(BS, (kDenseWps<N, R>))
@@ -524,7 +523,7 @@ __global__ void __launch_bounds__(BS, (kDenseWps<N, R>))
   constexpr int TPW = NB * NB / (BS / 64);  // output tiles per wave
   constexpr int EPT = N2 / BS;  // elements per thread when rho_n is staged
   extern __shared__ __align__(16) unsigned char s_dyn[];
-  R* s_re = reinterpret_cast<R*>(s_dyn);  // rho_n, at the end D
+  R* s_re = reinterpret_cast<R*>(s_dyn);  // rho_n
   R* s_im = s_re + N * LD;
   R* w_re = s_im + N * LD;  // workspace: X_u, then Y_u
   R* w_im = w_re + N * LD;

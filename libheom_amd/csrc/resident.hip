@@ -266,9 +266,10 @@ __global__ void __launch_bounds__(BS) resident_kernel(const FormDev d, const Res
 // starts as ctrl_init_kernel does.  Up to 512 elements, where a lane has 256
 // registers, y, y_new and k1..k6 stay in registers; LDS holds the operator
 // inputs: 0/1 the y / y_new pair (swapped on acceptance), 2/3 the stage inputs,
-// and 4..9 the lanes' own k's of the larger problems.  The error norm is summed in a fixed order (wavefront
-// shuffles, then the waves: one after another, or with a.tree as
-// err_finalize_kernel adds the partials of one-wave workgroups).  Up to eight
+// and 4..9 the lanes' own k's of the larger problems.  The error norm is summed in a
+// fixed order: wavefront shuffles, then the waves, one after another, or with a.tree as
+// dopri_step_kernel adds up to sixteen partials of one-wave workgroups (lane w of its
+// first wavefront holds partial w): a change there has to be made here.  Up to eight
 // wavefronts every lane runs the step control on it (no round trip through LDS);
 // with more, lane 0 does (all sixteen wavefronts computing the power of the error
 // took 20% of a solve).
