@@ -284,8 +284,9 @@ int heom_solver_reset(heom_solver_handle s); /* forget dt_save (adaptive_step_si
  * in resident launches with the state in LDS: one per output interval (RK4, lsrk4;
  * Dormand-Prince for 1, 2 or 4 levels, not redfield_hilb), or one per heom_solve_dev
  * call (RK4, lsrk4 and Dormand-Prince with the step control on the device), and
- * replay the launches of long runs from HIP graphs (512 steps, 128 attempts and
- * more, hierarchies of up to 2^17 and 2^16 elements); 0: launch every stage kernel.
+ * replay the launches of long runs from HIP graphs (fixed steps from 8 replays of up
+ * to 8 steps, hierarchies of up to 2^16 elements, from 64 up to 2^17; Dormand-Prince
+ * after 128 attempts, up to 2^16 elements); 0: launch every stage kernel.
  * Graph replay gives the same bits.  Resident fixed-step launches do for up to 5
  * levels and real parameters, and else agree to rounding; resident Dormand-Prince
  * sums its error norm in another order in heom_solve_dev, so a borderline attempt may

@@ -406,13 +406,17 @@ void Solver::launch_stage(int s, double dt) {
 // A run of many short stages waits longer between its kernels when the host launches
 // them one by one (RK4, 16 000 stages of 364 ADOs of 2x2: 4.80 us per stage, 4.41 from
 // graphs), but a graph costs its instantiation, some 100 us, on every solve: fixed steps
-// are replayed in graphs of up to kGraphSteps steps when the solve takes kGraphMin of
-// them, Dormand-Prince attempts one at a time after kGraphAttempts of them.  Longer stages
+// are replayed in graphs of up to kGraphSteps steps when the solve makes kGraphReplays or
+// more of them, Dormand-Prince attempts one at a time after kGraphAttempts of them.  70 ADOs
+// of 5x5, RK4, intervals x steps, launched -> graphs of 8 (of 16): 1 x 32 0.76 -> 0.85 (0.95)
+// ms, 1 x 128 2.98 -> 2.66 (2.71), 10 x 10 2.69 -> 2.43 (2.68), 10 x 40 9.66 -> 8.20 (8.18);
+// graphs of 4, 10 x 5 1.53 -> 1.36; graphs of 2, 100 x 3 10.2 -> 8.3.  Longer stages
 // hide the host's launches, and then a graph's start costs more than it saves: RK4 step and
 // attempt of 253 ADOs of 7x7 18.7 -> 17.7 and 42.3 -> 39.0 us, 2024 ADOs (99 000 elements)
 // 21.5 and 44.8 -> 21.4 and 45.3, 12 650 ADOs 60.9 and 122.4 -> 61.6 and 126.9; RK4 step of
-// 80 000 elements in 4x4 31.2 -> 30.1, of 167 000 in 3x3 42.3 -> 42.9.
-constexpr int kGraphSteps = 16, kGraphMin = 512, kGraphIntervals = 8, kGraphAttempts = 128;
+// 80 000 elements in 4x4 31.2 -> 30.1, of 167 000 in 3x3 42.3 -> 42.9.  Fixed steps of
+// more than kGraphAttemptSize elements therefore have to make eight times the replays.
+constexpr int kGraphSteps = 8, kGraphReplays = 8, kGraphAttempts = 128;
 constexpr long long kGraphStepSize = 1 << 17, kGraphAttemptSize = 1 << 16;  // elements
 
 // Launch `body` from graph `key`, which is recorded the first time.  The body launches
@@ -459,6 +463,21 @@ void Solver::fixed_steps(double t0, double t1, double dt, long long& n_full, dou
   dt_last = dt_1;
 }
 
+// Steps per graph of a solve, 0 for none: the largest power of two that an interval holds,
+// when it is replayed kGraphReplays times `scale` or more
+int Solver::graph_size(const double* t_list, int n_t, double dt, int scale) {
+  std::vector<long long> n(n_t > 1 ? n_t - 1 : 0);
+  double last = 0.0;
+  for (int i = 0; i + 1 < n_t; ++i) fixed_steps(t_list[i], t_list[i + 1], dt, n[i], last);
+  const long long longest = n.empty() ? 0 : *std::max_element(n.begin(), n.end());
+  int size = kGraphSteps;
+  while (size > 1 && size > longest) size /= 2;
+  if (size < 2) return 0;
+  long long replays = 0;
+  for (const long long k : n) replays += k / size;
+  return replays >= kGraphReplays * scale ? size : 0;
+}
+
 void Solver::rk4_interval(double t0, double t1, double dt) {
   long long n_full = 0;
   double dt_1 = dt;
@@ -485,8 +504,7 @@ void Solver::rk4_interval(double t0, double t1, double dt) {
     if (q->opt.renorm_rho0) renorm(false);
   };
   for (long long n = 0; n < n_full;) {
-    int size = graph_steps && graph_warm ? kGraphSteps : 1;
-    while (size > n_full - n) size = graph_parts ? size / 2 : 1;
+    const int size = graph_steps > 0 && graph_warm && n_full - n >= graph_steps ? graph_steps : 1;
     if (size > 1)
       replay(size, [&] {
         for (int k = 0; k < size; ++k) step();
@@ -651,17 +669,9 @@ int Solver::solve(void* rho_dev, const double* t_list, int n_t, double dt, doubl
   int gave_up = 0;
   unsigned long long gen = q->generation;
   if (kind != HEOM_RKDP) {  // fixed step: rk4, lsrk4
-    graph_steps = graph_parts = false;
-    if (use_resident && res.scheme == 0 && ms <= kGraphStepSize) {
-      long long total = 0, n = 0;
-      double last = 0.0;
-      for (int i = 0; i + 1 < n_t; ++i) {
-        fixed_steps(t_list[i], t_list[i + 1], dt, n, last);
-        total += n;
-      }
-      graph_steps = total >= kGraphMin;
-      graph_parts = graph_steps && n_t > kGraphIntervals;
-    }
+    graph_steps = use_resident && res.scheme == 0 && ms <= kGraphStepSize
+                      ? graph_size(t_list, n_t, dt, ms <= kGraphAttemptSize ? 1 : 8)
+                      : 0;
     for (int i = 0; i < n_t - 1; ++i) {
       on_output(i, P[SL_Y].p);
       if (operator_changed(gen)) {

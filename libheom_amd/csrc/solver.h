@@ -142,9 +142,9 @@ class Solver {
   bool recording = false;
   hipStream_t stream() const { return recording ? rec_stream : q->stream; }
   void replay(int key, const std::function<void()>& body);
-  bool graph_steps = false;  // fixed steps: this solve is long enough
+  int graph_steps = 0;       // fixed steps of a graph of this solve, 0: none
+  static int graph_size(const double* t_list, int n_t, double dt, int scale);
   bool graph_warm = false;   // a step of this operator has been launched (its kernels are loaded)
-  bool graph_parts = false;  // and has enough intervals for graphs of less than kGraphSteps
   long long direct_attempts = 0;  // Dormand-Prince: attempts of this solve launched one by one
   void rk4_interval(double t0, double t1, double dt);
   // resident integrator (small problems): scheme != 0 when the problem qualifies

@@ -49,8 +49,8 @@ def scaled(N, dep, seed, **kw):
     return m
 
 
-# steps per interval: the whole set of graph sizes (31 = 16 + 8 + 4 + 2 + 1), one interval
-# longer than all graphs, and few intervals with a remainder
+# steps per interval: several graphs and a remainder in every interval (31 = 3 x 8 + 7), one
+# interval longer than all graphs, and few intervals with a remainder
 @pytest.mark.parametrize("steps,n_int", [(31, 18), (600, 1), (203, 3)])
 @pytest.mark.parametrize("method,dtype,proj", [("rk4", "complex128", False),
                                                ("lsrk4", "complex64", False),
@@ -63,6 +63,26 @@ def test_fixed_steps(method, dtype, proj, steps, n_int):
     t = dt * (steps + 0.5) * np.arange(n_int + 1)
     st = runs(q, m, method, t, {"dt": dt})
     assert st["n_attempts"] >= n_int * (steps + 1)
+
+
+# the shortest intervals replay graphs of 2 and 4 steps; 8 replays of them are the fewest
+@pytest.mark.parametrize("steps,n_int", [(2, 9), (3, 8), (4, 12), (7, 8), (9, 8), (65, 1)])
+@pytest.mark.parametrize("dtype,proj", [("complex128", False), ("complex64", True)])
+def test_short_intervals(dtype, proj, steps, n_int):
+    print("replay short", dtype, proj, steps, n_int, flush=True)
+    m = scaled(5, 4, 6)
+    q = H.heom_hilb(4, dtype=dtype, renorm_rho0=proj).load(m, H.hip(0))
+    t = 1e-3 * (steps + 0.5) * np.arange(n_int + 1)
+    st = runs(q, m, "rk4", t, {"dt": 1e-3})
+    assert st["n_attempts"] == n_int * (steps + 1)
+
+
+# above 65 536 elements eight times the replays are asked for
+def test_large_hierarchy():
+    m = configs.random_model(7, 3, 4, 4, seed=3, dense_v=False, complex_params=False)
+    assert 1 << 16 < m["rho0"].size <= 1 << 17
+    q = H.heom_hilb(4).load(m, H.hip(0))
+    runs(q, m, "rk4", 1e-4 * 24.5 * np.arange(26), {"dt": 1e-4})
 
 
 @pytest.mark.parametrize("N,dep,dtype,proj",
