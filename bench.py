@@ -124,7 +124,7 @@ def summarize_trace(path, top=12, live_us=5.0):
     for name, v in sorted(by.items(), key=lambda kv: -sum(kv[1]))[:top]:
         live = [x for x in v if x >= live_us]
         short = name.replace("void ", "").replace("hamd::(anonymous namespace)::", "")
-        short = short.replace("hamd::", "").split("(")[0]
+        short = short.replace("(hamd::Epi)", "").replace("hamd::", "").split("(")[0]
         out.append("| `%s` | %d | %.2f | %.1f | %.2f | %d | %s |" % (
             short, len(v), sum(v) / 1e3, 100.0 * sum(v) / total, statistics.mean(v), len(live),
             "%.2f" % statistics.mean(live) if live else "-"))

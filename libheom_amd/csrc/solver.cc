@@ -581,8 +581,8 @@ int Solver::run_attempts(bool stale) {
   __atomic_store_n(mail, 0ull, __ATOMIC_RELEASE);
   // a projection of rho_0 (after every attempt; it acts only on an accepted one)
   // makes the stored D stale.  Stage 0 then takes the place of the step pass's stream:
-  // 7-site chain, projected: 138 us per attempt (FP64 151) with stage 0 storing D alone
-  // and a launch more for the stage input, 134 us (FP64 145)
+  // 7-site chain, projected, 1 ps: 136.5 us per attempt (FP64 147.4) with stage 0 storing D
+  // alone and a launch more for the stage input, 127.4 us (FP64 136.9)
   const auto step = [&](bool first) {
     const bool eval = proj || (first && stale);
     launch_step(STEP_CONTROL | (first ? STEP_FIRST : 0) | (eval ? 0 : STEP_INPUT));
